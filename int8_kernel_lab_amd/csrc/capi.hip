@@ -442,13 +442,13 @@ int i8conv_describe(int id, const i8conv_shape *shape, char *buf, size_t len) {
                     ", " + std::to_string(p.pw_waves) +
                     " waves; unaligned pointers:"
               : "") +
-        (p.dma ? " pipelined" : " register-staged") + " tile " +
+        (p.m32 ? " 32x32 MFMA" : p.dma ? " pipelined" : " register-staged") + " tile " +
         std::to_string(p.bm) + "px x " + std::to_string(p.bn) + "oc" +
         (p.m_step > 0 && p.m_step < p.bm ? " (" + std::to_string(p.m_step) + "px stored)" : "") +
         ", grid " + tiles(g.gemm_m, p.m_step > 0 ? p.m_step : p.bm) + "x" +
         tiles(g.gemm_n, p.bn) + (p.splits > 1 ? "x" + std::to_string(p.splits) + " splits" : "") +
         ", " + std::to_string(p.stages) + " k-stages" +
-        (p.dma && gemm_dma_copy_waves(p) > 0 ? ", " + std::to_string(gemm_dma_copy_waves(p)) + " copy waves" : "");
+        (p.dma && !p.m32 && gemm_dma_copy_waves(p) > 0 ? ", " + std::to_string(gemm_dma_copy_waves(p)) + " copy waves" : "");
   } else {
     PatchPlan p;
     if (id == I8CONV_KERNEL_STRIP) plan_strip(*shape, g, &p);
@@ -746,6 +746,20 @@ int i8conv_launch_requant(const i8conv_shape *shape, const int8_t *input, const 
                    ? std::string(" (or bias, mult, shift and output 16-byte aligned)")
                    : std::string()));
     return I8CONV_WORKSPACE_TOO_SMALL;
+  }
+  // The 32 x 32 x 32 MFMA kernel requantizes in its epilogue and leaves the
+  // workspace alone (16 x 224x224, 32 -> 64 7x7 stride 2: 101 us through the
+  // int32 workspace and the pass, 35 us).
+  if (id == I8CONV_KERNEL_GENERIC && g.gemm_n % 4 == 0 && aligned(output, 4)) {
+    const GemmPlan p = plan_generic(*shape, g);
+    if (p.m32) {
+      ConvArgs args = make_args(*shape, g, input, filter, bias, nullptr);
+      args.q_mult = mult;
+      args.q_shift = shift;
+      args.q_zp = zero_point;
+      args.q_y = output;
+      return launch_gemm32(args, p, stream);
+    }
   }
   int32_t *acc = static_cast<int32_t *>(workspace);
   void *conv_ws = static_cast<char *>(workspace) + acc_bytes;

@@ -92,6 +92,9 @@ struct GemmPlan {
   // c % 128 == 0: the LDS-DMA pipelined kernel (kernel_gemm_dma.hip), else
   // the register-staged one (kernel_gemm.hip)
   bool dma = false;
+  // generic only: the 32 x 32 x 32 MFMA kernel (kernel_gemm32.hip) runs the
+  // layer, on bm x bn tiles
+  bool m32 = false;
   // split-K only: the deep-channel kernel instead of the GEMM
   bool deep = false;
   DeepPlan deep_plan;
@@ -108,6 +111,9 @@ bool gemm_dma_tile_supported(int bm, int bn);
 // every wave copies and runs MFMAs)
 int gemm_dma_copy_waves(const GemmPlan &p);
 GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g);
+// output tiles of the 16 x 16 MFMA kernels' grid for a layer (the measure of
+// a small or large grid in the dispatch policy)
+int64_t staged_tiles(const i8conv_shape &s, const i8conv_geometry &g);
 int gemm_dma_step(int64_t gemm_m, int64_t tiles_n, int bm, int bn);
 GemmPlan plan_splitk(const i8conv_shape &s, const i8conv_geometry &g);
 size_t splitk_workspace_bytes(const i8conv_geometry &g, const GemmPlan &p);
@@ -158,6 +164,10 @@ int launch_splitk(const ConvArgs &a, const GemmPlan &p, void *workspace,
                   void *stream, const RequantArgs *rq = nullptr);
 // kernel_gemm_dma.hip; splits > 1 writes partial sums to a.partial
 int launch_gemm_dma(const ConvArgs &a, const GemmPlan &p, int splits, void *stream);
+// kernel_gemm32.hip: whether a layer's sizes fit it, and its launch (int8
+// output when a.q_y is set: N % 4 == 0 and a 4-byte aligned q_y)
+bool gemm32_eligible(const i8conv_geometry &g);
+int launch_gemm32(const ConvArgs &a, const GemmPlan &p, void *stream);
 // kernel_pointwise.hip: C and N with an instance (C in {64, 128, 256,
 // 512}, N in {32, 64, 128, 256}), the output-channel slices it splits N
 // into (each of 16384 / C channels, at most N), the waves of a launch, its

@@ -321,8 +321,9 @@ int launch_gemm(const ConvArgs &a, const GemmPlan &p, void *stream) {
   args.splits = 1;
   args.stages_per_split = p.stages;
   if (p.pw && !args.q_y && pointwise_pointers_ok(args)) return launch_pointwise(args, nullptr, stream);
+  if (p.m32) return launch_gemm32(args, p, stream);
   if (args.q_y && !p.dma) {
-    set_error("requantized GEMM output needs the pipelined kernel (C % 128 == 0)");
+    set_error("requantized GEMM output needs the pipelined or the 32 x 32 x 32 MFMA kernel");
     return I8CONV_BAD_ARGUMENT;
   }
   if (p.dma) return launch_gemm_dma(args, p, 1, stream);

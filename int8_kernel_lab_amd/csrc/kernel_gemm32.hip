@@ -1,0 +1,490 @@
+// Generic implicit GEMM on the 32 x 32 x 32 INT8 MFMA, for any input channel
+// count (C % 16 == 0): the generic kernel's form for layers whose channels
+// are no multiple of 128, for small grids of strided and 1x1 layers, and for
+// the largest ones (plan_generic in shape.cpp has the rule and both sides'
+// figures).  Same GEMM view as kernel_gemm_dma.hip (M = n*out_h*out_w pixels,
+// N output channels, k = (fy*s + fx)*c + ci); what it does differently:
+//   * pixels are the MFMA's rows and output channels its columns, so a lane
+//     holds one channel of sixteen pixels and every 4-byte store of a wave
+//     writes two whole 128-byte pieces of output rows, whatever N is.  With
+//     the roles the other way round a 16-byte store scatters 32-byte pieces
+//     over 32 pixels: 128 x 128 x 8 images, 64 -> 128 channels, 1x3: 28.1
+//     against 15.1 us; 256 x 256, 64 -> 255 channels, 3x3: 43 us with the
+//     element stores of the 16 x 16 forms, 23 us here;
+//   * v_mfma_i32_32x32x32 does the operations of two 16 x 16 x 64 with half
+//     the operand reads: on random operands, all SIMDs busy, it sustains 3.45
+//     POP/s against 2.8 (the shader clock follows the power drawn);
+//   * k-stages of 128 bytes per row come by LDS-DMA (R stage buffers, one
+//     barrier per stage).  A 128-byte row is a whole L2 line: the same copies
+//     in 64-byte halves land at 70 instead of 130 GB/s per compute unit;
+//   * with kLaneTap each lane decomposes its own 16-byte chunk's k into tap
+//     and channel, so a stage may span taps (C % 128 != 0); otherwise a stage
+//     lies inside one tap and the channel chunk is the outer loop, the taps
+//     the inner one;
+//   * workgroups are persistent: the next tile's first R stages are copied
+//     before the tile's stores go out.  Small tiles share a compute unit two
+//     to four at a time, which hides their copy issue and LDS latency better
+//     than more stage buffers did (R = 2, 4, 6, 9 within 8 %);
+//   * int8 output: each lane requantizes its channel (parameters read once
+//     per tile), and the four lanes of a quad turn their bytes into one
+//     pixel's four channels per lane.
+#include <hip/hip_runtime.h>
+
+#include <limits.h>
+
+#include <algorithm>
+#include <string>
+#include <type_traits>
+
+#include "i8conv_internal.hpp"
+
+namespace i8conv {
+namespace {
+
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+template <int N>
+using Set = std::integral_constant<int, N>;
+
+
+// What the epilogue writes: int32, or requantized int8 (N % 4 == 0).
+enum OutKind { kOutInt32, kOutInt8 };
+
+__device__ __forceinline__ v16i mfma32(v4i a, v4i b, v16i c) {
+  return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+}
+
+// LDS rows of kBytes: logical 16-byte chunk j of row r sits at chunk j ^
+// f(r).  A fragment read has lanes 0..31 on 32 consecutive rows of one chunk
+// and lanes 32..63 on the next chunk: f takes each value once among the rows
+// that share a position modulo 512 bytes, and four consecutive rows differ
+// modulo 128 bytes (the ds_read_b128 rule in i8conv_device.hpp).
+template <int kBytes>
+__device__ __forceinline__ int swz_f(int row) {
+  if constexpr (kBytes == 64) return ((row >> 3) + (row >> 1)) & 3;
+  return ((row >> 2) + 2 * (row & 3)) & 7;
+}
+
+// Byte transpose over the four lanes of a quad: lane k ends with byte k of
+// lanes 0, 1, 2, 3 of its quad, in that order.
+__device__ __forceinline__ uint32_t quad_transpose(uint32_t v, int lane) {
+  // swap across lane bit 0: even lanes keep bytes 0, 2 and take the odd
+  // lane's; odd lanes keep bytes 1, 3
+  const uint32_t a = uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0xb1, 0xf, 0xf, false));  // 1 0 3 2
+  v = __builtin_amdgcn_perm(a, v, lane & 1 ? 0x03070105u : 0x06020400u);
+  // across lane bit 1, in halfwords
+  const uint32_t b = uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x4e, 0xf, 0xf, false));  // 2 3 0 1
+  return __builtin_amdgcn_perm(b, v, lane & 2 ? 0x03020706u : 0x05040100u);
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// at most `stages` stages of CPW copies outstanding (0 <= stages <= MOST)
+template <int CPW, int MOST>
+__device__ __forceinline__ void wait_stages(int stages) {
+  if constexpr (MOST == 0) {
+    wait_vm<0>();
+  } else {
+    if (stages >= MOST)
+      wait_vm<(CPW * MOST < 63 ? CPW * MOST : 63)>();
+    else
+      wait_stages<CPW, MOST - 1>(stages);
+  }
+}
+
+__device__ __forceinline__ void barrier_lds() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// BM pixels x BN channels over WM x WN waves; KS k-steps of 32 bytes per
+// stage, fragments read GS k-steps at a time; R stage buffers; kOcc waves per
+// SIMD.
+template <int BM, int BN, int WM, int WN, int KS, int GS, int R, bool kLaneTap, int kOut,
+          int kPolicy, int kOcc>
+__global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, int tiles) {
+  constexpr int P = 32 * KS;              // bytes per LDS row: one k-stage
+  constexpr int kWaves = WM * WN;
+  constexpr int TM = BM / WM, TN = BN / WN;  // pixels and channels per wave
+  constexpr int FM = TM / 32, FN = TN / 32;  // 32 x 32 blocks per wave
+  constexpr int kTile = (BM + BN) * P;    // bytes per stage buffer
+  constexpr int RPC = 1024 / P;           // rows per 1 KB copy
+  constexpr int CPW = (BM + BN) / RPC / kWaves;  // copies per wave and stage
+  constexpr int CPA = BN / RPC / kWaves;         // of which filter rows
+  constexpr int CPB = CPW - CPA;
+  constexpr bool kByte = kOut != kOutInt32;
+  constexpr int kParams = kByte ? 3 : 1;  // bias, multipliers, shifts
+  constexpr int kParamBytes = kParams * BN * 4;
+  constexpr int ST = FM * FN * (kByte ? 4 : 16);  // stores per wave and tile
+  static_assert(CPA >= 1 && CPB >= 1 && BN % (RPC * kWaves) == 0, "tile shape");
+  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave % WM, wn = wave / WM;
+  const v4u xd = make_desc(a.x, a.x_bytes);
+  const v4u wd = make_desc(a.w, a.w_bytes);
+  const uint32_t lds0 = lds_addr(smem);
+  const uint32_t lds_params = lds0 + R * kTile;
+  int8_t *const params = smem + R * kTile;
+  const int stages = (a.gemm_k + P - 1) / P;
+  const int tiles_n = (a.gemm_n + BN - 1) / BN;
+
+  // this lane's chunk of every row it copies, and its row within a copy
+  const int crow = lane / (P / 16);
+  const int lk = 16 * ((lane % (P / 16)) ^ swz_f<P>(wave * RPC + crow));
+
+  uint32_t abase[CPA];
+  int pix[CPB], iy0[CPB], ix0[CPB];
+  int tile_m = 0, tile_n = 0, m_end = 0;
+
+  auto setup = [&](int t) {
+    tile_m = (t / tiles_n) * a.m_step;
+    tile_n = (t % tiles_n) * BN;
+    m_end = min(a.gemm_m, tile_m + a.m_step);
+#pragma unroll
+    for (int j = 0; j < CPA; ++j) {
+      const int oc = tile_n + (wave + kWaves * j) * RPC + crow;
+      abase[j] = oc < a.gemm_n ? uint32_t(oc) * uint32_t(a.gemm_k) + uint32_t(lk) : kOutOfRange;
+    }
+#pragma unroll
+    for (int j = 0; j < CPB; ++j) {
+      const int m = tile_m + (wave + kWaves * j) * RPC + crow;
+      if (m < m_end) {
+        const int b = int(fast_div(uint32_t(m), a.div_ohw));
+        const int rem = m - b * a.out_h * a.out_w;
+        const int oy = int(fast_div(uint32_t(rem), a.div_ow));
+        const int ox = rem - oy * a.out_w;
+        iy0[j] = oy * a.stride_h - a.pad_h;
+        ix0[j] = ox * a.stride_w - a.pad_w;
+        pix[j] = ((b * a.h + iy0[j]) * a.wd + ix0[j]) * a.c + (kLaneTap ? 0 : lk);
+      } else {
+        iy0[j] = -(1 << 29);
+        ix0[j] = 0;
+        pix[j] = 0;
+      }
+    }
+  };
+
+  // The k-stages of a tile in order, one tap() per stage.  Where a stage
+  // lies inside one tap (C % P == 0) the channel chunk is the outer loop and
+  // the filter taps the inner ones.
+  struct StageTap {
+    int dy, dx, off, k0;
+    bool live;
+  };
+  int next_fy = 0, next_fx = 0, next_ci = 0, next_k = 0;
+  const int row_step = a.dil_h * a.wd * a.c, col_step = a.dil_w * a.c;
+  auto restart = [&]() { next_fy = next_fx = next_ci = next_k = 0; };
+  auto stage_tap = [&]() {
+    StageTap t;
+    if constexpr (kLaneTap) {
+      t.k0 = next_k;
+      const int kk = t.k0 + lk;
+      const int tap = int(fast_div(uint32_t(kk), a.div_c));
+      const int ci = kk - tap * a.c;
+      const int fy = int(fast_div(uint32_t(tap), a.div_s));
+      const int fx = tap - fy * a.s;
+      t.live = kk < a.gemm_k;
+      t.dy = t.live ? fy * a.dil_h : -(1 << 29);
+      t.dx = fx * a.dil_w;
+      t.off = fy * row_step + fx * col_step + ci;
+      next_k += P;
+    } else {
+      t.live = true;
+      t.k0 = (next_fy * a.s + next_fx) * a.c + next_ci;
+      t.dy = next_fy * a.dil_h;
+      t.dx = next_fx * a.dil_w;
+      t.off = (t.dy * a.wd + t.dx) * a.c + next_ci;
+      if (++next_fx == a.s) {
+        next_fx = 0;
+        if (++next_fy == a.r) {
+          next_fy = 0;
+          next_ci += P;
+        }
+      }
+    }
+    return t;
+  };
+  auto copy = [&](const StageTap &t, uint32_t buf, int j) {
+    if (j < CPA) {
+      const uint32_t off = abase[j] + uint32_t(t.k0);
+      lds_copy16(wd, buf + uint32_t(wave + kWaves * j) * 1024u, t.live ? off : kOutOfRange);
+    } else {
+      const int b = j - CPA;
+      const bool ok = unsigned(iy0[b] + t.dy) < unsigned(a.h) && unsigned(ix0[b] + t.dx) < unsigned(a.wd);
+      lds_copy16(xd, buf + uint32_t(wave + kWaves * j) * 1024u,
+                 ok ? uint32_t(pix[b] + t.off) : kOutOfRange);
+    }
+  };
+  // per-channel parameters of the tile at tile_n into parameter slot `slot`
+  auto copy_params = [&](int slot) {
+    if (wave * 64 < BN) {
+      const uint32_t bytes = uint32_t(a.gemm_n) * 4u;
+      const uint32_t off = uint32_t(tile_n + wave * 64 + lane) * 4u;
+      const uint32_t dst = lds_params + uint32_t(slot * kParamBytes) + uint32_t(wave) * 256u;
+      lds_copy4(make_desc(a.bias, bytes), dst, off);
+      if constexpr (kByte) {
+        lds_copy4(make_desc(a.q_mult, bytes), dst + BN * 4u, off);
+        lds_copy4(make_desc(a.q_shift, bytes), dst + BN * 8u, off);
+      }
+    }
+  };
+  auto prologue = [&](int slot) {
+    copy_params(slot);
+    restart();
+#pragma unroll
+    for (int s = 0; s < R; ++s) {
+      if (s >= stages) break;
+      const StageTap t = stage_tap();
+#pragma unroll
+      for (int j = 0; j < CPW; ++j) copy(t, lds0 + uint32_t(s * kTile), j);
+    }
+  };
+
+  // workgroup b runs on XCD b % 8: each XCD walks a contiguous run of tiles
+  const int G = int(gridDim.x);
+  const int xcds = G >= 8 ? 8 : 1;
+  const int xcd = int(blockIdx.x) % xcds;
+  const int step = (G - xcd + xcds - 1) / xcds;  // workgroups on this XCD
+  const int first = int(int64_t(tiles) * xcd / xcds);
+  const int last = int(int64_t(tiles) * (xcd + 1) / xcds);
+  int t = first + int(blockIdx.x) / xcds;
+  if (t >= last) return;
+
+  // fragment read offsets in a stage buffer: row 32 i + lane % 32 of the
+  // wave's filter (or pixel) rows, chunk 2 ks + lane / 32
+  const int frow = lane & 31;
+  const int ff = swz_f<P>(frow);
+  int koff[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) koff[ks] = frow * P + 16 * ((2 * ks + (lane >> 5)) ^ ff);
+  const int abuf = wn * TN * P, bbuf = (BN + wm * TM) * P;
+
+  setup(t);
+  int slot = 0;
+  bool pend = false;  // ST stores of the previous tile follow the prologue's copies
+  prologue(slot);
+  for (;;) {
+    if (pend)
+      wait_vm<(ST < 63 ? ST : 63)>();
+    else
+      wait_stages<CPW, R - 1>(min(R, stages) - 1);
+    barrier_lds();
+
+    v16i acc[FN][FM];
+    const int8_t *const pr = params + slot * kParamBytes;
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+      const int v = *reinterpret_cast<const int *>(pr + (wn * TN + 32 * i + (lane & 31)) * 4);
+      v16i c;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) c[e] = v;
+#pragma unroll
+      for (int j = 0; j < FM; ++j) acc[i][j] = c;
+    }
+    // Fragments of GS k-steps, two sets: one feeds the MFMAs while the other
+    // is read.
+    constexpr int NP = KS / GS;  // sets per stage
+    v4i fa[2][GS][FN], fb[2][GS][FM];
+    auto read = [&](auto set, const int8_t *buf, int part, int q) {
+      const int ks = q / (FN + FM), n = q % (FN + FM);
+      const int8_t *const p = buf + koff[part * GS + ks];
+      if (n < FN)
+        fa[set.value][ks][n] = *reinterpret_cast<const v4i *>(p + abuf + 32 * P * n);
+      else
+        fb[set.value][ks][n - FN] = *reinterpret_cast<const v4i *>(p + bbuf + 32 * P * (n - FN));
+    };
+    constexpr int kMfma = GS * FN * FM;
+    constexpr int kReads = GS * (FN + FM);
+#pragma unroll
+    for (int q = 0; q < kReads; ++q) read(Set<0>{}, smem, 0, q);
+
+    int ring = 0;
+    auto stage = [&](auto first, int s) {
+      const int next = ring + 1 == R ? 0 : ring + 1;
+      const int8_t *const buf = smem + ring * kTile;
+      const int8_t *const nbuf = smem + next * kTile;
+      const bool more = s + R < stages;
+      StageTap tap{};
+      if (more) tap = stage_tap();
+      auto part = [&](auto set, auto last, int pt) {
+        if (last.value) {
+          // every wave has read all of stage s, and stage s + 1 has landed
+          if (s + 1 < stages && !(pend && s + 1 < R))
+            wait_stages<CPW, R - 2>(min(R - 2, stages - 2 - s));
+          barrier_lds();
+        }
+#pragma unroll
+        for (int n = 0; n < kMfma; ++n) {
+#pragma unroll
+          for (int q = n * kReads / kMfma; q < (n + 1) * kReads / kMfma; ++q)
+            read(Set<1 - set.value>{}, last.value ? nbuf : buf, last.value ? 0 : pt + 1, q);
+          if (last.value && more) {
+#pragma unroll
+            for (int q = n * CPW / kMfma; q < (n + 1) * CPW / kMfma; ++q)
+              copy(tap, lds0 + uint32_t(ring * kTile), q);
+          }
+          const int ks = n / (FN * FM), i = n / FM % FN, j = n % FM;
+          acc[i][j] = mfma32(fb[set.value][ks][j], fa[set.value][ks][i], acc[i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      if constexpr (NP == 1) {
+        part(first, std::true_type{}, 0);
+      } else {
+        static_assert(NP % 2 == 0, "one set per stage, or an even number");
+        part(Set<0>{}, std::false_type{}, 0);
+        if constexpr (NP == 4) {
+          part(Set<1>{}, std::false_type{}, 1);
+          part(Set<0>{}, std::false_type{}, 2);
+        }
+        part(Set<1>{}, std::true_type{}, NP - 1);
+      }
+      ring = next;
+    };
+    for (int s = 0; s < stages; ++s) {
+      stage(Set<0>{}, s);
+      if constexpr (NP == 1) {
+        if (++s == stages) break;
+        stage(Set<1>{}, s);
+      }
+    }
+
+    // the next tile's copies go out before this tile's stores
+    const int out_m = tile_m, out_n = tile_n, out_end = m_end;
+    t += step;
+    const bool again = t < last;
+    if (again) {
+      setup(t);
+      prologue(slot ^ 1);
+    }
+    // lane (q, h) holds channel 32 i + q of the pixels 8 g + 4 h + e
+    const int rows = out_end - out_m;
+    const uint32_t pitch = uint32_t(a.gemm_n) * (kByte ? 1u : 4u);
+    const int px0 = wm * TM + 4 * (lane >> 5);
+    const int oc0 = out_n + wn * TN + (lane & 31);
+    if constexpr (!kByte) {
+      const auto yr = make_rsrc(a.y + size_t(out_m) * size_t(a.gemm_n), uint32_t(rows) * pitch);
+#pragma unroll
+      for (int j = 0; j < FM; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int px = px0 + 32 * j + 8 * (e >> 2) + (e & 3);
+          const uint32_t off = uint32_t(px) * pitch + uint32_t(oc0) * 4u;
+#pragma unroll
+          for (int i = 0; i < FN; ++i)
+            __builtin_amdgcn_raw_buffer_store_b32(
+                acc[i][j][e], yr,
+                px < rows && oc0 + 32 * i < a.gemm_n ? off + 128u * i : kOutOfRange, 0, kPolicy);
+        }
+    } else {
+      const auto yr = make_rsrc(a.q_y + size_t(out_m) * size_t(a.gemm_n), uint32_t(rows) * pitch);
+#pragma unroll
+      for (int i = 0; i < FN; ++i) {
+        const int8_t *const pq = pr + (wn * TN + 32 * i + (lane & 31)) * 4;
+        const int m = *reinterpret_cast<const int *>(pq + BN * 4);
+        const int sh = *reinterpret_cast<const int *>(pq + BN * 8);
+        const RequantOdd o = requant_odd_params(m, sh, a.q_zp);
+        const bool odd = __builtin_amdgcn_ballot_w64(!o.ok) == 0;
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            uint32_t y[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              y[e] = uint32_t(odd ? requant1_odd(acc[i][j][4 * g + e], o.mo, o.k, o.sh)
+                                  : requant1(acc[i][j][4 * g + e], m, sh, a.q_zp));
+            const int px = px0 + 32 * j + 8 * g;
+            // four pixels' bytes of one channel per lane, turned into one
+            // pixel's four channels per lane of a quad
+            const uint32_t lo = __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0400u);
+            const uint32_t hi = __builtin_amdgcn_perm(y[3], y[2], 0x0c0c0400u);
+            const uint32_t v = quad_transpose(__builtin_amdgcn_perm(hi, lo, 0x05040100u), lane);
+            const int p = px + (lane & 3), oc = oc0 + 32 * i - (lane & 3);
+            __builtin_amdgcn_raw_buffer_store_b32(
+                v, yr, p < rows && oc < a.gemm_n ? uint32_t(p) * pitch + uint32_t(oc) : kOutOfRange,
+                0, kPolicy);
+          }
+      }
+    }
+    if (!again) return;
+    slot ^= 1;
+    pend = true;
+  }
+}
+
+template <int BM, int BN, int WM, int WN, int GS, bool kLaneTap, int kOcc, int kGroups, int kOut,
+          int kPolicy>
+int launch_tile(const ConvArgs &a, hipStream_t stream) {
+  constexpr int KS = 4, R = 2;
+  auto kern = gemm32_kernel<BM, BN, WM, WN, KS, GS, R, kLaneTap, kOut, kPolicy, kOcc>;
+  const size_t lds = size_t(R) * (BM + BN) * 32 * KS + 2 * (kOut == kOutInt32 ? 1 : 3) * BN * 4;
+  const int tiles = int(((int64_t(a.gemm_m) + BM - 1) / BM) * ((a.gemm_n + BN - 1) / BN));
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    if (e != hipSuccess) {
+      set_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
+      return I8CONV_HIP_ERROR;
+    }
+  }
+  I8_LAUNCH(kern, dim3(unsigned(std::min(tiles, 256 * kGroups))), dim3(64 * WM * WN), lds, stream, a,
+            tiles);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error(std::string("gemm32 kernel launch: ") + hipGetErrorString(e));
+    return I8CONV_HIP_ERROR;
+  }
+  return I8CONV_OK;
+}
+
+// The cache policies of kernel_gemm_dma.hip: int32 write-through where the
+// pixel pitch keeps sectors whole and the output is at most 128 MiB,
+// evict-first above, ordinary for other pitches and for int8.
+template <int BM, int BN, int WM, int WN, int GS, bool kLaneTap, int kOcc, int kGroups>
+int launch_out(const ConvArgs &a, hipStream_t s) {
+  if (a.q_y)
+    return launch_tile<BM, BN, WM, WN, GS, kLaneTap, kOcc, kGroups, kOutInt8, 0>(a, s);
+  if (a.gemm_n % 8 != 0)
+    return launch_tile<BM, BN, WM, WN, GS, kLaneTap, kOcc, kGroups, kOutInt32, 0>(a, s);
+  if (int64_t(a.gemm_m) * a.gemm_n * 4 > kStreamOutputBytes)
+    return launch_tile<BM, BN, WM, WN, GS, kLaneTap, kOcc, kGroups, kOutInt32, kStoreStream>(a, s);
+  return launch_tile<BM, BN, WM, WN, GS, kLaneTap, kOcc, kGroups, kOutInt32, kStoreThrough>(a, s);
+}
+
+}  // namespace
+
+bool gemm32_eligible(const i8conv_geometry &g) {
+  // 32-bit tile and k arithmetic, and a tile's output window below 2 GiB
+  return g.gemm_m <= (1 << 30) && g.gemm_k <= (1 << 30) && g.gemm_n <= (1 << 20) &&
+         ((g.gemm_m + 63) / 64) * ((int64_t(g.gemm_n) + 63) / 64) <= INT32_MAX;
+}
+
+int launch_gemm32(const ConvArgs &args, const GemmPlan &p, void *stream) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  ConvArgs a = args;
+  a.m_step = p.bm;
+  if (a.q_y && a.gemm_n % 4 != 0) {
+    set_error("gemm32: int8 output needs N % 4 == 0");
+    return I8CONV_BAD_ARGUMENT;
+  }
+  switch (p.bm * 1000 + p.bn) {
+    case 64064: return launch_out<64, 64, 2, 2, 2, true, 4, 4>(a, s);
+    case 128064: return launch_out<128, 64, 2, 2, 1, true, 3, 3>(a, s);
+    case 128128: return launch_out<128, 128, 4, 2, 2, true, 4, 2>(a, s);
+    case 256256:
+      // a stage lies inside one tap
+      if (a.c % kStageBytes == 0) return launch_out<256, 256, 4, 2, 1, false, 2, 1>(a, s);
+      break;
+  }
+  set_error("gemm32: unsupported tile " + std::to_string(p.bm) + "x" + std::to_string(p.bn));
+  return I8CONV_BAD_ARGUMENT;
+}
+
+}  // namespace i8conv

@@ -17,6 +17,10 @@
 //      128 tiles: large layers of any filter (it beat every halo/strip plan
 //      from 28x28 x 32 images up to 256x256 x 16, stride 1 or 2, 3x3 or 5x5,
 //      dilated or not);
+//      Likewise the 32 x 32 x 32 MFMA GEMM (C % 128 != 0) wherever it has a
+//      plan: it beat the halo and strip kernels on every such layer (1x3, 64
+//      -> 128: 14.2 against 22.3 us; 256x256, 64 -> 63, 69, 255: 9.3, 11.1,
+//      23 against 16.4, 19.2, 43; dilated 64 -> 128: 5.3 against 6.3);
 //   4. otherwise an input-reuse kernel for a stride-1 spatial filter
 //      (r*s > 1): halo when eligible, else strip (small dilated layers,
 //      asymmetric 1x3/3x1, C = 64 layers wider than the row kernel's four
@@ -78,11 +82,11 @@ int dispatch_uncached(const i8conv_shape &s) {
   const bool halo = plan_halo(s, g, &pp);
   if (halo && pp.row) return I8CONV_KERNEL_HALO;
   const GemmPlan gp = plan_generic(s, g);
-  const int64_t tiles = ((g.gemm_m + gp.bm - 1) / gp.bm) *
-                        ((int64_t(g.gemm_n) + gp.bn - 1) / gp.bn);
+  const int64_t tiles = staged_tiles(s, g);
   const bool spatial = int64_t(s.r) * s.s > 1;
   if (tiles <= 16 && (gp.stages >= 16 || (!spatial && gp.stages >= 8)))
     return I8CONV_KERNEL_SPLITK;
+  if (gp.m32 && !gp.dma) return I8CONV_KERNEL_GENERIC;
   if (gp.dma && tiles >= 128) return I8CONV_KERNEL_GENERIC;
   if (spatial && s.stride_h == 1 && s.stride_w == 1) {
     if (halo) return I8CONV_KERNEL_HALO;

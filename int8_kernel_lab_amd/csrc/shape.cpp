@@ -150,15 +150,11 @@ static bool pointwise_eligible(const i8conv_shape &s, const i8conv_geometry &g) 
          g.gemm_m * s.c < (int64_t(1) << 31) && g.gemm_m * g.gemm_n * 4 < (int64_t(1) << 31);
 }
 
-GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
+static GemmPlan plan_staged(const i8conv_shape &s, const i8conv_geometry &g) {
   GemmPlan p;
   p.stages = int(ceil_div(g.gemm_k, kStageBytes));
   p.splits = 1;
   p.stages_per_split = p.stages;
-  if (pointwise_eligible(s, g)) {
-    p.pw = true;
-    p.pw_waves = pointwise_waves(g.gemm_m, pointwise_slices(s.c, int(g.gemm_n)));
-  }
   if (dma_eligible(s)) {
     p.dma = true;
     p.bn = g.gemm_n <= 64 ? 64 : 128;
@@ -178,6 +174,63 @@ GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
     }
   }
   if (!gemm_tile_supported(p.bm, p.bn)) p.bm = 128;
+  return p;
+}
+
+int64_t staged_tiles(const i8conv_shape &s, const i8conv_geometry &g) {
+  const GemmPlan p = plan_staged(s, g);
+  return ceil_div(g.gemm_m, p.bm) * ceil_div(g.gemm_n, p.bn);
+}
+
+// Which kernel runs a generic layer, and on which tile (microseconds per
+// back-to-back launch on one MI355X, before -> after unless said otherwise).
+// C % 128 != 0: the 32 x 32 x 32 MFMA kernel instead of the register-staged
+// one, on the largest tile that keeps the compute units covered:
+//   * 128 x 128, two workgroups per unit, for N > 64 with at least 256 tiles
+//     (256x256, 64 -> 255 3x3: 43 -> 23; 7 x 196x196, 80 -> 209 1x3: 202 ->
+//     59; 16 x 224x224, 32 -> 96 4x4 stride 4: 15.8 -> 8.6, 64 x 64: 10.0);
+//   * 128 x 64, three per unit, with at least 512 tiles (16 x 224x224, 32 ->
+//     64 7x7 stride 2: 101 -> 35; 256x256, 64 -> 63: 16.4 -> 9.3);
+//   * 64 x 64, four per unit, below that (416x416, 32 -> 64 3x3 stride 2: 7.3
+//     -> 5.9, 128 x 64: 7.6; 4 x 28x28, 192 -> 192 3x3: 19.9 -> 12.6);
+//   * the register-staged kernel keeps layers of at most 64 channels and one
+//     round of 64-pixel tiles: each of its stages costs less where a unit
+//     has one tile (7 x 38x38, 288 -> 32 3x3: 12.5 against 17.8; 224x224, 32
+//     -> 64 7x7 stride 2: 10.8 against 12.5).
+// C % 128 == 0: the pipelined kernel, except
+//   * grids of fewer than 128 of its tiles, which leave half the units idle:
+//     64 x 64 (52x52, 256 -> 512 3x3 stride 2: 12.7 -> 9.3);
+//   * at least two rounds of 256 x 256 tiles: a third fewer copied bytes per
+//     operation (16 x 256x256, 256 -> 256 3x3: 780 -> 706; 5x5 stride 2 with
+//     int8 output: 484 -> 457).
+GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
+  GemmPlan p = plan_staged(s, g);
+  if (pointwise_eligible(s, g)) {
+    p.pw = true;
+    p.pw_waves = pointwise_waves(g.gemm_m, pointwise_slices(s.c, int(g.gemm_n)));
+    if (p.dma) return p;  // the fallback for unaligned pointers stays pipelined
+  }
+  if (!gemm32_eligible(g)) return p;
+  auto tiles = [&](int bm, int bn) { return ceil_div(g.gemm_m, bm) * ceil_div(g.gemm_n, bn); };
+  int bm = 0, bn = 0;
+  if (p.dma) {
+    if (g.gemm_n > 128 && p.stages >= 8 && tiles(256, 256) >= 512)
+      bm = bn = 256;
+    else if (tiles(p.bm, p.bn) < 128)
+      bm = bn = 64;
+  } else if (g.gemm_n > 64 && tiles(128, 128) >= 256) {
+    bm = bn = 128;
+  } else if (tiles(128, 64) >= 512) {
+    bm = 128, bn = 64;
+  } else if (g.gemm_n > 64 || tiles(64, 64) > 256) {
+    bm = bn = 64;
+  }
+  if (bm > 0) {
+    p.m32 = true;
+    p.bm = bm;
+    p.bn = bn;
+    p.m_step = bm;
+  }
   return p;
 }
 

@@ -1,0 +1,83 @@
+"""The generic kernel's 32 x 32 x 32 MFMA form, bit-exact against the oracle
+with int32 and int8 output: each of its tiles at their edges (pixel and channel
+tails, a k tail inside a stage, stages that span taps), through `generic` and
+through the dispatched requantized launch."""
+import numpy as np
+import pytest
+
+import int8_kernel_lab_amd as lab
+from oracle import oracle
+from tests.conftest import say
+from tests.test_gpu_parity import assert_bit_exact, run_kernel
+from tests.test_requant import _qparams
+
+CASES = {
+    # 64 x 64: one pixel past a tile and one channel past a tile, C = 80;
+    # C = 16 with 27 bytes short of two stages; a strided C = 384 layer whose
+    # pipelined grid would be small; gemm_k of exactly one stage
+    "64_m65_n65_c80": ("64px x 64oc", lab.ConvShape(1, 5, 13, 80, 65, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "64_c16_5x3": ("64px x 64oc", lab.ConvShape(3, 19, 23, 16, 68, 5, 3, 2, 0, 2, 1, 1, 2)),
+    "64_c384_s2": ("64px x 64oc", lab.ConvShape(2, 23, 21, 384, 132, 3, 3, 1, 1, 2, 2, 1, 1)),
+    "64_k128": ("64px x 64oc", lab.ConvShape(18, 31, 33, 32, 36, 2, 2, 0, 0, 1, 1, 1, 1)),
+    # 128 x 64: C = 32 and 48, odd channel counts, padding wider than the image
+    "128x64_c32_k63": ("128px x 64oc", lab.ConvShape(5, 121, 119, 32, 63, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "128x64_c48_k4": ("128px x 64oc", lab.ConvShape(1, 250, 263, 48, 4, 7, 7, 3, 3, 1, 1, 1, 1)),
+    # 128 x 128: N = 65 and 255 (one, then two channel tiles), 1x3 dilated
+    "128_k65": ("128px x 128oc", lab.ConvShape(2, 129, 130, 64, 65, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "128_k255": ("128px x 128oc", lab.ConvShape(1, 130, 131, 64, 255, 1, 3, 0, 2, 1, 1, 1, 2)),
+    "128_k260": ("128px x 128oc", lab.ConvShape(1, 123, 125, 112, 260, 1, 1, 0, 0, 1, 1, 1, 1)),
+    # 256 x 256: 514 tiles (two full rounds and a partial one), N = 132
+    "256_k132": ("256px x 256oc", lab.ConvShape(2, 256, 257, 128, 132, 3, 3, 1, 1, 1, 1, 1, 1)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_gemm32_runs_these_layers(name):
+    tile, shape = CASES[name]
+    assert f"32x32 MFMA tile {tile}" in lab.describe("generic", shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_gemm32_bit_exact(name):
+    _, shape = CASES[name]
+    x, w, b = lab.make_case_data(shape, seed=31)
+    expected = oracle.conv(shape, x, w, b)
+    say(f"[gpu] generic (32x32 MFMA) on {name} {shape}")
+    assert_bit_exact(run_kernel("generic", shape, x, w, b), expected, name)
+    if lab.dispatch(shape) != "generic":
+        return
+    for seed, zp in ((32, 5), (None, -9)):
+        if seed is None:
+            # every channel in the odd-multiplier form's domain
+            rng = np.random.default_rng(33)
+            mult = (rng.integers(2 ** 29, 2 ** 30, size=shape.k) * 2 + 1).astype(np.int32)
+            shift = rng.integers(44, 47, size=shape.k).astype(np.int32)
+        else:
+            mult, shift = _qparams(shape.k, seed=seed)
+        say(f"[gpu] requantized, seed {seed}")
+        got = lab.conv2d_requant(x, w, b, mult, shift, zp, shape)
+        np.testing.assert_array_equal(got, oracle.requantize(expected, mult, shift, zp))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["64_m65_n65_c80", "128_k260"])
+def test_gemm32_output_at_four_bytes(name):
+    # an output 4 bytes past an allocation's start, nothing written around it
+    _, shape = CASES[name]
+    x, w, b = lab.make_case_data(shape, seed=34)
+    count = shape.output_elements
+    bufs = [lab.DeviceBuffer.from_array(a) for a in (x, w, b)]
+    yb = lab.DeviceBuffer(4 * count + 16)
+    try:
+        yb.fill(0xA5)
+        say(f"[gpu] generic (32x32 MFMA) on {name} with the output at +4 bytes")
+        lab.launch("generic", shape, *bufs, yb.ptr + 4)
+        lab.synchronize()
+        raw = yb.download(np.int32, count + 4)
+    finally:
+        for buf in bufs + [yb]:
+            buf.close()
+    poison = np.uint32(0xA5A5A5A5).view(np.int32)
+    assert raw[0] == poison and np.all(raw[count + 1:] == poison)
+    assert_bit_exact(raw[1:count + 1].reshape(shape.output_shape), oracle.conv(shape, x, w, b), name)
