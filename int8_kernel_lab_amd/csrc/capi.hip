@@ -761,6 +761,16 @@ int i8conv_launch_requant(const i8conv_shape *shape, const int8_t *input, const 
       return launch_gemm32(args, p, stream);
     }
   }
+  // The row kernel likewise (32 x 56x56, 64 -> 64: 10.5 + 8.1 us with the
+  // pass).
+  if (id == I8CONV_KERNEL_HALO) {
+    PatchPlan pp;
+    if (plan_halo(*shape, g, &pp) && pp.row && !pp.streamed) {
+      const ConvArgs args = make_args(*shape, g, input, filter, bias, nullptr);
+      const RequantArgs q{mult, shift, zero_point, output};
+      return launch_row(args, pp, stream, &q);
+    }
+  }
   int32_t *acc = static_cast<int32_t *>(workspace);
   void *conv_ws = static_cast<char *>(workspace) + acc_bytes;
   const int r = i8conv_launch(id, shape, input, filter, bias, acc, conv_ws,

@@ -186,7 +186,6 @@ bool pointwise_pointers_ok(const ConvArgs &a);
 bool pointwise_requant_supported(int c, int n);
 int launch_patch(const ConvArgs &a, const PatchPlan &p, void *stream);
 int launch_halo_resident(const ConvArgs &a, const PatchPlan &p, void *stream);
-int launch_row(const ConvArgs &a, const PatchPlan &p, void *stream);
 // Requantized int8 output (kernel_requant.hip): per output channel k,
 // y = clamp(zero_point + round(acc * mult[k] / 2^shift[k]), -128, 127).
 struct RequantArgs {
@@ -195,6 +194,9 @@ struct RequantArgs {
   int32_t zero_point;
   int8_t *y;  // NHWK int8
 };
+// q: requantized int8 output instead of int32 (any N and alignment)
+int launch_row(const ConvArgs &a, const PatchPlan &p, void *stream,
+               const RequantArgs *q = nullptr);
 int launch_requant(const int32_t *acc, int64_t pixels, int32_t channels, const int32_t *mult,
                    const int32_t *shift, int32_t zero_point, int8_t *out, void *stream);
 // kernel_layout.hip: batched [rows][cols] -> [cols][rows] of esize-byte

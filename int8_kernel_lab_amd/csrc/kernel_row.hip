@@ -31,6 +31,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "halo_common.hpp"
 
@@ -44,25 +45,36 @@ struct RowArgs {
   int n, out_h, out_w, gemm_n;
   int row_bytes;    // LDS bytes between consecutive rows
 };
+// ... and of the requantizing form (int8 output: y unused)
+struct RowQuantArgs : RowArgs {
+  int32_t zp;
+  const int32_t *mult, *shift;
+  int8_t *q;
+};
+// kPolicy of the requantizing form
+constexpr int kRowQuant = -1;
+template <int kPolicy>
+using RowArgsOf = std::conditional_t<kPolicy == kRowQuant, RowQuantArgs, RowArgs>;
 
-// RowArgs, the kernel's last argument, read from the kernel-argument segment
+// RowArgs (or RowQuantArgs), the kernel's last argument, read from the kernel-argument segment
 // where it is called.  The segment pointer passes through an empty asm, so
 // the compiler cannot hoist the loads to the kernel's entry, where they would
 // hold SGPRs that the copy code reuses and make it wait for them (~0.3 us)
 // before its first copy.  The offset: three 8-byte pointers and five 4-byte
 // words, rounded up to the struct's 8-byte alignment.
 constexpr uint32_t kRowArgsOffset = (3 * 8 + 5 * 4 + 7) / 8 * 8;
-static_assert(alignof(RowArgs) == 8, "RowArgs offset assumes 8-byte alignment");
-__device__ __forceinline__ RowArgs row_args() {
+static_assert(alignof(RowArgs) == 8 && alignof(RowQuantArgs) == 8, "8-byte aligned arguments");
+template <class Args>
+__device__ __forceinline__ Args row_args() {
   uint64_t kp = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
   asm volatile("" : "+s"(kp));
   const auto *src =
       reinterpret_cast<const __attribute__((address_space(4))) uint32_t *>(kp + kRowArgsOffset);
-  static_assert(sizeof(RowArgs) % 4 == 0, "argument block of whole words");
-  uint32_t w[sizeof(RowArgs) / 4];
+  static_assert(sizeof(Args) % 4 == 0, "argument block of whole words");
+  uint32_t w[sizeof(Args) / 4];
 #pragma unroll
-  for (int i = 0; i < int(sizeof(RowArgs) / 4); ++i) w[i] = src[i];
-  RowArgs r;
+  for (int i = 0; i < int(sizeof(Args) / 4); ++i) w[i] = src[i];
+  Args r;
   __builtin_memcpy(&r, w, sizeof(r));
   return r;
 }
@@ -115,6 +127,15 @@ struct RowState {
   int colofs[3][NFR];       // LDS offset of this lane's column + fx / k-block in a row
 };
 
+// Requantization of a lane's four channels per fragment (RowQuantArgs): the
+// odd-multiplier form's constants where the wave's channels all allow it,
+// else the plain multipliers and shifts.
+template <int FN>
+struct RowQuant {
+  v4i m[FN], k[FN], sh[FN];
+  bool odd;
+};
+
 // Input row ir (K == ir % 3, compile time, fixes the accumulator roles):
 // the fragments of every channel group at the three column offsets fx, and
 // the filter rows fy in MASK (bit fy; compile time, so the MFMAs of a row
@@ -129,7 +150,8 @@ struct RowState {
 // is hidden behind MFMAs instead of stalling them.  The last input row (only
 // filter row 2 left: MASK 4, or 7 in a one-row block) reads row 0 again.
 template <int FN, int CG, int NFR, int kPolicy, int K, int MASK, bool kCheck>
-__device__ __forceinline__ void row_step(const RowArgs &p, RowState<FN, CG, NFR> &st,
+__device__ __forceinline__ void row_step(const RowArgsOf<kPolicy> &p, RowState<FN, CG, NFR> &st,
+                                         const RowQuant<FN> &rq,
                                          v4i (&frag)[3][NFR], const int8_t *rows,
                                          const int8_t *bias_lds, int ir, int rows_out,
                                          int m_row0, int tile_n, int wave, int lane) {
@@ -192,6 +214,32 @@ __device__ __forceinline__ void row_step(const RowArgs &p, RowState<FN, CG, NFR>
   for (int i = 0; i < FN; ++i)
     bv[i] = *reinterpret_cast<const v4i *>(bias_lds + (i * 16 + 4 * (lane >> 4)) * 4);
   const int m_row = m_row0 + (ir - 2) * p.out_w;
+  if constexpr (kPolicy == kRowQuant) {
+    // four channels of a pixel as one 4-byte store (a wave's 16 channels of a
+    // pixel by four lanes; ordinary, merged into lines in the L2)
+    const bool vec = (p.gemm_n & 3) == 0 && (reinterpret_cast<uintptr_t>(p.q) & 3) == 0;
+#pragma unroll
+    for (int j = 0; j < NFR; ++j) {
+      const int col = 16 * j + (lane & 15);
+      if (col >= p.out_w) continue;
+#pragma unroll
+      for (int i = 0; i < FN; ++i) {
+        const int oc0 = tile_n + wave * 16 * FN + i * 16 + 4 * (lane >> 4);
+        const v4i v = add_wrap4(st.acc[s2][j][i], bv[i]);
+        const uint32_t y = rq.odd ? requant4_odd(v, rq.m[i], rq.k[i], rq.sh[i])
+                                  : requant4(v, rq.m[i], rq.sh[i], p.zp);
+        int8_t *dst = p.q + size_t(m_row + col) * size_t(p.gemm_n) + oc0;
+        if (vec) {
+          if (oc0 < p.gemm_n) *reinterpret_cast<uint32_t *>(dst) = y;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (oc0 + e < p.gemm_n) dst[e] = int8_t(y >> (8 * e));
+        }
+      }
+    }
+    return;
+  } else {
   // output window: this output row's out_w pixels
   const OutWindow ow = out_window(p.y, int64_t(p.n) * p.out_h * p.out_w, p.gemm_n, m_row, p.out_w);
   const bool vec = (p.gemm_n & 3) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && ow.ok;
@@ -213,6 +261,7 @@ __device__ __forceinline__ void row_step(const RowArgs &p, RowState<FN, CG, NFR>
           if (oc0 + e < p.gemm_n) store_out1(dst + e, v[e]);
       }
     }
+  }
   }
 }
 
@@ -236,7 +285,8 @@ __device__ __forceinline__ void take_chunks(FilterRing<FN, 9 * CG> &ring,
 template <int FN, int CG, int NFR, int kPolicy>
 __global__ __launch_bounds__(kThreads, 1) void row_kernel(
     const int8_t *x_pre, const int8_t *w_pre, const int32_t *bias_pre, uint32_t n_pre,
-    uint32_t hw_pre, uint32_t pads_pre, uint32_t gemm_n_pre, uint32_t ring_pre, RowArgs p_arg) {
+    uint32_t hw_pre, uint32_t pads_pre, uint32_t gemm_n_pre, uint32_t ring_pre,
+    RowArgsOf<kPolicy> p_arg) {
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   (void)p_arg;  // read through row_args() once the copies are issued
   constexpr int kSteps = 9 * CG;
@@ -309,8 +359,37 @@ __global__ __launch_bounds__(kThreads, 1) void row_kernel(
   }
   for (int c = 0; c < ring.slots && c < kChunks; ++c) ring.issue(c, c);
 
-  const RowArgs p = row_args();
+  const auto p = row_args<RowArgsOf<kPolicy>>();
   pin_sgprs(p);
+  RowQuant<FN> rq;
+  if constexpr (kPolicy == kRowQuant) {
+    bool odd = true;
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+      const int oc0 = tile_n + wave * 16 * FN + i * 16 + 4 * (lane >> 4);
+      rq.m[i] = load_bias4(p.mult, gemm_n, oc0);
+      rq.sh[i] = load_bias4(p.shift, gemm_n, oc0);
+    }
+    v4i mo[FN], sh[FN];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const RequantOdd o = requant_odd_params(rq.m[i][e], rq.sh[i][e], p.zp);
+        odd = odd && o.ok;
+        mo[i][e] = o.mo;
+        rq.k[i][e] = o.k;
+        sh[i][e] = o.sh;
+      }
+    rq.odd = __builtin_amdgcn_ballot_w64(!odd) == 0;
+    if (rq.odd) {
+#pragma unroll
+      for (int i = 0; i < FN; ++i) {
+        rq.m[i] = mo[i];
+        rq.sh[i] = sh[i];
+      }
+    }
+  }
   RowState<FN, CG, NFR> st;
 #pragma unroll
   for (int fx = 0; fx < 3; ++fx)
@@ -330,7 +409,7 @@ __global__ __launch_bounds__(kThreads, 1) void row_kernel(
   // taking chunk 0 also publishes the input rows (its barrier).
   constexpr int kC1 = (3 * CG + 1) / 2, kC2 = (6 * CG + 1) / 2;
 #define I8_ROW(K, MASK, CHECK, IR)                                                         \
-  row_step<FN, CG, NFR, kPolicy, K, MASK, CHECK>(p, st, frag, rows, bias_lds, IR, rows_out, m_row0, \
+  row_step<FN, CG, NFR, kPolicy, K, MASK, CHECK>(p, st, rq, frag, rows, bias_lds, IR, rows_out, m_row0, \
                                         tile_n, wave, lane)
   take_chunks<FN, CG, NFR, 0, kC1>(ring, st);
   v4i frag[3][NFR];
@@ -387,10 +466,9 @@ struct RowPre {
   uint32_t n, hw, pads, gemm_n, ring;
 };
 
-template <int FN, int CG, int NFR>
-int launch_t(const RowPre &a, const RowArgs &h, dim3 grid, size_t lds, hipStream_t s) {
-  auto kern = (h.gemm_n & 7) == 0 ? row_kernel<FN, CG, NFR, kStoreThrough>
-                                  : row_kernel<FN, CG, NFR, 0>;
+template <int FN, int CG, int NFR, int kPolicy>
+int launch_policy(const RowPre &a, const RowArgsOf<kPolicy> &h, dim3 grid, size_t lds, hipStream_t s) {
+  auto kern = row_kernel<FN, CG, NFR, kPolicy>;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -410,6 +488,13 @@ int launch_t(const RowPre &a, const RowArgs &h, dim3 grid, size_t lds, hipStream
   return I8CONV_OK;
 }
 
+template <int FN, int CG, int NFR>
+int launch_t(const RowPre &a, const RowQuantArgs &h, dim3 grid, size_t lds, hipStream_t s) {
+  if (h.q) return launch_policy<FN, CG, NFR, kRowQuant>(a, h, grid, lds, s);
+  if ((h.gemm_n & 7) == 0) return launch_policy<FN, CG, NFR, kStoreThrough>(a, h, grid, lds, s);
+  return launch_policy<FN, CG, NFR, 0>(a, h, grid, lds, s);
+}
+
 }  // namespace
 
 bool row_instance_exists(int fn, int cg, int nfr) {
@@ -420,7 +505,7 @@ bool row_instance_exists(int fn, int cg, int nfr) {
          (fn == 1 && (cg == 1 || cg == 2 || (cg == 4 && nfr <= 2)));
 }
 
-int launch_row(const ConvArgs &a, const PatchPlan &p, void *stream) {
+int launch_row(const ConvArgs &a, const PatchPlan &p, void *stream, const RequantArgs *q) {
   const int fn = p.bn / 64;
   const int cg = a.c / 64;
   const int nfr = (a.out_w + 15) / 16;
@@ -451,7 +536,13 @@ int launch_row(const ConvArgs &a, const PatchPlan &p, void *stream) {
   pre.pads = uint32_t(a.pad_h) | uint32_t(a.pad_w) << 8 | uint32_t(p.ranges) << 16;
   pre.gemm_n = uint32_t(a.gemm_n);
   pre.ring = uint32_t(p.ring) | uint32_t(p.rows) << 8;
-  RowArgs h{};
+  RowQuantArgs h{};
+  if (q) {
+    h.mult = q->mult;
+    h.shift = q->shift;
+    h.zp = q->zero_point;
+    h.q = q->y;
+  }
   h.y = a.y;
   h.n = a.n;
   h.out_h = a.out_h;
