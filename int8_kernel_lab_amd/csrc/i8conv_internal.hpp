@@ -4,6 +4,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <string>
 
 #include "i8conv.h"
@@ -227,6 +228,32 @@ int wait_spin_limit();
 // by the first kernel launched and cleared, `stop` by every kernel launched
 // while it is set (the last one's end stands).  Both null otherwise.
 #ifdef __HIPCC__
+// A kernel's dynamic LDS limit, raised to the budget once per device: the
+// attribute call is part of every launch's host time otherwise.  One object
+// per kernel (a function-local static of its launcher).
+class LdsLimit {
+ public:
+  template <class Kernel>
+  int raise(Kernel kern, size_t lds) {
+    if (lds <= 64 * 1024) return I8CONV_OK;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    const uint64_t bit = e == hipSuccess && dev >= 0 && dev < 64 ? uint64_t(1) << dev : 0;
+    if (bit && (raised_.load(std::memory_order_relaxed) & bit)) return I8CONV_OK;
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBudget);
+    if (e != hipSuccess) {
+      set_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
+      return I8CONV_HIP_ERROR;
+    }
+    raised_.fetch_or(bit, std::memory_order_relaxed);
+    return I8CONV_OK;
+  }
+
+ private:
+  std::atomic<uint64_t> raised_{0};
+};
+
 struct LaunchEvents {
   hipEvent_t start = nullptr;
   hipEvent_t stop = nullptr;

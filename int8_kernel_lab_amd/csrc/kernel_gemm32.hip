@@ -426,14 +426,8 @@ int launch_tile(const ConvArgs &a, hipStream_t stream) {
   auto kern = gemm32_kernel<BM, BN, WM, WN, KS, GS, R, kLaneTap, kOut, kPolicy, kOcc>;
   const size_t lds = size_t(R) * (BM + BN) * 32 * KS + 2 * (kOut == kOutInt32 ? 1 : 3) * BN * 4;
   const int tiles = int(((int64_t(a.gemm_m) + BM - 1) / BM) * ((a.gemm_n + BN - 1) / BN));
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-    if (e != hipSuccess) {
-      set_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
-      return I8CONV_HIP_ERROR;
-    }
-  }
+  static LdsLimit limit;
+  if (const int rc = limit.raise(kern, lds); rc != I8CONV_OK) return rc;
   I8_LAUNCH(kern, dim3(unsigned(std::min(tiles, 256 * kGroups))), dim3(64 * WM * WN), lds, stream, a,
             tiles);
   const hipError_t e = hipGetLastError();

@@ -425,14 +425,8 @@ int launch_tile(const ConvArgs &a, int splits, hipStream_t stream) {
   const size_t lds = size_t(ring) * size_t(BM + BN) * kStageBytes;
   auto kern = splits > 1 ? gemm_dma_kernel<BM, BN, WM, WN, true, NCW>
                          : gemm_dma_kernel<BM, BN, WM, WN, false, NCW>;
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-    if (e != hipSuccess) {
-      set_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
-      return I8CONV_HIP_ERROR;
-    }
-  }
+  static LdsLimit limits[2];
+  if (const int rc = limits[splits > 1].raise(kern, lds); rc != I8CONV_OK) return rc;
   I8_LAUNCH(kern, dim3(unsigned(tiles), unsigned(splits)), dim3(64 * (WM * WN + NCW)),
                      lds, stream, a);
   const hipError_t e = hipGetLastError();

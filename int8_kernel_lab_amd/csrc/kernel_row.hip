@@ -469,15 +469,8 @@ struct RowPre {
 template <int FN, int CG, int NFR, int kPolicy>
 int launch_policy(const RowPre &a, const RowArgsOf<kPolicy> &h, dim3 grid, size_t lds, hipStream_t s) {
   auto kern = row_kernel<FN, CG, NFR, kPolicy>;
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             int(lds));
-    if (e != hipSuccess) {
-      set_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
-      return I8CONV_HIP_ERROR;
-    }
-  }
+  static LdsLimit limit;
+  if (const int rc = limit.raise(kern, lds); rc != I8CONV_OK) return rc;
   I8_LAUNCH(kern, grid, dim3(kThreads), lds, s, a.x, a.w, a.bias, a.n, a.hw, a.pads,
                      a.gemm_n, a.ring, h);
   const hipError_t e = hipGetLastError();

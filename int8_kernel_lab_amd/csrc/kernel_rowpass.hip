@@ -791,15 +791,8 @@ struct PreArgs {
 template <int R, int NFR, bool kQ>
 int launch_q(const PreArgs &a, const PassArgs &h, dim3 grid, size_t lds, hipStream_t s) {
   auto kern = rowpass_kernel<R, NFR, walk_groups(NFR), kQ>;
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             int(lds));
-    if (e != hipSuccess) {
-      set_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
-      return I8CONV_HIP_ERROR;
-    }
-  }
+  static LdsLimit limit;
+  if (const int rc = limit.raise(kern, lds); rc != I8CONV_OK) return rc;
   I8_LAUNCH(kern, grid, dim3(2 * kThreads), lds, s, a.x, a.w, a.bias, a.n, a.hw, a.pads,
                      a.gemm_n, h);
   const hipError_t e = hipGetLastError();
