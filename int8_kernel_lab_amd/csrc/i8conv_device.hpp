@@ -400,10 +400,8 @@ I8_HD inline int swz128_chunk(int row, int phys) { return phys ^ swz128_f(row); 
 // The XOR-of-row-bits layout of 128-byte rows: chunk j of row r at
 // r*128 + 16*(j ^ (r & 7) ^ ((r >> 3) & 1)).  Each 16 lanes of a fragment
 // read cover all sixteen 4-bank groups, but it breaks the 32-lane
-// condition: fragment reads are 2-way conflicts.  The pipelined GEMM keeps
-// it all the same: there the conflict-free swz128 measured 1-2 % slower
-// (A/B, configs 3 and 5b and 256x256 layers; the GEMM's time is not in its
-// LDS reads), so swz128x is its layout.  Its own inverse.
+// condition: fragment reads are 2-way conflicts.  Kept as the counterexample
+// of the layout check; no kernel uses it.  Its own inverse.
 I8_HD inline int swz128x(int row, int chunk) {
   return row * 128 + ((chunk ^ (row & 7) ^ ((row >> 3) & 1)) << 4);
 }

@@ -37,11 +37,10 @@
 #include <type_traits>
 
 #include "i8conv_internal.hpp"
+#include "mfma32_tile.hpp"
 
 namespace i8conv {
 namespace {
-
-typedef int v16i __attribute__((ext_vector_type(16)));
 
 template <int N>
 using Set = std::integral_constant<int, N>;
@@ -49,33 +48,6 @@ using Set = std::integral_constant<int, N>;
 
 // What the epilogue writes: int32, or requantized int8 (N % 4 == 0).
 enum OutKind { kOutInt32, kOutInt8 };
-
-__device__ __forceinline__ v16i mfma32(v4i a, v4i b, v16i c) {
-  return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
-}
-
-// LDS rows of kBytes: logical 16-byte chunk j of row r sits at chunk j ^
-// f(r).  A fragment read has lanes 0..31 on 32 consecutive rows of one chunk
-// and lanes 32..63 on the next chunk: f takes each value once among the rows
-// that share a position modulo 512 bytes, and four consecutive rows differ
-// modulo 128 bytes (the ds_read_b128 rule in i8conv_device.hpp).
-template <int kBytes>
-__device__ __forceinline__ int swz_f(int row) {
-  if constexpr (kBytes == 64) return ((row >> 3) + (row >> 1)) & 3;
-  return ((row >> 2) + 2 * (row & 3)) & 7;
-}
-
-// Byte transpose over the four lanes of a quad: lane k ends with byte k of
-// lanes 0, 1, 2, 3 of its quad, in that order.
-__device__ __forceinline__ uint32_t quad_transpose(uint32_t v, int lane) {
-  // swap across lane bit 0: even lanes keep bytes 0, 2 and take the odd
-  // lane's; odd lanes keep bytes 1, 3
-  const uint32_t a = uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0xb1, 0xf, 0xf, false));  // 1 0 3 2
-  v = __builtin_amdgcn_perm(a, v, lane & 1 ? 0x03070105u : 0x06020400u);
-  // across lane bit 1, in halfwords
-  const uint32_t b = uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x4e, 0xf, 0xf, false));  // 2 3 0 1
-  return __builtin_amdgcn_perm(b, v, lane & 2 ? 0x03020706u : 0x05040100u);
-}
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -101,13 +73,13 @@ __device__ __forceinline__ void barrier_lds() {
   asm volatile("" ::: "memory");
 }
 
-// BM pixels x BN channels over WM x WN waves; KS k-steps of 32 bytes per
-// stage, fragments read GS k-steps at a time; R stage buffers; kOcc waves per
-// SIMD.
-template <int BM, int BN, int WM, int WN, int KS, int GS, int R, bool kLaneTap, int kOut,
-          int kPolicy, int kOcc>
+// BM pixels x BN channels over WM x WN waves; fragments read GS k-steps of 32
+// bytes at a time; R stage buffers; kOcc waves per SIMD.
+template <int BM, int BN, int WM, int WN, int GS, int R, bool kLaneTap, int kOut, int kPolicy,
+          int kOcc>
 __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, int tiles) {
-  constexpr int P = 32 * KS;              // bytes per LDS row: one k-stage
+  constexpr int P = kStageBytes;             // bytes per LDS row: one k-stage
+  constexpr int KS = P / 32;                 // k-steps per stage
   constexpr int kWaves = WM * WN;
   constexpr int TM = BM / WM, TN = BN / WN;  // pixels and channels per wave
   constexpr int FM = TM / 32, FN = TN / 32;  // 32 x 32 blocks per wave
@@ -136,7 +108,7 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
 
   // this lane's chunk of every row it copies, and its row within a copy
   const int crow = lane / (P / 16);
-  const int lk = 16 * ((lane % (P / 16)) ^ swz_f<P>(wave * RPC + crow));
+  const int lk = 16 * ((lane % (P / 16)) ^ swz32_f(wave * RPC + crow));
 
   uint32_t abase[CPA];
   int pix[CPB], iy0[CPB], ix0[CPB];
@@ -259,7 +231,7 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
   // fragment read offsets in a stage buffer: row 32 i + lane % 32 of the
   // wave's filter (or pixel) rows, chunk 2 ks + lane / 32
   const int frow = lane & 31;
-  const int ff = swz_f<P>(frow);
+  const int ff = swz32_f(frow);
   int koff[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) koff[ks] = frow * P + 16 * ((2 * ks + (lane >> 5)) ^ ff);
@@ -363,54 +335,24 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
       setup(t);
       prologue(slot ^ 1);
     }
-    // lane (q, h) holds channel 32 i + q of the pixels 8 g + 4 h + e
     const int rows = out_end - out_m;
-    const uint32_t pitch = uint32_t(a.gemm_n) * (kByte ? 1u : 4u);
-    const int px0 = wm * TM + 4 * (lane >> 5);
-    const int oc0 = out_n + wn * TN + (lane & 31);
+    const int px0 = wm * TM, oc0 = out_n + wn * TN;
     if constexpr (!kByte) {
-      const auto yr = make_rsrc(a.y + size_t(out_m) * size_t(a.gemm_n), uint32_t(rows) * pitch);
-#pragma unroll
-      for (int j = 0; j < FM; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int px = px0 + 32 * j + 8 * (e >> 2) + (e & 3);
-          const uint32_t off = uint32_t(px) * pitch + uint32_t(oc0) * 4u;
-#pragma unroll
-          for (int i = 0; i < FN; ++i)
-            __builtin_amdgcn_raw_buffer_store_b32(
-                acc[i][j][e], yr,
-                px < rows && oc0 + 32 * i < a.gemm_n ? off + 128u * i : kOutOfRange, 0, kPolicy);
-        }
+      const auto yr = make_rsrc(a.y + size_t(out_m) * size_t(a.gemm_n),
+                                uint32_t(rows) * uint32_t(a.gemm_n) * 4u);
+      store_tile32<kPolicy>(acc, yr, rows, px0, oc0, a.gemm_n, lane);
     } else {
-      const auto yr = make_rsrc(a.q_y + size_t(out_m) * size_t(a.gemm_n), uint32_t(rows) * pitch);
+      const auto yr = make_rsrc(a.q_y + size_t(out_m) * size_t(a.gemm_n),
+                                uint32_t(rows) * uint32_t(a.gemm_n));
 #pragma unroll
       for (int i = 0; i < FN; ++i) {
         const int8_t *const pq = pr + (wn * TN + 32 * i + (lane & 31)) * 4;
-        const int m = *reinterpret_cast<const int *>(pq + BN * 4);
-        const int sh = *reinterpret_cast<const int *>(pq + BN * 8);
-        const RequantOdd o = requant_odd_params(m, sh, a.q_zp);
-        const bool odd = __builtin_amdgcn_ballot_w64(!o.ok) == 0;
+        const Requant32 r = requant32_params(*reinterpret_cast<const int *>(pq + BN * 4),
+                                             *reinterpret_cast<const int *>(pq + BN * 8), a.q_zp);
 #pragma unroll
         for (int j = 0; j < FM; ++j)
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            uint32_t y[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              y[e] = uint32_t(odd ? requant1_odd(acc[i][j][4 * g + e], o.mo, o.k, o.sh)
-                                  : requant1(acc[i][j][4 * g + e], m, sh, a.q_zp));
-            const int px = px0 + 32 * j + 8 * g;
-            // four pixels' bytes of one channel per lane, turned into one
-            // pixel's four channels per lane of a quad
-            const uint32_t lo = __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0400u);
-            const uint32_t hi = __builtin_amdgcn_perm(y[3], y[2], 0x0c0c0400u);
-            const uint32_t v = quad_transpose(__builtin_amdgcn_perm(hi, lo, 0x05040100u), lane);
-            const int p = px + (lane & 3), oc = oc0 + 32 * i - (lane & 3);
-            __builtin_amdgcn_raw_buffer_store_b32(
-                v, yr, p < rows && oc < a.gemm_n ? uint32_t(p) * pitch + uint32_t(oc) : kOutOfRange,
-                0, kPolicy);
-          }
+          store_block32_int8(acc[i][j], r, a.q_zp, yr, rows, px0 + 32 * j, oc0 + 32 * i, a.gemm_n,
+                             lane);
       }
     }
     if (!again) return;
@@ -422,9 +364,9 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
 template <int BM, int BN, int WM, int WN, int GS, bool kLaneTap, int kOcc, int kGroups, int kOut,
           int kPolicy>
 int launch_tile(const ConvArgs &a, hipStream_t stream) {
-  constexpr int KS = 4, R = 2;
-  auto kern = gemm32_kernel<BM, BN, WM, WN, KS, GS, R, kLaneTap, kOut, kPolicy, kOcc>;
-  const size_t lds = size_t(R) * (BM + BN) * 32 * KS + 2 * (kOut == kOutInt32 ? 1 : 3) * BN * 4;
+  constexpr int R = 2;
+  auto kern = gemm32_kernel<BM, BN, WM, WN, GS, R, kLaneTap, kOut, kPolicy, kOcc>;
+  const size_t lds = size_t(R) * (BM + BN) * kStageBytes + 2 * (kOut == kOutInt32 ? 1 : 3) * BN * 4;
   const int tiles = int(((int64_t(a.gemm_m) + BM - 1) / BM) * ((a.gemm_n + BN - 1) / BN));
   static LdsLimit limit;
   if (const int rc = limit.raise(kern, lds); rc != I8CONV_OK) return rc;

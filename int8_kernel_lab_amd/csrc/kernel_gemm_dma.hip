@@ -12,21 +12,36 @@
 //   * a ring of three stage buffers: stage s + 2 is in flight while stage s
 //     feeds the MFMAs, one barrier per stage; the copies of stage s + 2 are
 //     issued between the MFMA groups of stage s, or by copy waves (below);
-//   * the LDS rows use the swz128x layout (see i8conv_device.hpp).  A copy writes lane
-//     i's 16 bytes to LDS slot i of its 1 KB block, so the swizzle is applied
-//     on the source side: the lane of slot (row, physical chunk) fetches the
+//   * v_mfma_i32_32x32x32 with pixels as rows and channels as columns, and its
+//     conflict-free LDS row swizzle (mfma32_tile.hpp).  A copy writes lane i's
+//     16 bytes to LDS slot i of its 1 KB block, so the swizzle is applied on
+//     the source side: the lane of slot (row, physical chunk) fetches the
 //     logical chunk that belongs there;
 //   * because a stage lies inside one tap, the tap decomposition is uniform
 //     per stage: each lane keeps its rows' pixel origin and adds one tap
 //     offset per stage, with two compares for padding;
-//   * eight MFMA waves, two per SIMD, on the 256 x 128, 256 x 64 and
-//     128 x 128 tiles (wave tiles 64 x 64 or 64 x 32), so one wave's MFMAs
-//     run while the other waits on its fragment reads; four on the small
-//     128 x 64 tile;
 //   * on the 256 x 128 and 128 x 128 tiles with four or more k-stages per
-//     workgroup, four more waves that only issue the copies: an MFMA wave
-//     that also issues copies stalls whenever the buffer unit's queue is
-//     full, and its MFMAs wait behind the stalled issue;
+//     workgroup, waves that only issue the copies: an MFMA wave that also
+//     issues copies stalls whenever the buffer unit's queue is full, and its
+//     MFMAs wait behind the stalled issue.  256 x 128: eight MFMA waves of 64
+//     x 64 and eight copy waves, four waves per SIMD (stride-2 128 -> 256
+//     layer, 32 x 56x56: 13.6 us with eight copy waves, 14.9 with four; four
+//     MFMA waves of 128 x 64 are 3 % faster on long reductions with int32
+//     output but 17 % slower with int8, whose requantization then runs on
+//     half the waves).  128 x 128: four MFMA waves of 64 x 64 and four copy
+//     waves (32 x 14x14, 512 -> 512: 20.5 us; eight MFMA waves of 64 x 32,
+//     which read half as much again from LDS, 21.5);
+//   * an MFMA wave reads the fragments of the next k-step between the MFMAs of
+//     the current one, across the stage barrier too.  Against the 16 x 16 x
+//     64 form that read a stage's fragments and then ran its MFMAs (us per
+//     launch over three sets of tensors, same box): 32 x 56x56, 128 -> 256
+//     stride 2: 14.8 -> 12.9, with int8 output 15.2 -> 13.5; 16 x 28x28 1x1
+//     512 -> 384: 13.0 -> 10.4; 64 x 28x28 1x1 384 -> 192: 25.0 -> 19.0; 5 x
+//     86x86, 384 -> 96: 31.8 -> 26.0; 32 x 14x14, 512 -> 512: 20.4 -> 18.7; 8
+//     x 64x64 dilated 256 -> 256: 22.6 -> 21.9 over 60 ms, no difference
+//     over seconds, where the power drawn sets the clock: its MFMAs alone
+//     take 15.4 us with the launch (2.9 POP/s), its stores, which come at the
+//     end of its one round of tiles, 5;
 //   * accumulators stay in VGPRs (built with -amdgpu-mfma-vgpr-form);
 //   * XCD-aware tile order (see below);
 //   * fragments wholly past the last pixel row run no MFMAs.
@@ -36,18 +51,12 @@
 #include <type_traits>
 
 #include "i8conv_internal.hpp"
+#include "mfma32_tile.hpp"
 
 namespace i8conv {
 namespace {
 
 constexpr int kRing = 3;  // stage buffers in LDS
-
-typedef unsigned int v4u_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ v4i add_wrap(v4i a, v4i b) {
-  // int32 addition with two's-complement wrap, like the MFMA accumulator.
-  return __builtin_bit_cast(v4i, __builtin_bit_cast(v4u_t, a) + __builtin_bit_cast(v4u_t, b));
-}
 
 // Calls run(std::integral_constant<int, F>) with F = min(live, FMAX).
 template <int F, int FMAX, class Run>
@@ -74,8 +83,9 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
   constexpr int NW = NCW > 0 ? NCW : NMW;  // copy waves
   constexpr int TMW = BM / WM;  // pixels per wave
   constexpr int TNW = BN / WN;  // output channels per wave
-  constexpr int FM = TMW / 16;
-  constexpr int FN = TNW / 16;
+  constexpr int FM = TMW / 32;  // 32 x 32 blocks
+  constexpr int FN = TNW / 32;
+  constexpr int KS = kStageBytes / 32;  // k-steps per stage
   constexpr int kRows = BM + BN;             // LDS rows per stage: filter, then pixels
   constexpr int kTile = kRows * kStageBytes;  // bytes per stage buffer
   constexpr int kCopies = kRows / 8;          // 1 KB copies per stage
@@ -125,7 +135,7 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
 #pragma unroll
   for (int j = 0; j < CPA; ++j) {
     const int r = 8 * (wave + NW * j) + (lane >> 3);
-    const int lc = swz128x_chunk(r, lane & 7);
+    const int lc = (lane & 7) ^ swz32_f(r);
     const int oc = tile_n + r;
     abase[j] = oc < a.gemm_n ? uint32_t(oc) * uint32_t(a.gemm_k) + uint32_t(lc * 16)
                              : kOutOfRange;
@@ -135,7 +145,7 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
 #pragma unroll
   for (int j = 0; j < CPB; ++j) {
     const int r = 8 * (wave + NW * (CPA + j)) + (lane >> 3);  // >= BN
-    const int lc = swz128x_chunk(r, lane & 7);
+    const int lc = (lane & 7) ^ swz32_f(r);
     const int m = tile_m + r - BN;
     if (m < m_end) {
       const int b = int(fast_div(uint32_t(m), a.div_ohw));
@@ -206,51 +216,75 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
     return;
   }
 
-  // Fragment read offsets inside a stage buffer, per k-step half h.
-  int aoff[2][FN], boff[2][FM];
+  // Fragment read offsets inside a stage buffer, per k-step: row 32 i + lane
+  // % 32 (32 rows are four whole periods of the swizzle), chunk 2 ks + lane
+  // / 32.
+  int koff[KS];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int ch = 4 * h + (lane >> 4);
-#pragma unroll
-    for (int i = 0; i < FN; ++i) aoff[h][i] = swz128x(wn * TNW + i * 16 + (lane & 15), ch);
-#pragma unroll
-    for (int j = 0; j < FM; ++j)
-      boff[h][j] = BN * kStageBytes + swz128x(wm * TMW + j * 16 + (lane & 15), ch);
-  }
+  for (int ks = 0; ks < KS; ++ks)
+    koff[ks] = (lane & 31) * kStageBytes + 16 * ((2 * ks + (lane >> 5)) ^ swz32_f(lane & 31));
+  const int abuf = wn * TNW * kStageBytes, bbuf = (BN + wm * TMW) * kStageBytes;
 
-  v4i acc[FN][FM];
+  v16i acc[FN][FM];
 #pragma unroll
   for (int i = 0; i < FN; ++i)
 #pragma unroll
-    for (int j = 0; j < FM; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+    for (int j = 0; j < FM; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
 
   if (NCW > 0) {
     // MFMA wave of a split workgroup: the copy waves fill the ring.  The
-    // wave's fragments that lie wholly at or past m_end (the padding of a
-    // last pixel tile: 120 of the 128 rows of the deep-K layer's fourth)
-    // get no fragment reads and no MFMAs: the walk runs with the live
-    // fragment count as a compile-time constant.
+    // wave's blocks that lie wholly at or past m_end (the padding of a last
+    // pixel tile: 120 of the 128 rows of the deep-K layer's fourth) get no
+    // fragment reads and no MFMAs: the walk runs with the live block count
+    // as a compile-time constant.
     const int row0 = tile_m + wm * TMW;
-    const int live = m_end <= row0 ? 0 : min(FM, (m_end - row0 + 15) / 16);
+    const int live = m_end <= row0 ? 0 : min(FM, (m_end - row0 + 31) / 32);
     auto walk = [&](auto live_frags) {
       constexpr int F = decltype(live_frags)::value;
+      // The fragments of one k-step in two register sets: the next k-step's
+      // reads go out between the MFMAs of the current one.  The last k-step
+      // of a stage reads the next stage's first, so the barrier that says
+      // that stage has landed (and that every wave has read all of this one)
+      // comes before it.
+      v4i af[2][FN], bf[2][F > 0 ? F : 1];
+      auto read = [&](auto set, const int8_t *buf, int h, int q) {
+        if (q < FN)
+          af[set.value][q] = *reinterpret_cast<const v4i *>(buf + abuf + koff[h] + 32 * kStageBytes * q);
+        else
+          bf[set.value][q - FN] =
+              *reinterpret_cast<const v4i *>(buf + bbuf + koff[h] + 32 * kStageBytes * (q - FN));
+      };
+      constexpr int kReads = F > 0 ? FN + F : 0, kMfma = FN * F;
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kReads; ++q) read(std::integral_constant<int, 0>{}, smem, 0, q);
+      int ring = 0;
       for (int st = s_begin; st < s_end; ++st) {
-        __syncthreads();
-        const int8_t *buf = smem + ((st - s_begin) % kRing) * kTile;
-        v4i af[2][FN], bf[2][F > 0 ? F : 1];
+        const int next = ring + 1 == kRing ? 0 : ring + 1;
+        const int8_t *buf = smem + ring * kTile, *nbuf = smem + next * kTile;
+        auto step = [&](auto set, auto h) {
+          constexpr bool kLast = h.value == KS - 1;
+          if (kLast && st + 1 < s_end) __syncthreads();
+          if constexpr (kMfma > 0) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+            for (int n = 0; n < kMfma; ++n) {
 #pragma unroll
-          for (int i = 0; i < FN; ++i) af[h][i] = *reinterpret_cast<const v4i *>(buf + aoff[h][i]);
-#pragma unroll
-          for (int j = 0; j < F; ++j) bf[h][j] = *reinterpret_cast<const v4i *>(buf + boff[h][j]);
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int i = 0; i < FN; ++i)
-#pragma unroll
-            for (int j = 0; j < F; ++j) acc[i][j] = mfma16(af[h][i], bf[h][j], acc[i][j]);
+              for (int q = n * kReads / kMfma; q < (n + 1) * kReads / kMfma; ++q)
+                read(std::integral_constant<int, 1 - set.value>{}, kLast ? nbuf : buf,
+                     kLast ? 0 : h.value + 1, q);
+              acc[n / F][n % F] = mfma32(bf[set.value][n % F], af[set.value][n / F], acc[n / F][n % F]);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        };
+        static_assert(KS == 4, "four k-steps per stage");
+        step(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 1>{}, std::integral_constant<int, 3>{});
+        ring = next;
       }
     };
     with_live_frags<0, FM>(live, walk);
@@ -269,24 +303,25 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
     const bool more = st + 2 < s_end;
     const StageTap next = stage_tap(more ? st + 2 : st);
     const int8_t *buf = smem + ((st - s_begin) % kRing) * kTile;
-    v4i af[2][FN], bf[2][FM];
+    v4i af[KS][FN], bf[KS][FM];
 #pragma unroll
-    for (int i = 0; i < FN; ++i) af[0][i] = *reinterpret_cast<const v4i *>(buf + aoff[0][i]);
+    for (int h = 0; h < KS; ++h) {
 #pragma unroll
-    for (int j = 0; j < FM; ++j) bf[0][j] = *reinterpret_cast<const v4i *>(buf + boff[0][j]);
+      for (int i = 0; i < FN; ++i)
+        af[h][i] = *reinterpret_cast<const v4i *>(buf + abuf + koff[h] + 32 * kStageBytes * i);
 #pragma unroll
-    for (int i = 0; i < FN; ++i) af[1][i] = *reinterpret_cast<const v4i *>(buf + aoff[1][i]);
-#pragma unroll
-    for (int j = 0; j < FM; ++j) bf[1][j] = *reinterpret_cast<const v4i *>(buf + boff[1][j]);
-    // MFMAs in 2*FN groups of FM, with the copies of stage st + 2 spread
+      for (int j = 0; j < FM; ++j)
+        bf[h][j] = *reinterpret_cast<const v4i *>(buf + bbuf + koff[h] + 32 * kStageBytes * j);
+    }
+    // MFMAs in KS * FN groups of FM, with the copies of stage st + 2 spread
     // between the groups: a copy whose issue stalls (the buffer unit takes a
     // few in flight per wave) then holds back only a few queued MFMAs.
-    constexpr int kGroups = 2 * FN;
+    constexpr int kGroups = KS * FN;
 #pragma unroll
     for (int g = 0; g < kGroups; ++g) {
       const int h = g / FN, i = g % FN;
 #pragma unroll
-      for (int j = 0; j < FM; ++j) acc[i][j] = mfma16(af[h][i], bf[h][j], acc[i][j]);
+      for (int j = 0; j < FM; ++j) acc[i][j] = mfma32(bf[h][j], af[h][i], acc[i][j]);
       if (more) {
 #pragma unroll
         for (int c = (g * CPW + kGroups - 1) / kGroups; c < ((g + 1) * CPW + kGroups - 1) / kGroups; ++c)
@@ -296,125 +331,60 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
     }
   }
 
-  // Epilogue: lane holds channels oc0..oc0+3 of pixel px for each fragment.
-  // The channel fragments of one pixel fragment are stored back to back
-  // (i innermost), so the wave's 16-channel slices of a pixel row, 64 bytes
-  // each, reach the L2 together and fill whole 128-byte lines; written
-  // through (sector-aligned pitches) the layer then writes exactly its
-  // output bytes.
-  int32_t *out = a.y;
-  if (kSplit) out = a.partial + size_t(blockIdx.y) * size_t(a.gemm_m) * size_t(a.gemm_n);
-  const OutWindow ow = out_window(out, a.gemm_m, a.gemm_n, tile_m, a.m_step);
-  const bool vec = (a.gemm_n & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 && ow.ok;
-  v4i bias[FN];
-#pragma unroll
-  for (int i = 0; i < FN; ++i) {
-    const int oc0 = tile_n + wn * TNW + i * 16 + 4 * (lane >> 4);
-    bias[i] = kSplit ? v4i{0, 0, 0, 0} : load_bias4(a.bias, a.gemm_n, oc0);
-  }
-  auto store_tile = [&](auto policy) {
-#pragma unroll
-    for (int j = 0; j < FM; ++j) {
-      const int px = tile_m + wm * TMW + j * 16 + (lane & 15);
-      if (px >= m_end) continue;
-#pragma unroll
-      for (int i = 0; i < FN; ++i) {
-        const int oc0 = tile_n + wn * TNW + i * 16 + 4 * (lane >> 4);
-        const v4i v = add_wrap(acc[i][j], bias[i]);
-        if (vec) {
-          if (oc0 < a.gemm_n)
-            store_out4<decltype(policy)::value>(
-                ow.r, (uint32_t(px - tile_m) * uint32_t(a.gemm_n) + uint32_t(oc0)) * 4u, v);
-        } else {
-          int32_t *dst = out + size_t(px) * size_t(a.gemm_n) + oc0;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (oc0 + e < a.gemm_n) store_out1(dst + e, v[e]);
-        }
-      }
-    }
-  };
-  // Outputs beyond 128 MiB: fragment by fragment, evict-first.  Written
-  // through, such outputs ran up to 1.75x slower (16x256x256x256 1x1: 220
-  // -> 388 us; 268 MB and up all lost), while every output of the baseline
-  // layers (0.8-51 MB) gains from it.
-  auto store_tile_by_fragment = [&]() {
+  // Epilogue (mfma32_tile.hpp): whole 128-byte pieces of output rows per
+  // store.
+  const int rows = m_end - tile_m;
+  const int px0 = wm * TMW, oc0 = tile_n + wn * TNW;
+  if (!kSplit && a.q_y) {
+    const auto yr = make_rsrc(a.q_y + size_t(tile_m) * size_t(a.gemm_n),
+                              uint32_t(rows) * uint32_t(a.gemm_n));
+    const auto br = make_rsrc(a.bias, uint32_t(a.gemm_n) * 4u);
+    const auto mr = make_rsrc(a.q_mult, uint32_t(a.gemm_n) * 4u);
+    const auto sr = make_rsrc(a.q_shift, uint32_t(a.gemm_n) * 4u);
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
-      const int oc0 = tile_n + wn * TNW + i * 16 + 4 * (lane >> 4);
+      const uint32_t off = uint32_t(oc0 + 32 * i + (lane & 31)) * 4u;
+      const uint32_t bias = __builtin_amdgcn_raw_buffer_load_b32(br, off, 0, 0);
+      const Requant32 r =
+          requant32_params(int32_t(__builtin_amdgcn_raw_buffer_load_b32(mr, off, 0, 0)),
+                           int32_t(__builtin_amdgcn_raw_buffer_load_b32(sr, off, 0, 0)), a.q_zp);
 #pragma unroll
       for (int j = 0; j < FM; ++j) {
-        const int px = tile_m + wm * TMW + j * 16 + (lane & 15);
-        if (px >= m_end) continue;
-        const v4i v = add_wrap(acc[i][j], bias[i]);
-        if (vec) {
-          if (oc0 < a.gemm_n)
-            store_out4<kStoreStream>(
-                ow.r, (uint32_t(px - tile_m) * uint32_t(a.gemm_n) + uint32_t(oc0)) * 4u, v);
-        } else {
-          int32_t *dst = out + size_t(px) * size_t(a.gemm_n) + oc0;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (oc0 + e < a.gemm_n) store_out1(dst + e, v[e]);
-        }
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = int(uint32_t(acc[i][j][e]) + bias);
+        store_block32_int8(acc[i][j], r, a.q_zp, yr, rows, px0 + 32 * j, oc0 + 32 * i, a.gemm_n,
+                           lane);
       }
     }
-  };
-  // Requantized int8 output: a lane's four channels of a pixel as one
-  // 4-byte store (a pixel's 16-channel slice, 16 bytes, per four lanes;
-  // ordinary stores, merged into lines in the L2).  Per 16-channel fragment
-  // row, the odd-multiplier form (requant4_odd: four VALU operations per
-  // value) where every channel of the wave's fragment row is in its domain
-  // (a ballot over the active lanes), else the exact form (requant4, three
-  // quarter-rate multiplies per value).  With int8 output, same box: the
-  // 3x3 stride-2 128 -> 256-channel layer (config 3) 16.67-16.74 -> 15.73-
-  // 15.76 us per launch, the dilated 256-channel one (config 5b) 25.64-25.69
-  // -> 24.53-24.64.
-  auto store_tile_requant = [&]() {
+    return;
+  }
+  int32_t *out = a.y;
+  if (kSplit) {
+    out = a.partial + size_t(blockIdx.y) * size_t(a.gemm_m) * size_t(a.gemm_n);
+  } else {
+    const auto br = make_rsrc(a.bias, uint32_t(a.gemm_n) * 4u);
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
-      const int oc0 = tile_n + wn * TNW + i * 16 + 4 * (lane >> 4);
-      if (oc0 >= a.gemm_n) continue;
-      const v4i m = *reinterpret_cast<const v4i *>(a.q_mult + oc0);
-      const v4i sh = *reinterpret_cast<const v4i *>(a.q_shift + oc0);
-      v4i mo, k, h;
-      bool ok = true;
+      const uint32_t bias = __builtin_amdgcn_raw_buffer_load_b32(
+          br, uint32_t(oc0 + 32 * i + (lane & 31)) * 4u, 0, 0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const RequantOdd o = requant_odd_params(m[e], sh[e], a.q_zp);
-        ok = ok && o.ok;
-        mo[e] = o.mo;
-        k[e] = o.k;
-        h[e] = o.sh;
-      }
-      if (__builtin_amdgcn_ballot_w64(!ok) == 0) {
+      for (int j = 0; j < FM; ++j)
 #pragma unroll
-        for (int j = 0; j < FM; ++j) {
-          const int px = tile_m + wm * TMW + j * 16 + (lane & 15);
-          if (px >= m_end) continue;
-          *reinterpret_cast<uint32_t *>(a.q_y + size_t(px) * size_t(a.gemm_n) + oc0) =
-              requant4_odd(add_wrap(acc[i][j], bias[i]), mo, k, h);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < FM; ++j) {
-          const int px = tile_m + wm * TMW + j * 16 + (lane & 15);
-          if (px >= m_end) continue;
-          *reinterpret_cast<uint32_t *>(a.q_y + size_t(px) * size_t(a.gemm_n) + oc0) =
-              requant4(add_wrap(acc[i][j], bias[i]), m, sh, a.q_zp);
-        }
-      }
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = int(uint32_t(acc[i][j][e]) + bias);
     }
-  };
-  // one uniform branch for the whole epilogue
-  if (!kSplit && a.q_y)
-    store_tile_requant();
-  else if (!kSplit && int64_t(a.gemm_m) * a.gemm_n * 4 > kStreamOutputBytes)
-    store_tile_by_fragment();
+  }
+  const auto yr = make_rsrc(out + size_t(tile_m) * size_t(a.gemm_n),
+                            uint32_t(rows) * uint32_t(a.gemm_n) * 4u);
+  // Outputs beyond 128 MiB: evict-first.  Written through, such outputs ran
+  // up to 1.75x slower (16x256x256x256 1x1: 220 -> 388 us; 268 MB and up all
+  // lost), while every output of the baseline layers (0.8-51 MB) gains from
+  // it.
+  if (!kSplit && int64_t(a.gemm_m) * a.gemm_n * 4 > kStreamOutputBytes)
+    store_tile32<kStoreStream>(acc, yr, rows, px0, oc0, a.gemm_n, lane);
   else if (sector_pitch(a.gemm_n))
-    store_tile(std::integral_constant<int, kStoreThrough>{});
+    store_tile32<kStoreThrough>(acc, yr, rows, px0, oc0, a.gemm_n, lane);
   else
-    store_tile(std::integral_constant<int, 0>{});
+    store_tile32<0>(acc, yr, rows, px0, oc0, a.gemm_n, lane);
 }
 
 template <int BM, int BN, int WM, int WN, int NCW = 0>
@@ -454,7 +424,7 @@ int gemm_dma_copy_waves(const GemmPlan &p) {
   // anyway, and the split roles only add a barrier hop per stage.
   // The planner picks 256 x 128 only for more than four k-stages.
   const int per_workgroup = p.splits > 1 ? p.stages_per_split : p.stages;
-  if (p.bm == 256 && p.bn == 128) return 4;
+  if (p.bm == 256 && p.bn == 128) return 8;
   return p.bm == 128 && p.bn == 128 && per_workgroup >= 4 ? 4 : 0;
 }
 
@@ -466,7 +436,7 @@ int launch_gemm_dma(const ConvArgs &args, const GemmPlan &p, int splits, void *s
   // one tap, a stage range per split, a tile it was built for, and LDS rows
   // the ring can hold
   const int stages = a.gemm_k / kStageBytes;
-  if (a.c % kStageBytes != 0 || a.gemm_k % kStageBytes != 0 || stages < 1 ||
+  if (a.c % kStageBytes != 0 || a.gemm_n > (1 << 20) || a.gemm_k % kStageBytes != 0 || stages < 1 ||
       (splits > 1 && (a.stages_per_split < 1 || int64_t(splits - 1) * a.stages_per_split >= stages)) ||
       !gemm_dma_tile_supported(p.bm, p.bn) || a.m_step % 16 != 0 || a.m_step > p.bm ||
       a.m_step < 16 ||
@@ -474,16 +444,14 @@ int launch_gemm_dma(const ConvArgs &args, const GemmPlan &p, int splits, void *s
     set_error("pipelined gemm plan out of range");
     return I8CONV_BAD_ARGUMENT;
   }
-  // eight MFMA waves, two per SIMD (wave tiles 64 x 64, or 64 x 32 on the
-  // narrower tiles), except the small 128 x 64 tile; plus four copy waves on
-  // the wide tiles when the workgroup has k-stages enough
+  // copy waves on the wide tiles when the workgroup has k-stages enough
   const bool spec = gemm_dma_copy_waves(p) > 0;
   switch (p.bm * 1000 + p.bn) {
     case 128064: return launch_tile<128, 64, 2, 2>(a, splits, s);
     case 128128:
-      return spec ? launch_tile<128, 128, 2, 4, 4>(a, splits, s) : launch_tile<128, 128, 2, 4>(a, splits, s);
+      return spec ? launch_tile<128, 128, 2, 2, 4>(a, splits, s) : launch_tile<128, 128, 2, 4>(a, splits, s);
     case 256064: return launch_tile<256, 64, 4, 2>(a, splits, s);
-    case 256128: return launch_tile<256, 128, 4, 2, 4>(a, splits, s);
+    case 256128: return launch_tile<256, 128, 4, 2, 8>(a, splits, s);
   }
   set_error("unsupported pipelined gemm tile");
   return I8CONV_BAD_ARGUMENT;

@@ -1,0 +1,108 @@
+// The 32 x 32 x 32 INT8 MFMA's building blocks, shared by the GEMM kernels:
+// the LDS row swizzle of its fragments and the stores of its accumulators.
+// Pixels are the MFMA's rows (A) and output channels its columns (B): lane
+// (q, h) = (lane % 32, lane / 32) holds channel q of the 32 x 32 block's
+// pixels 8 g + 4 h + e in element 4 g + e.
+#pragma once
+
+#include "i8conv_device.hpp"
+
+namespace i8conv {
+
+#if defined(__HIPCC__)
+
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ v16i mfma32(v4i a, v4i b, v16i c) {
+  return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+}
+
+// LDS rows of 128 bytes: logical 16-byte chunk j of row r sits at chunk j ^
+// swz32_f(r).  A fragment read has lanes 0..31 on 32 consecutive rows of one
+// chunk and lanes 32..63 on the next chunk: f takes each of its eight values
+// once among the rows that share a position modulo 512 bytes, and four
+// consecutive rows differ modulo 128 bytes (the ds_read_b128 rule in
+// i8conv_device.hpp).
+__device__ __forceinline__ int swz32_f(int row) { return ((row >> 2) + 2 * (row & 3)) & 7; }
+
+// Byte transpose over the four lanes of a quad: lane k ends with byte k of
+// lanes 0, 1, 2, 3 of its quad, in that order.
+__device__ __forceinline__ uint32_t quad_transpose(uint32_t v, int lane) {
+  // across lane bit 0: even lanes keep bytes 0, 2 and take the odd lane's;
+  // odd lanes keep bytes 1, 3
+  const uint32_t a =
+      uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0xb1, 0xf, 0xf, false));  // 1 0 3 2
+  v = __builtin_amdgcn_perm(a, v, lane & 1 ? 0x03070105u : 0x06020400u);
+  // across lane bit 1, in halfwords
+  const uint32_t b =
+      uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x4e, 0xf, 0xf, false));  // 2 3 0 1
+  return __builtin_amdgcn_perm(b, v, lane & 2 ? 0x03020706u : 0x05040100u);
+}
+
+// Stores a wave's FN x FM blocks as int32: rows [0, rows) of a window with
+// `n` channels per pixel, px0 the wave's first pixel in it and oc0 its first
+// channel.  Each store writes two whole 128-byte pieces of output rows,
+// whatever n is.  The window is below 2 GiB.
+template <int kPolicy, int FM, int FN>
+__device__ __forceinline__ void store_tile32(const v16i (&acc)[FN][FM], __amdgpu_buffer_rsrc_t out,
+                                             int rows, int px0, int oc0, int n, int lane) {
+  const uint32_t pitch = uint32_t(n) * 4u;
+  const int px = px0 + 4 * (lane >> 5), oc = oc0 + (lane & 31);
+#pragma unroll
+  for (int j = 0; j < FM; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int p = px + 32 * j + 8 * (e >> 2) + (e & 3);
+      const uint32_t off = uint32_t(p) * pitch + uint32_t(oc) * 4u;
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+        __builtin_amdgcn_raw_buffer_store_b32(
+            acc[i][j][e], out, p < rows && oc + 32 * i < n ? off + 128u * i : kOutOfRange, 0,
+            kPolicy);
+    }
+}
+
+// One channel's requantization constants for the blocks of a wave: the
+// odd-multiplier form where all of the wave's lanes allow it, else the exact
+// one.
+struct Requant32 {
+  int32_t mult, shift;
+  RequantOdd o;
+  bool odd;
+};
+__device__ __forceinline__ Requant32 requant32_params(int32_t mult, int32_t shift, int32_t zp) {
+  Requant32 r;
+  r.mult = mult;
+  r.shift = shift;
+  r.o = requant_odd_params(mult, shift, zp);
+  r.odd = __builtin_amdgcn_ballot_w64(!r.o.ok) == 0;
+  return r;
+}
+
+// One 32 x 32 block requantized to int8 (n % 4 == 0, window 4-byte aligned):
+// a lane packs four pixels' bytes of its channel, and the quad's transpose
+// turns them into one pixel's four channels per lane, a 4-byte store; a
+// pixel's 32 channels go out as one 32-byte piece.
+__device__ __forceinline__ void store_block32_int8(const v16i &acc, const Requant32 &r, int32_t zp,
+                                                   __amdgpu_buffer_rsrc_t out, int rows, int px0,
+                                                   int oc0, int n, int lane) {
+  const int oc = oc0 + (lane & 28);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    uint32_t y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      y[e] = uint32_t(r.odd ? requant1_odd(acc[4 * g + e], r.o.mo, r.o.k, r.o.sh)
+                            : requant1(acc[4 * g + e], r.mult, r.shift, zp));
+    const uint32_t lo = __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm(y[3], y[2], 0x0c0c0400u);
+    const uint32_t v = quad_transpose(__builtin_amdgcn_perm(hi, lo, 0x05040100u), lane);
+    const int p = px0 + 4 * (lane >> 5) + 8 * g + (lane & 3);
+    __builtin_amdgcn_raw_buffer_store_b32(
+        v, out, p < rows && oc < n ? uint32_t(p) * uint32_t(n) + uint32_t(oc) : kOutOfRange, 0, 0);
+  }
+}
+
+#endif  // __HIPCC__
+
+}  // namespace i8conv

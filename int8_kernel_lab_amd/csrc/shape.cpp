@@ -75,8 +75,11 @@ bool gemm_tile_supported(int bm, int bn) {
 }
 
 // The LDS-DMA pipelined kernel (kernel_gemm_dma.hip) needs every 128-byte
-// k-stage inside one filter tap: c % 128 == 0.
-static bool dma_eligible(const i8conv_shape &s) { return s.c % kStageBytes == 0; }
+// k-stage inside one filter tap: c % 128 == 0, and a tile's output window
+// below 2 GiB.
+static bool dma_eligible(const i8conv_shape &s) {
+  return s.c % kStageBytes == 0 && s.k <= (1 << 20);
+}
 
 // Generic tile choice.  Pipelined kernel: 128 output channels per tile
 // (64 when N <= 64), and 256 pixels when that still gives the grid about
