@@ -167,7 +167,7 @@ int launch_splitk(const ConvArgs &a, const GemmPlan &p, void *workspace,
 int launch_gemm_dma(const ConvArgs &a, const GemmPlan &p, int splits, void *stream);
 // kernel_gemm32.hip: whether a layer's sizes fit it, and its launch (int8
 // output when a.q_y is set: N % 4 == 0 and a 4-byte aligned q_y)
-bool gemm32_eligible(const i8conv_geometry &g);
+bool gemm32_eligible(const i8conv_shape &s, const i8conv_geometry &g);
 int launch_gemm32(const ConvArgs &a, const GemmPlan &p, void *stream);
 // kernel_pointwise.hip: C and N with an instance (C in {64, 128, 256,
 // 512}, N in {32, 64, 128, 256}), the output-channel slices it splits N

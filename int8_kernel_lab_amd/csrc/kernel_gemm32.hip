@@ -151,21 +151,43 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
   };
   int next_fy = 0, next_fx = 0, next_ci = 0, next_k = 0;
   const int row_step = a.dil_h * a.wd * a.c, col_step = a.dil_w * a.c;
-  auto restart = [&]() { next_fy = next_fx = next_ci = next_k = 0; };
+  // kLaneTap: this lane's chunk moves on by 128 bytes per stage, that is by
+  // `d` taps and channels plus at most one carry of each, in full-rate adds
+  // and selects (dividing by C and S anew each stage took a third of the
+  // issue slots of the small tiles: 16 x 224x224, 32 -> 64 7x7 stride 2)
+  const int d_tap = P / a.c, d_ci = P - d_tap * a.c;
+  const int d_fy = int(fast_div(uint32_t(d_tap), a.div_s)), d_fx = d_tap - d_fy * a.s;
+  const int d_off = d_fy * row_step + d_fx * col_step + d_ci;
+  const int wrap_dx = a.s * a.dil_w, wrap_off = row_step - a.s * col_step;
+  const int tap0 = int(fast_div(uint32_t(lk), a.div_c)), ci0 = lk - tap0 * a.c;
+  const int fy0 = int(fast_div(uint32_t(tap0), a.div_s)), fx0 = tap0 - fy0 * a.s;
+  int lane_ci = 0, lane_dx = 0, lane_dy = 0, lane_off = 0;
+  auto restart = [&]() {
+    next_fy = next_fx = next_ci = next_k = 0;
+    if constexpr (kLaneTap) {
+      lane_ci = ci0;
+      lane_dx = fx0 * a.dil_w;
+      lane_dy = fy0 * a.dil_h;
+      lane_off = fy0 * row_step + fx0 * col_step + ci0;
+    }
+  };
   auto stage_tap = [&]() {
     StageTap t;
     if constexpr (kLaneTap) {
       t.k0 = next_k;
-      const int kk = t.k0 + lk;
-      const int tap = int(fast_div(uint32_t(kk), a.div_c));
-      const int ci = kk - tap * a.c;
-      const int fy = int(fast_div(uint32_t(tap), a.div_s));
-      const int fx = tap - fy * a.s;
-      t.live = kk < a.gemm_k;
-      t.dy = t.live ? fy * a.dil_h : -(1 << 29);
-      t.dx = fx * a.dil_w;
-      t.off = fy * row_step + fx * col_step + ci;
+      t.live = lk < a.gemm_k - next_k;
+      t.dy = t.live ? lane_dy : -(1 << 29);
+      t.dx = lane_dx;
+      t.off = lane_off;
       next_k += P;
+      lane_ci += d_ci;
+      const bool carry = lane_ci >= a.c;
+      lane_ci -= carry ? a.c : 0;
+      lane_dx += d_fx * a.dil_w + (carry ? a.dil_w : 0);
+      const bool wrap = lane_dx >= wrap_dx;
+      lane_dx -= wrap ? wrap_dx : 0;
+      lane_dy += d_fy * a.dil_h + (wrap ? a.dil_h : 0);
+      lane_off += d_off + (carry ? col_step - a.c : 0) + (wrap ? wrap_off : 0);
     } else {
       t.live = true;
       t.k0 = (next_fy * a.s + next_fx) * a.c + next_ci;
@@ -396,9 +418,10 @@ int launch_out(const ConvArgs &a, hipStream_t s) {
 
 }  // namespace
 
-bool gemm32_eligible(const i8conv_geometry &g) {
-  // 32-bit tile and k arithmetic, and a tile's output window below 2 GiB
-  return g.gemm_m <= (1 << 30) && g.gemm_k <= (1 << 30) && g.gemm_n <= (1 << 20) &&
+bool gemm32_eligible(const i8conv_shape &s, const i8conv_geometry &g) {
+  // 32-bit tile, tap and k arithmetic, and a tile's output window below 2 GiB
+  return int64_t(s.r) * s.dilation_h <= (1 << 28) && int64_t(s.s) * s.dilation_w <= (1 << 28) &&
+         g.gemm_m <= (1 << 30) && g.gemm_k <= (1 << 30) && g.gemm_n <= (1 << 20) &&
          ((g.gemm_m + 63) / 64) * ((int64_t(g.gemm_n) + 63) / 64) <= INT32_MAX;
 }
 
@@ -413,7 +436,9 @@ int launch_gemm32(const ConvArgs &args, const GemmPlan &p, void *stream) {
   switch (p.bm * 1000 + p.bn) {
     case 64064: return launch_out<64, 64, 2, 2, 2, true, 4, 4>(a, s);
     case 128064: return launch_out<128, 64, 2, 2, 1, true, 3, 3>(a, s);
-    case 128128: return launch_out<128, 128, 4, 2, 2, true, 4, 2>(a, s);
+    // four waves of 64 x 64: eight of 32 x 64 spill at four waves per SIMD (7 x
+    // 196x196, 80 -> 209 1x3: 72 us, 48 with four; 256x256, 64 -> 255: 23.6, 21)
+    case 128128: return launch_out<128, 128, 2, 2, 1, true, 2, 2>(a, s);
     case 256256:
       // a stage lies inside one tap
       if (a.c % kStageBytes == 0) return launch_out<256, 256, 4, 2, 1, false, 2, 1>(a, s);

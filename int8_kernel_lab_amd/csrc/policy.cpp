@@ -20,7 +20,7 @@
 //      Likewise the 32 x 32 x 32 MFMA GEMM (C % 128 != 0) wherever it has a
 //      plan: it beat the halo and strip kernels on every such layer (1x3, 64
 //      -> 128: 14.2 against 22.3 us; 256x256, 64 -> 63, 69, 255: 9.3, 11.1,
-//      23 against 16.4, 19.2, 43; dilated 64 -> 128: 5.3 against 6.3);
+//      21 against 16.4, 19.2, 43; dilated 64 -> 128: 5.3 against 6.3);
 //   4. otherwise an input-reuse kernel for a stride-1 spatial filter
 //      (r*s > 1): halo when eligible, else strip (small dilated layers,
 //      asymmetric 1x3/3x1, C = 64 layers wider than the row kernel's four

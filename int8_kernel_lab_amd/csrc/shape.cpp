@@ -190,8 +190,8 @@ int64_t staged_tiles(const i8conv_shape &s, const i8conv_geometry &g) {
 // C % 128 != 0: the 32 x 32 x 32 MFMA kernel instead of the register-staged
 // one, on the largest tile that keeps the compute units covered:
 //   * 128 x 128, two workgroups per unit, for N > 64 with at least 256 tiles
-//     (256x256, 64 -> 255 3x3: 43 -> 23; 7 x 196x196, 80 -> 209 1x3: 202 ->
-//     59; 16 x 224x224, 32 -> 96 4x4 stride 4: 15.8 -> 8.6, 64 x 64: 10.0);
+//     (256x256, 64 -> 255 3x3: 43 -> 21; 7 x 196x196, 80 -> 209 1x3: 202 ->
+//     48; 16 x 224x224, 32 -> 96 4x4 stride 4: 15.8 -> 8.6, 64 x 64: 10.0);
 //   * 128 x 64, three per unit, with at least 512 tiles (16 x 224x224, 32 ->
 //     64 7x7 stride 2: 101 -> 35; 256x256, 64 -> 63: 16.4 -> 9.3);
 //   * 64 x 64, four per unit, below that (416x416, 32 -> 64 3x3 stride 2: 7.3
@@ -213,7 +213,7 @@ GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
     p.pw_waves = pointwise_waves(g.gemm_m, pointwise_slices(s.c, int(g.gemm_n)));
     if (p.dma) return p;  // the fallback for unaligned pointers stays pipelined
   }
-  if (!gemm32_eligible(g)) return p;
+  if (!gemm32_eligible(s, g)) return p;
   auto tiles = [&](int bm, int bn) { return ceil_div(g.gemm_m, bm) * ceil_div(g.gemm_n, bn); };
   int bm = 0, bn = 0;
   if (p.dma) {
