@@ -448,6 +448,7 @@ int i8conv_describe(int id, const i8conv_shape *shape, char *buf, size_t len) {
         ", grid " + tiles(g.gemm_m, p.m_step > 0 ? p.m_step : p.bm) + "x" +
         tiles(g.gemm_n, p.bn) + (p.splits > 1 ? "x" + std::to_string(p.splits) + " splits" : "") +
         ", " + std::to_string(p.stages) + " k-stages" +
+        (p.kg > 1 ? ", " + std::to_string(p.kg) + " wave groups" : "") +
         (p.dma && !p.m32 && gemm_dma_copy_waves(p) > 0 ? ", " + std::to_string(gemm_dma_copy_waves(p)) + " copy waves" : "");
   } else {
     PatchPlan p;

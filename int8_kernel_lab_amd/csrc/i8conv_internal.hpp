@@ -94,8 +94,9 @@ struct GemmPlan {
   // the register-staged one (kernel_gemm.hip)
   bool dma = false;
   // generic only: the 32 x 32 x 32 MFMA kernel (kernel_gemm32.hip) runs the
-  // layer, on bm x bn tiles
+  // layer, on bm x bn tiles; kg groups of waves share a tile's reduction
   bool m32 = false;
+  int kg = 1;
   // split-K only: the deep-channel kernel instead of the GEMM
   bool deep = false;
   DeepPlan deep_plan;

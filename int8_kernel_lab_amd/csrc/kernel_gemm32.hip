@@ -73,11 +73,14 @@ __device__ __forceinline__ void barrier_lds() {
   asm volatile("" ::: "memory");
 }
 
-// BM pixels x BN channels over WM x WN waves; fragments read GS k-steps of 32
-// bytes at a time; R stage buffers; kOcc waves per SIMD.
-template <int BM, int BN, int WM, int WN, int GS, int R, bool kLaneTap, int kOut, int kPolicy,
-          int kOcc>
-__global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, int tiles) {
+// BM pixels x BN channels over WM x WN waves; KG groups of such waves, each
+// with stage buffers of its own, take the k-stages in turn (group g the
+// stages g, g + KG, ...) and add their sums up through LDS at the end;
+// fragments read GS k-steps of 32 bytes at a time; R stage buffers per group;
+// kOcc waves per SIMD.
+template <int BM, int BN, int WM, int WN, int KG, int GS, int R, bool kLaneTap, int kOut,
+          int kPolicy, int kOcc>
+__global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArgs a, int tiles) {
   constexpr int P = kStageBytes;             // bytes per LDS row: one k-stage
   constexpr int KS = P / 32;                 // k-steps per stage
   constexpr int kWaves = WM * WN;
@@ -93,17 +96,21 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
   constexpr int kParamBytes = kParams * BN * 4;
   constexpr int ST = FM * FN * (kByte ? 4 : 16);  // stores per wave and tile
   static_assert(CPA >= 1 && CPB >= 1 && BN % (RPC * kWaves) == 0, "tile shape");
+  static_assert(KG == 1 || (kLaneTap && FM == 1 && FN == 1 && 4 % KG == 0), "k groups");
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = wave_id / kWaves, wave = wave_id % kWaves;
   const int wm = wave % WM, wn = wave / WM;
   const v4u xd = make_desc(a.x, a.x_bytes);
   const v4u wd = make_desc(a.w, a.w_bytes);
-  const uint32_t lds0 = lds_addr(smem);
-  const uint32_t lds_params = lds0 + R * kTile;
-  int8_t *const params = smem + R * kTile;
-  const int stages = (a.gemm_k + P - 1) / P;
+  int8_t *const bufs = smem + group * R * kTile;  // this group's stage buffers
+  const uint32_t lds0 = lds_addr(bufs);
+  int8_t *const params = smem + KG * R * kTile;
+  const uint32_t lds_params = lds_addr(params);
+  // stages per group (the last ones may lie past the reduction: zeros)
+  const int stages = (a.gemm_k + KG * P - 1) / (KG * P);
   const int tiles_n = (a.gemm_n + BN - 1) / BN;
 
   // this lane's chunk of every row it copies, and its row within a copy
@@ -151,19 +158,21 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
   };
   int next_fy = 0, next_fx = 0, next_ci = 0, next_k = 0;
   const int row_step = a.dil_h * a.wd * a.c, col_step = a.dil_w * a.c;
-  // kLaneTap: this lane's chunk moves on by 128 bytes per stage, that is by
+  // kLaneTap: this lane's chunk moves on by 128 KG bytes per stage, that is by
   // `d` taps and channels plus at most one carry of each, in full-rate adds
   // and selects (dividing by C and S anew each stage took a third of the
   // issue slots of the small tiles: 16 x 224x224, 32 -> 64 7x7 stride 2)
-  const int d_tap = P / a.c, d_ci = P - d_tap * a.c;
+  const int d_tap = int(fast_div(uint32_t(KG * P), a.div_c)), d_ci = KG * P - d_tap * a.c;
   const int d_fy = int(fast_div(uint32_t(d_tap), a.div_s)), d_fx = d_tap - d_fy * a.s;
   const int d_off = d_fy * row_step + d_fx * col_step + d_ci;
   const int wrap_dx = a.s * a.dil_w, wrap_off = row_step - a.s * col_step;
-  const int tap0 = int(fast_div(uint32_t(lk), a.div_c)), ci0 = lk - tap0 * a.c;
+  const int k0 = group * P + lk;
+  const int tap0 = int(fast_div(uint32_t(k0), a.div_c)), ci0 = k0 - tap0 * a.c;
   const int fy0 = int(fast_div(uint32_t(tap0), a.div_s)), fx0 = tap0 - fy0 * a.s;
   int lane_ci = 0, lane_dx = 0, lane_dy = 0, lane_off = 0;
   auto restart = [&]() {
-    next_fy = next_fx = next_ci = next_k = 0;
+    next_fy = next_fx = next_ci = 0;
+    next_k = group * P;
     if constexpr (kLaneTap) {
       lane_ci = ci0;
       lane_dx = fx0 * a.dil_w;
@@ -179,7 +188,7 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
       t.dy = t.live ? lane_dy : -(1 << 29);
       t.dx = lane_dx;
       t.off = lane_off;
-      next_k += P;
+      next_k += KG * P;
       lane_ci += d_ci;
       const bool carry = lane_ci >= a.c;
       lane_ci -= carry ? a.c : 0;
@@ -217,10 +226,10 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
   };
   // per-channel parameters of the tile at tile_n into parameter slot `slot`
   auto copy_params = [&](int slot) {
-    if (wave * 64 < BN) {
+    if (wave_id * 64 < BN) {
       const uint32_t bytes = uint32_t(a.gemm_n) * 4u;
-      const uint32_t off = uint32_t(tile_n + wave * 64 + lane) * 4u;
-      const uint32_t dst = lds_params + uint32_t(slot * kParamBytes) + uint32_t(wave) * 256u;
+      const uint32_t off = uint32_t(tile_n + wave_id * 64 + lane) * 4u;
+      const uint32_t dst = lds_params + uint32_t(slot * kParamBytes) + uint32_t(wave_id) * 256u;
       lds_copy4(make_desc(a.bias, bytes), dst, off);
       if constexpr (kByte) {
         lds_copy4(make_desc(a.q_mult, bytes), dst + BN * 4u, off);
@@ -274,7 +283,8 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
     const int8_t *const pr = params + slot * kParamBytes;
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
-      const int v = *reinterpret_cast<const int *>(pr + (wn * TN + 32 * i + (lane & 31)) * 4);
+      const int v = group > 0 ? 0 : *reinterpret_cast<const int *>(
+          pr + (wn * TN + 32 * i + (lane & 31)) * 4);
       v16i c;
 #pragma unroll
       for (int e = 0; e < 16; ++e) c[e] = v;
@@ -296,13 +306,13 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
     constexpr int kMfma = GS * FN * FM;
     constexpr int kReads = GS * (FN + FM);
 #pragma unroll
-    for (int q = 0; q < kReads; ++q) read(Set<0>{}, smem, 0, q);
+    for (int q = 0; q < kReads; ++q) read(Set<0>{}, bufs, 0, q);
 
     int ring = 0;
     auto stage = [&](auto first, int s) {
       const int next = ring + 1 == R ? 0 : ring + 1;
-      const int8_t *const buf = smem + ring * kTile;
-      const int8_t *const nbuf = smem + next * kTile;
+      const int8_t *const buf = bufs + ring * kTile;
+      const int8_t *const nbuf = bufs + next * kTile;
       const bool more = s + R < stages;
       StageTap tap{};
       if (more) tap = stage_tap();
@@ -349,10 +359,64 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
       }
     }
 
-    // the next tile's copies go out before this tile's stores
     const int out_m = tile_m, out_n = tile_n, out_end = m_end;
     t += step;
     const bool again = t < last;
+    if constexpr (KG > 1) {
+      // each wave's sums go to its 4 KB of the first stage buffers (every
+      // wave has read its last stage), four elements per 1 KB; then group g
+      // adds up and stores the elements of quads g, g + KG, ...
+      const int rows = out_end - out_m;
+      const int px0 = wm * TM + 4 * (lane >> 5), oc0 = out_n + wn * TN;
+      auto part_of = [&](int grp, int q) {
+        return reinterpret_cast<v4i *>(smem + grp * R * kTile + wave * 4096 + q * 1024 + lane * 16);
+      };
+      static_assert(kWaves * 4096 <= R * kTile, "sums fit the stage buffers");
+      barrier_lds();
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *part_of(group, q) = v4i{acc[0][0][4 * q], acc[0][0][4 * q + 1], acc[0][0][4 * q + 2],
+                                 acc[0][0][4 * q + 3]};
+      barrier_lds();
+      const int8_t *const pq = pr + (wn * TN + (lane & 31)) * 4;
+      Requant32 r{};
+      if constexpr (kByte)
+        r = requant32_params(*reinterpret_cast<const int *>(pq + BN * 4),
+                             *reinterpret_cast<const int *>(pq + BN * 8), a.q_zp);
+#pragma unroll
+      for (int u = 0; u < 4 / KG; ++u) {
+        const int q = group + KG * u;
+        v4u sum = *reinterpret_cast<const v4u *>(part_of(0, q));
+#pragma unroll
+        for (int g = 1; g < KG; ++g) sum += *reinterpret_cast<const v4u *>(part_of(g, q));
+        const v4i v = __builtin_bit_cast(v4i, sum);
+        if constexpr (kByte) {
+          const auto yr = make_rsrc(a.q_y + size_t(out_m) * size_t(a.gemm_n),
+                                    uint32_t(rows) * uint32_t(a.gemm_n));
+          store_quad_int8(v, r, a.q_zp, yr, rows, px0 + 8 * q, oc0, a.gemm_n, lane);
+        } else {
+          const auto yr = make_rsrc(a.y + size_t(out_m) * size_t(a.gemm_n),
+                                    uint32_t(rows) * uint32_t(a.gemm_n) * 4u);
+          const int oc = oc0 + (lane & 31);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int px = px0 + 8 * q + e;
+            __builtin_amdgcn_raw_buffer_store_b32(
+                v[e], yr,
+                px < rows && oc < a.gemm_n
+                    ? (uint32_t(px) * uint32_t(a.gemm_n) + uint32_t(oc)) * 4u : kOutOfRange,
+                0, kPolicy);
+          }
+        }
+      }
+      if (!again) return;
+      barrier_lds();
+      setup(t);
+      slot ^= 1;
+      prologue(slot);
+      continue;
+    }
+    // the next tile's copies go out before this tile's stores
     if (again) {
       setup(t);
       prologue(slot ^ 1);
@@ -383,17 +447,18 @@ __global__ __launch_bounds__(64 * WM * WN, kOcc) void gemm32_kernel(ConvArgs a, 
   }
 }
 
-template <int BM, int BN, int WM, int WN, int GS, bool kLaneTap, int kOcc, int kGroups, int kOut,
-          int kPolicy>
+template <int BM, int BN, int WM, int WN, int KG, int GS, bool kLaneTap, int kOcc, int kGroups,
+          int kOut, int kPolicy>
 int launch_tile(const ConvArgs &a, hipStream_t stream) {
   constexpr int R = 2;
-  auto kern = gemm32_kernel<BM, BN, WM, WN, GS, R, kLaneTap, kOut, kPolicy, kOcc>;
-  const size_t lds = size_t(R) * (BM + BN) * kStageBytes + 2 * (kOut == kOutInt32 ? 1 : 3) * BN * 4;
+  auto kern = gemm32_kernel<BM, BN, WM, WN, KG, GS, R, kLaneTap, kOut, kPolicy, kOcc>;
+  const size_t lds =
+      size_t(KG) * R * (BM + BN) * kStageBytes + 2 * (kOut == kOutInt32 ? 1 : 3) * BN * 4;
   const int tiles = int(((int64_t(a.gemm_m) + BM - 1) / BM) * ((a.gemm_n + BN - 1) / BN));
   static LdsLimit limit;
   if (const int rc = limit.raise(kern, lds); rc != I8CONV_OK) return rc;
-  I8_LAUNCH(kern, dim3(unsigned(std::min(tiles, 256 * kGroups))), dim3(64 * WM * WN), lds, stream, a,
-            tiles);
+  I8_LAUNCH(kern, dim3(unsigned(std::min(tiles, 256 * kGroups))), dim3(64 * WM * WN * KG),
+            lds, stream, a, tiles);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error(std::string("gemm32 kernel launch: ") + hipGetErrorString(e));
@@ -405,15 +470,15 @@ int launch_tile(const ConvArgs &a, hipStream_t stream) {
 // The cache policies of kernel_gemm_dma.hip: int32 write-through where the
 // pixel pitch keeps sectors whole and the output is at most 128 MiB,
 // evict-first above, ordinary for other pitches and for int8.
-template <int BM, int BN, int WM, int WN, int GS, bool kLaneTap, int kOcc, int kGroups>
+template <int BM, int BN, int WM, int WN, int KG, int GS, bool kLaneTap, int kOcc, int kGroups>
 int launch_out(const ConvArgs &a, hipStream_t s) {
   if (a.q_y)
-    return launch_tile<BM, BN, WM, WN, GS, kLaneTap, kOcc, kGroups, kOutInt8, 0>(a, s);
+    return launch_tile<BM, BN, WM, WN, KG, GS, kLaneTap, kOcc, kGroups, kOutInt8, 0>(a, s);
   if (a.gemm_n % 8 != 0)
-    return launch_tile<BM, BN, WM, WN, GS, kLaneTap, kOcc, kGroups, kOutInt32, 0>(a, s);
+    return launch_tile<BM, BN, WM, WN, KG, GS, kLaneTap, kOcc, kGroups, kOutInt32, 0>(a, s);
   if (int64_t(a.gemm_m) * a.gemm_n * 4 > kStreamOutputBytes)
-    return launch_tile<BM, BN, WM, WN, GS, kLaneTap, kOcc, kGroups, kOutInt32, kStoreStream>(a, s);
-  return launch_tile<BM, BN, WM, WN, GS, kLaneTap, kOcc, kGroups, kOutInt32, kStoreThrough>(a, s);
+    return launch_tile<BM, BN, WM, WN, KG, GS, kLaneTap, kOcc, kGroups, kOutInt32, kStoreStream>(a, s);
+  return launch_tile<BM, BN, WM, WN, KG, GS, kLaneTap, kOcc, kGroups, kOutInt32, kStoreThrough>(a, s);
 }
 
 }  // namespace
@@ -434,14 +499,17 @@ int launch_gemm32(const ConvArgs &args, const GemmPlan &p, void *stream) {
     return I8CONV_BAD_ARGUMENT;
   }
   switch (p.bm * 1000 + p.bn) {
-    case 64064: return launch_out<64, 64, 2, 2, 2, true, 4, 4>(a, s);
-    case 128064: return launch_out<128, 64, 2, 2, 1, true, 3, 3>(a, s);
+    case 64064:
+      if (p.kg == 4) return launch_out<64, 64, 2, 2, 4, 2, true, 4, 1>(a, s);
+      if (p.kg == 2) return launch_out<64, 64, 2, 2, 2, 2, true, 4, 2>(a, s);
+      return launch_out<64, 64, 2, 2, 1, 2, true, 4, 4>(a, s);
+    case 128064: return launch_out<128, 64, 2, 2, 1, 1, true, 3, 3>(a, s);
     // four waves of 64 x 64: eight of 32 x 64 spill at four waves per SIMD (7 x
     // 196x196, 80 -> 209 1x3: 72 us, 48 with four; 256x256, 64 -> 255: 23.6, 21)
-    case 128128: return launch_out<128, 128, 2, 2, 1, true, 2, 2>(a, s);
+    case 128128: return launch_out<128, 128, 2, 2, 1, 1, true, 2, 2>(a, s);
     case 256256:
       // a stage lies inside one tap
-      if (a.c % kStageBytes == 0) return launch_out<256, 256, 4, 2, 1, false, 2, 1>(a, s);
+      if (a.c % kStageBytes == 0) return launch_out<256, 256, 4, 2, 1, 1, false, 2, 1>(a, s);
       break;
   }
   set_error("gemm32: unsupported tile " + std::to_string(p.bm) + "x" + std::to_string(p.bn));

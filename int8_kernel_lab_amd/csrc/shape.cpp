@@ -195,14 +195,19 @@ int64_t staged_tiles(const i8conv_shape &s, const i8conv_geometry &g) {
 //   * 128 x 64, three per unit, with at least 512 tiles (16 x 224x224, 32 ->
 //     64 7x7 stride 2: 101 -> 35; 256x256, 64 -> 63: 16.4 -> 9.3);
 //   * 64 x 64, four per unit, below that (416x416, 32 -> 64 3x3 stride 2: 7.3
-//     -> 5.9, 128 x 64: 7.6; 4 x 28x28, 192 -> 192 3x3: 19.9 -> 12.6);
-//   * the register-staged kernel keeps layers of at most 64 channels and one
-//     round of 64-pixel tiles: each of its stages costs less where a unit
-//     has one tile (7 x 38x38, 288 -> 32 3x3: 12.5 against 17.8; 224x224, 32
-//     -> 64 7x7 stride 2: 10.8 against 12.5).
+//     -> 5.9, 128 x 64: 7.6).  With at most two tiles per unit a stage's
+//     latency counts, not its throughput: then groups of waves share a tile's
+//     stages, two of them from six stages on (4 x 28x28, 192 -> 192 3x3, 14
+//     stages: 19.9 -> 13.1 -> 10.6; 7 x 38x38, 288 -> 32, 21 stages: 17.8 ->
+//     14.2), four from 24 stages on and at most one tile per unit (193x34,
+//     432 -> 96, 31 stages: one group 26.1, two 18.6, four 17.3; at 14 stages
+//     four are slower than two, 11.4);
+//   * the register-staged kernel keeps layers of at most 64 channels, fewer
+//     than six stages and one round of 64-pixel tiles (2 x 30x30, 48 -> 64
+//     3x3: 5.5 against 6.0).
 // C % 128 == 0: the pipelined kernel, except
 //   * grids of fewer than 128 of its tiles, which leave half the units idle:
-//     64 x 64 (52x52, 256 -> 512 3x3 stride 2: 12.7 -> 9.3);
+//     64 x 64 (52x52, 256 -> 512 3x3 stride 2: 12.7 -> 7.9 with two groups);
 //   * at least two rounds of 256 x 256 tiles: a third fewer copied bytes per
 //     operation (16 x 256x256, 256 -> 256 3x3: 780 -> 706; 5x5 stride 2 with
 //     int8 output: 484 -> 457).
@@ -225,9 +230,11 @@ GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
     bm = bn = 128;
   } else if (tiles(128, 64) >= 512) {
     bm = 128, bn = 64;
-  } else if (g.gemm_n > 64 || tiles(64, 64) > 256) {
+  } else if (g.gemm_n > 64 || p.stages >= 6 || tiles(64, 64) > 256) {
     bm = bn = 64;
   }
+  if (bm == 64 && tiles(64, 64) <= 512 && p.stages >= 6)
+    p.kg = p.stages >= 24 && tiles(64, 64) <= 256 ? 4 : 2;
   if (bm > 0) {
     p.m32 = true;
     p.bm = bm;

@@ -18,6 +18,19 @@ CASES = {
     "64_m65_n65_c80": ("64px x 64oc", lab.ConvShape(1, 5, 13, 80, 65, 3, 3, 1, 1, 1, 1, 1, 1)),
     "64_c16_5x3": ("64px x 64oc", lab.ConvShape(3, 19, 23, 16, 68, 5, 3, 2, 0, 2, 1, 1, 2)),
     "64_c384_s2": ("64px x 64oc", lab.ConvShape(2, 23, 21, 384, 132, 3, 3, 1, 1, 2, 2, 1, 1)),
+    # groups of waves on a tile's stages: two (7 and 15 stages: the second
+    # group's last one past the reduction), four (25 and 26 stages), with a
+    # second tile for some workgroups
+    "64_g2_c96": ("64px x 64oc, grid 4x2, 7 k-stages, 2 wave groups",
+                  lab.ConvShape(1, 15, 14, 96, 72, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "64_g2_c208_k33": ("64px x 64oc, grid 38x1, 15 k-stages, 2 wave groups",
+                       lab.ConvShape(3, 27, 30, 208, 33, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "64_g2_450_tiles": ("64px x 64oc, grid 225x2, 6 k-stages, 2 wave groups",
+                        lab.ConvShape(10, 40, 36, 80, 100, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "64_g4_c352": ("64px x 64oc, grid 4x2, 25 k-stages, 4 wave groups",
+                   lab.ConvShape(2, 11, 10, 352, 68, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "64_g4_c656_5x1": ("64px x 64oc, grid 6x3, 26 k-stages, 4 wave groups",
+                       lab.ConvShape(5, 9, 8, 656, 132, 5, 1, 2, 0, 1, 1, 1, 1)),
     "64_k128": ("64px x 64oc", lab.ConvShape(18, 31, 33, 32, 36, 2, 2, 0, 0, 1, 1, 1, 1)),
     # 128 x 64: C = 32 and 48, odd channel counts, padding wider than the image
     "128x64_c32_k63": ("128px x 64oc", lab.ConvShape(5, 121, 119, 32, 63, 3, 3, 1, 1, 1, 1, 1, 1)),
