@@ -9,10 +9,16 @@
 // Tiled transposes (16-byte rows on both sides: rows * esize and cols *
 // esize multiples of 16, 16-byte aligned bases): one workgroup per 128 x
 // 128-byte tile (bytes: two tiles side by side where the source rows hold
-// 256 bytes or more), read as whole 128-byte source row pieces (8 lanes x 16
-// bytes), staged in LDS and written as whole 128-byte rows of the transposed
-// matrix.  With one side short instead (any length), the short-row and
-// short-column forms below run; otherwise an element-per-thread form.
+// 256 bytes or more) or 64 x 64-dword tile, read as whole source row pieces
+// (16 bytes a lane), staged in LDS and written as whole pieces of the
+// transposed matrix's rows.  With one side of at most 512 elements (any
+// number) and the other's rows whole 16-byte pieces, the short-row and
+// short-column forms below run (32 x 21x20 x 256 bytes: 3.9 us, tiled 4.4; 16
+// x 45x37 x 128: 6.1, tiled 4.3).  Everything else runs the tiled form with
+// pieces at any byte: an element per thread, its writes scattered, took 62 us
+// for 16 x 45x45 x 256 dwords (12 tiled, 5.5 TB/s), 298 for 32 x 448 x 63x63
+// bytes (30 tiled).  Tensors with a side below 16 elements keep the
+// element-per-thread form.
 //
 // Bytes: each lane takes 16 rows x 4 columns of the tile, reads them as 16
 // dwords (4 columns of a row each), turns every 4 x 4 byte block around with
@@ -32,6 +38,7 @@
 
 #include <algorithm>
 #include <string>
+#include <type_traits>
 
 #include "i8conv_internal.hpp"
 
@@ -39,7 +46,13 @@ namespace i8conv {
 namespace {
 
 constexpr int kTileRowBytes = 128;
-constexpr int kLdsPitch = 132;
+constexpr int kDwordTile = 64;  // dwords per side of a dword tile
+constexpr int kShortSide = 16;   // shorter sides than this: an element per thread
+constexpr int kShortMost = 512;  // longest short side of the short-row and short-column forms
+// Dword transposes of at least so many bytes store evict-first (32 x 56x56 x
+// 128: 15.8 us, written through 19.3; 256 channels: 36.3, 37.8), smaller ones
+// through (32 x 14x14 x 512: 5.6 us, evict-first 6.5).
+constexpr int64_t kStreamTransposeBytes = 32 << 20;
 
 __device__ __forceinline__ int byte_tile_row(int i) { return 32 * i + 8 * (i >> 4); }
 
@@ -57,9 +70,30 @@ __device__ __forceinline__ void transpose4x4(const uint32_t (&a)[4], uint32_t (&
   o[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
 }
 
-template <int kSub>
+// 16 bytes at src + off of a tensor of `bytes` bytes, off any value: a piece
+// that runs past its row's end takes the next row's bytes (never stored), and
+// only what lies past the tensor reads as zero.
+__device__ __forceinline__ v4i load16_any(const int8_t *src, int64_t off, int64_t bytes) {
+  v4i v{0, 0, 0, 0};
+  if (off + 16 <= bytes) {
+    __builtin_memcpy(&v, src + off, 16);  // unaligned global loads are legal on gfx950
+  } else if (off < bytes) {
+    uint8_t b[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) b[e] = off + e < bytes ? uint8_t(src[off + e]) : uint8_t(0);
+    __builtin_memcpy(&v, b, 16);
+  }
+  return v;
+}
+
+// kAny: rows, columns and bases of any length and alignment.  Pieces then
+// start at any byte; a column's last 16 rows are stored by a lane that starts
+// early enough to end with them (some bytes are written twice, with the same
+// values), and only a last tile of fewer than 16 rows stores single bytes.
+template <int kSub, bool kAny>
 __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *src, int8_t *dst,
-                                                                  int rows, int cols, int tiles_r,
+                                                                  int64_t batch, int rows,
+                                                                  int cols, int tiles_r,
                                                                   int tiles_c) {
   constexpr int T = kTileRowBytes;
   constexpr int kTileDw = 32 * T + 8 * (T / 16);  // one 128 x 128 tile
@@ -75,20 +109,42 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
   const int r0 = tr * T, c0 = tc * T * kSub;
   // read: tile row i = source row r0 + i, bytes [c0, c0 + 128 kSub); piece
   // pc of the row goes to tile pc / 8
-  for (int idx = threadIdx.x; idx < T * 8 * kSub; idx += kThreads) {
+  auto place = [&](int idx, v4i v) {
     const int i = idx / (8 * kSub), pc = idx % (8 * kSub);
-    const uint32_t cb = uint32_t(c0 + pc * 16);
-    const bool ok = r0 + i < rows && cb < uint32_t(cols);
-    *reinterpret_cast<v4i *>(&tile[(pc >> 3) * kTileDw + byte_tile_row(i) + 4 * (pc & 7)]) =
-        load16(sr, ok ? uint32_t(r0 + i) * uint32_t(cols) + cb : kOutOfRange);
+    *reinterpret_cast<v4i *>(&tile[(pc >> 3) * kTileDw + byte_tile_row(i) + 4 * (pc & 7)]) = v;
+  };
+  if constexpr (kAny) {
+    // every load before the first LDS write: left to itself the compiler waits
+    // for each (16 x 256 x 45x45: 5.5 against 6.7 us)
+    v4i in[4 * kSub];
+#pragma unroll
+    for (int u = 0; u < 4 * kSub; ++u) {
+      const int idx = int(threadIdx.x) + u * kThreads;
+      const int row = r0 + idx / (8 * kSub), col = c0 + idx % (8 * kSub) * 16;
+      in[u] = row < rows && col < cols
+                  ? load16_any(src, int64_t(mat) * int64_t(mat_bytes) + int64_t(row) * cols + col,
+                               batch * int64_t(mat_bytes))
+                  : v4i{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int u = 0; u < 4 * kSub; ++u) place(int(threadIdx.x) + u * kThreads, in[u]);
+  } else {
+    for (int idx = threadIdx.x; idx < T * 8 * kSub; idx += kThreads) {
+      const uint32_t row = uint32_t(r0 + idx / (8 * kSub)), cb = uint32_t(c0 + idx % (8 * kSub) * 16);
+      place(idx, load16(sr, row < uint32_t(rows) && cb < uint32_t(cols) ? row * uint32_t(cols) + cb
+                                                                       : kOutOfRange));
+    }
   }
   __syncthreads();
   // write: lane (column group cg, row group rg) -> columns 4 cg .. + 3 of
   // each tile, rows r0 + 16 rg .. + 15; the 8 row groups of a column are 8
   // consecutive lanes, so each output row gets 128 contiguous bytes
   const int cg = threadIdx.x >> 3, rg = threadIdx.x & 7;
-  const int i0 = 16 * rg;
-  if (r0 + i0 >= rows) return;  // rows % 16 == 0: a row group is whole or absent
+  int i0 = 16 * rg;
+  if (r0 + i0 >= rows) return;  // !kAny: rows % 16 == 0, a row group is whole or absent
+  const int live = min(T, rows - r0);
+  if (kAny && i0 + 16 > live) i0 = max(0, live - 16);
+  const int n = kAny ? min(16, live - i0) : 16;  // < 16 only in a tile of fewer rows
 #pragma unroll
   for (int sub = 0; sub < kSub; ++sub) {
     uint32_t out[4][4];  // [column][4-row group]
@@ -106,19 +162,35 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
       const int col = c0 + T * sub + 4 * cg + c;
       if (col >= cols) continue;
       const v4i v{int32_t(out[c][0]), int32_t(out[c][1]), int32_t(out[c][2]), int32_t(out[c][3])};
-      __builtin_amdgcn_raw_buffer_store_b128(v, dr, uint32_t(col) * uint32_t(rows) + uint32_t(r0 + i0),
-                                             0, kStoreThrough);
+      if constexpr (kAny) {
+        int8_t *const d = dst + int64_t(mat) * int64_t(mat_bytes) + int64_t(col) * rows + r0 + i0;
+        if (n == 16) {
+          __builtin_memcpy(d, &v, 16);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 15; ++e)
+            if (e < n) d[e] = int8_t(uint32_t(v[e >> 2]) >> (8 * (e & 3)));
+        }
+      } else {
+        __builtin_amdgcn_raw_buffer_store_b128(
+            v, dr, uint32_t(col) * uint32_t(rows) + uint32_t(r0 + i0), 0, kStoreThrough);
+      }
     }
   }
 }
 
-// Dwords: the tile has a 132-byte pitch (33 dwords: the 32 rows of one
-// column fall in distinct banks); each lane gathers 4 rows of one column.
+// Dwords: 64 x 64 tiles, so that both sides move in 256-byte pieces and each
+// lane has four 16-byte loads in flight.  A 65-dword pitch puts the 16 pieces
+// x 4 rows of a wave's LDS accesses in 64 distinct banks on both sides.  kAny
+// as above: a lane's four rows end with the tile's last row, single dwords in
+// a last tile of fewer than four.
+template <bool kAny, int kPolicy>
 __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t *src, int8_t *dst,
-                                                                   int rows, int cols, int tiles_r,
+                                                                   int64_t batch, int rows,
+                                                                   int cols, int tiles_r,
                                                                    int tiles_c) {
-  constexpr int T = kTileRowBytes / 4;  // tile side in dwords
-  __shared__ uint32_t tile[T * kLdsPitch / 4];
+  constexpr int T = kDwordTile, kPitch = T + 1;
+  __shared__ uint32_t tile[T * kPitch];
   const int per_mat = tiles_r * tiles_c;
   const int mat = int(blockIdx.x) / per_mat;
   const int t = int(blockIdx.x) - mat * per_mat;
@@ -129,30 +201,58 @@ __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t 
   const auto dr = make_rsrc(dst + size_t(mat) * mat_bytes, uint32_t(mat_bytes));
   const int r0 = tr * T, c0 = tc * T;
   const uint32_t row_bytes = uint32_t(cols) * 4;
-  // read: tile row i = source row r0 + i, bytes [c0*4, c0*4 + 128)
-  for (int idx = threadIdx.x; idx < T * 8; idx += kThreads) {
-    const int i = idx >> 3, piece = idx & 7;
+  const int piece = threadIdx.x & 15, line = threadIdx.x >> 4;
+  // read: tile row i = source row r0 + i, bytes [c0*4, c0*4 + 256)
+  v4i in[T / 16];
+#pragma unroll
+  for (int u = 0; u < T / 16; ++u) {
+    const int i = line + 16 * u;
     const uint32_t cb = uint32_t(c0 * 4 + piece * 16);
     const bool ok = r0 + i < rows && cb < row_bytes;
-    const v4i v = load16(sr, ok ? uint32_t(r0 + i) * row_bytes + cb : kOutOfRange);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) tile[(i * kLdsPitch + piece * 16) / 4 + e] = uint32_t(v[e]);
+    if constexpr (kAny)
+      in[u] = ok ? load16_any(src, int64_t(mat) * int64_t(mat_bytes) +
+                                       int64_t(r0 + i) * row_bytes + cb, batch * int64_t(mat_bytes))
+                 : v4i{0, 0, 0, 0};
+    else
+      in[u] = load16(sr, ok ? uint32_t(r0 + i) * row_bytes + cb : kOutOfRange);
   }
+#pragma unroll
+  for (int u = 0; u < T / 16; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tile[(line + 16 * u) * kPitch + piece * 4 + e] = uint32_t(in[u][e]);
   __syncthreads();
-  // write: output row j = column c0 + j, bytes [r0*4, r0*4 + 128): the lane
-  // gathers tile rows i0 .. i0 + 3 of column j (rows % 4 == 0: the 4 rows are
-  // all inside the matrix or all outside)
+  // write: output row j = column c0 + j, bytes [r0*4, r0*4 + 256): the lane
+  // gathers tile rows i0 .. i0 + 3 of column j (!kAny: rows % 4 == 0, the 4
+  // rows are all inside the matrix or all outside)
   const uint32_t out_row_bytes = uint32_t(rows) * 4;
-  for (int idx = threadIdx.x; idx < T * 8; idx += kThreads) {
-    const int j = idx >> 3, piece = idx & 7;
-    const int i0 = piece * 4;
-    const int c = c0 + j;
-    if (c >= cols || r0 + i0 >= rows) continue;
+  int i0 = piece * 4;
+  if (r0 + i0 >= rows) return;
+  const int live = min(T, rows - r0);
+  if (kAny && i0 + 4 > live) i0 = max(0, live - 4);
+  const int n = kAny ? min(4, live - i0) : 4;  // < 4 only in a tile of fewer rows
+#pragma unroll
+  for (int u = 0; u < T / 16; ++u) {
+    const int j = line + 16 * u, c = c0 + j;
+    if (c >= cols) continue;
     v4i v;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = int32_t(tile[((i0 + e) * kLdsPitch) / 4 + j]);
-    __builtin_amdgcn_raw_buffer_store_b128(v, dr, uint32_t(c) * out_row_bytes + uint32_t(r0 + i0) * 4,
-                                           0, 0);
+    for (int e = 0; e < 4; ++e) v[e] = int32_t(tile[(i0 + e) * kPitch + j]);
+    if constexpr (kAny) {
+      int8_t *const d = dst + int64_t(mat) * int64_t(mat_bytes) + int64_t(c) * out_row_bytes +
+                        int64_t(r0 + i0) * 4;
+      if (n == 4) {
+        __builtin_memcpy(d, &v, 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          const int32_t x = v[e];
+          if (e < n) __builtin_memcpy(d + 4 * e, &x, 4);
+        }
+      }
+    } else {
+      __builtin_amdgcn_raw_buffer_store_b128(
+          v, dr, uint32_t(c) * out_row_bytes + uint32_t(r0 + i0) * 4, 0, kPolicy);
+    }
   }
 }
 
@@ -308,30 +408,25 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
   const bool cols16 = (int64_t(cols) * esize) % 16 == 0;
   const auto *in = static_cast<const int8_t *>(src);
   auto *out = static_cast<int8_t *>(dst);
-  if (aligned16 && rows16 && cols16) {
-    const int T = kTileRowBytes / esize;
+  auto tiled = [&](auto any) {
+    constexpr bool kAny = decltype(any)::value;
+    const int T = esize == 1 ? kTileRowBytes : kDwordTile;
     const int tiles_r = (rows + T - 1) / T;
-    if (esize == 1) {
-      // two 128-column tiles per workgroup (256-byte source row pieces)
-      // where the source rows are long enough to fill them
-      const int sub = cols >= 2 * T ? 2 : 1;
-      const int tiles_c = (cols + sub * T - 1) / (sub * T);
-      const int64_t blocks = batch * tiles_r * tiles_c;  // < 2^31: checked by the caller
-      if (sub == 2)
-        hipLaunchKernelGGL(transpose_bytes_tiled<2>, dim3(unsigned(blocks)), dim3(kThreads), 0, s,
-                           in, out, rows, cols, tiles_r, tiles_c);
-      else
-        hipLaunchKernelGGL(transpose_bytes_tiled<1>, dim3(unsigned(blocks)), dim3(kThreads), 0, s,
-                           in, out, rows, cols, tiles_r, tiles_c);
-    } else {
-      const int tiles_c = (cols + T - 1) / T;
-      const int64_t blocks = batch * tiles_r * tiles_c;
-      hipLaunchKernelGGL(transpose_dwords_tiled, dim3(unsigned(blocks)), dim3(kThreads), 0, s, in,
-                         out, rows, cols, tiles_r, tiles_c);
-    }
+    // bytes: two 128-column tiles per workgroup (256-byte source row pieces)
+    // where the source rows are long enough to fill them
+    const int sub = esize == 1 && cols >= 2 * T ? 2 : 1;
+    const int tiles_c = (cols + sub * T - 1) / (sub * T);
+    const int64_t blocks = batch * tiles_r * tiles_c;  // < 2^31: checked by the caller
+    auto kern = esize != 1 ? (total * 4 >= kStreamTransposeBytes
+                                  ? transpose_dwords_tiled<kAny, kStoreStream>
+                                  : transpose_dwords_tiled<kAny, kStoreThrough>)
+                           : sub == 2 ? transpose_bytes_tiled<2, kAny> : transpose_bytes_tiled<1, kAny>;
+    hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kThreads), 0, s, in, out, batch, rows,
+                       cols, tiles_r, tiles_c);
     return launch_status("transpose launch");
-  }
-  if (aligned16 && rows16 && int64_t(cols) * esize * 16 <= kShortLds) {
+  };
+  if (aligned16 && rows16 && cols16) return tiled(std::false_type{});
+  if (aligned16 && rows16 && cols <= kShortMost && int64_t(cols) * esize * 16 <= kShortLds) {
     const int R = int(std::min<int64_t>(128, kShortLds / (int64_t(cols) * esize) / 16 * 16));
     const int tiles = (rows + R - 1) / R;
     const int64_t blocks = batch * tiles;
@@ -343,7 +438,7 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
                          out, rows, cols, R, tiles);
     return launch_status("transpose launch");
   }
-  if (aligned16 && cols16 && int64_t(rows) * esize * 16 <= kShortLds) {
+  if (aligned16 && cols16 && rows <= kShortMost && int64_t(rows) * esize * 16 <= kShortLds) {
     const int wb = int(std::min<int64_t>(kTileRowBytes, kShortLds / (int64_t(rows) * esize) / 16 * 16));
     const int W = wb / esize;
     const int tiles = (cols + W - 1) / W;
@@ -356,6 +451,7 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
                          out, rows, cols, W, tiles);
     return launch_status("transpose launch");
   }
+  if (rows >= kShortSide && cols >= kShortSide) return tiled(std::true_type{});
   const unsigned blocks = unsigned(std::min<int64_t>((total + kThreads - 1) / kThreads, 1 << 20));
   if (esize == 1)
     hipLaunchKernelGGL(transpose_elements<int8_t>, dim3(blocks), dim3(kThreads), 0, s,

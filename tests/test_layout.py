@@ -130,3 +130,42 @@ def test_pack_vect_c_bit_exact(n, h, w, c, v):
     np.testing.assert_array_equal(packed.reshape(n, c // v, h, w, v), oracle.pack_vect_c(x, v))
     back = _run_gpu(lab.unpack_vect_c, packed, x.size, np.int8, n, h, w, c, v)
     np.testing.assert_array_equal(back.reshape(x.shape), x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,rows,cols", [
+    # tiles of the any-length form: partial last tiles of one element, of fewer
+    # rows than a lane stores, and just short of whole, on both sides
+    (1, 16, 2049), (2, 33, 523), (1, 513, 529), (3, 129, 545), (1, 257, 1023), (1, 1025, 17),
+    (2, 576, 641), (1, 519, 4097)])
+def test_transposes_of_any_length_bit_exact(n, rows, cols):
+    from tests.conftest import say
+    rng = np.random.default_rng(rows * cols)
+    say(f"[gpu] transposes {n}x{rows}x{cols}")
+    x = rng.integers(-128, 128, size=(n, rows, cols), dtype=np.int64).astype(np.int8)
+    got = _run_gpu(lab.nchw_to_nhwc, x, x.size, np.int8, n, rows, 1, cols)
+    np.testing.assert_array_equal(got.reshape(n, cols, rows), x.transpose(0, 2, 1))
+    y = rng.integers(-(2 ** 31), 2 ** 31, size=(n, rows, cols), dtype=np.int64).astype(np.int32)
+    got = _run_gpu(lab.nhwk_to_nkhw, y, y.size, np.int32, n, 1, rows, cols)
+    np.testing.assert_array_equal(got.reshape(n, cols, rows), y.transpose(0, 2, 1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("off", [1, 4, 7])
+def test_transposes_between_unaligned_tensors_bit_exact(off):
+    from tests.conftest import say
+    n, rows, cols = 2, 144, 272
+    rng = np.random.default_rng(off)
+    x = rng.integers(-128, 128, size=(n, rows, cols), dtype=np.int64).astype(np.int8)
+    src, dst = lab.DeviceBuffer(x.size + 16), lab.DeviceBuffer(x.size + 16)
+    src.upload(np.concatenate([np.zeros(off, np.int8), x.reshape(-1), np.zeros(16 - off, np.int8)]))
+    dst.fill(0x5A)
+    say(f"[gpu] unaligned transpose, offset {off}")
+    lab.nchw_to_nhwc(src.ptr + off, dst.ptr + off, n, rows, 1, cols)
+    lab.synchronize()
+    out = dst.download(np.int8, x.size + 16)
+    np.testing.assert_array_equal(out[off:off + x.size].reshape(n, cols, rows),
+                                  x.transpose(0, 2, 1))
+    assert (out[:off] == 0x5A).all() and (out[off + x.size:] == 0x5A).all()
+    src.close()
+    dst.close()
