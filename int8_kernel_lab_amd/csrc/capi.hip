@@ -750,9 +750,10 @@ int i8conv_launch_requant(const i8conv_shape *shape, const int8_t *input, const 
   }
   // The 32 x 32 x 32 MFMA kernel requantizes in its epilogue and leaves the
   // workspace alone (16 x 224x224, 32 -> 64 7x7 stride 2: 101 us through the
-  // int32 workspace and the pass, 35 us).
-  if (id == I8CONV_KERNEL_GENERIC && g.gemm_n % 4 == 0 && aligned(output, 4)) {
-    const GemmPlan p = plan_generic(*shape, g);
+  // int32 workspace and the pass, 35 us; in byte stores where N % 4 != 0: 5 x
+  // 120x55, 192 -> 389 1x1: 90 and 22; 4 x 94x94, 256 -> 269: 47 and 16).
+  if (id == I8CONV_KERNEL_GENERIC) {
+    const GemmPlan p = plan_gemm32(*shape, g);
     if (p.m32) {
       ConvArgs args = make_args(*shape, g, input, filter, bias, nullptr);
       args.q_mult = mult;

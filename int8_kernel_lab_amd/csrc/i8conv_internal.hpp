@@ -113,6 +113,7 @@ bool gemm_dma_tile_supported(int bm, int bn);
 // every wave copies and runs MFMAs)
 int gemm_dma_copy_waves(const GemmPlan &p);
 GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g);
+GemmPlan plan_gemm32(const i8conv_shape &s, const i8conv_geometry &g);
 // output tiles of the 16 x 16 MFMA kernels' grid for a layer (the measure of
 // a small or large grid in the dispatch policy)
 int64_t staged_tiles(const i8conv_shape &s, const i8conv_geometry &g);

@@ -27,7 +27,9 @@
 //     than more stage buffers did (R = 2, 4, 6, 9 within 8 %);
 //   * int8 output: each lane requantizes its channel (parameters read once
 //     per tile), and the four lanes of a quad turn their bytes into one
-//     pixel's four channels per lane.
+//     pixel's four channels per lane; other channel counts and alignments
+//     store single bytes, a pixel's 32 channels side by side (4 x 94x94, 256 ->
+//     269 1x1: 16.1 us; int32 and a pass over it, 46.9).
 #include <hip/hip_runtime.h>
 
 #include <limits.h>
@@ -46,8 +48,9 @@ template <int N>
 using Set = std::integral_constant<int, N>;
 
 
-// What the epilogue writes: int32, or requantized int8 (N % 4 == 0).
-enum OutKind { kOutInt32, kOutInt8 };
+// What the epilogue writes: int32, or requantized int8 in 4-byte stores (N % 4
+// == 0, output 4-byte aligned) or byte stores (any N).
+enum OutKind { kOutInt32, kOutInt8, kOutInt8Bytes };
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -94,7 +97,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
   constexpr bool kByte = kOut != kOutInt32;
   constexpr int kParams = kByte ? 3 : 1;  // bias, multipliers, shifts
   constexpr int kParamBytes = kParams * BN * 4;
-  constexpr int ST = FM * FN * (kByte ? 4 : 16);  // stores per wave and tile
+  constexpr int ST = FM * FN * (kOut == kOutInt8 ? 4 : 16);  // stores per wave and tile
   static_assert(CPA >= 1 && CPB >= 1 && BN % (RPC * kWaves) == 0, "tile shape");
   static_assert(KG == 1 || (kLaneTap && FM == 1 && FN == 1 && 4 % KG == 0), "k groups");
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
@@ -393,7 +396,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
         if constexpr (kByte) {
           const auto yr = make_rsrc(a.q_y + size_t(out_m) * size_t(a.gemm_n),
                                     uint32_t(rows) * uint32_t(a.gemm_n));
-          store_quad_int8(v, r, a.q_zp, yr, rows, px0 + 8 * q, oc0, a.gemm_n, lane);
+          store_quad_int8<kOut == kOutInt8Bytes>(v, r, a.q_zp, yr, rows, px0 + 8 * q, oc0, a.gemm_n, lane);
         } else {
           const auto yr = make_rsrc(a.y + size_t(out_m) * size_t(a.gemm_n),
                                     uint32_t(rows) * uint32_t(a.gemm_n) * 4u);
@@ -437,8 +440,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
                                              *reinterpret_cast<const int *>(pq + BN * 8), a.q_zp);
 #pragma unroll
         for (int j = 0; j < FM; ++j)
-          store_block32_int8(acc[i][j], r, a.q_zp, yr, rows, px0 + 32 * j, oc0 + 32 * i, a.gemm_n,
-                             lane);
+          store_block32_int8<kOut == kOutInt8Bytes>(acc[i][j], r, a.q_zp, yr, rows, px0 + 32 * j,
+                                                    oc0 + 32 * i, a.gemm_n, lane);
       }
     }
     if (!again) return;
@@ -472,8 +475,10 @@ int launch_tile(const ConvArgs &a, hipStream_t stream) {
 // evict-first above, ordinary for other pitches and for int8.
 template <int BM, int BN, int WM, int WN, int KG, int GS, bool kLaneTap, int kOcc, int kGroups>
 int launch_out(const ConvArgs &a, hipStream_t s) {
-  if (a.q_y)
+  if (a.q_y && a.gemm_n % 4 == 0 && (reinterpret_cast<uintptr_t>(a.q_y) & 3) == 0)
     return launch_tile<BM, BN, WM, WN, KG, GS, kLaneTap, kOcc, kGroups, kOutInt8, 0>(a, s);
+  if (a.q_y)
+    return launch_tile<BM, BN, WM, WN, KG, GS, kLaneTap, kOcc, kGroups, kOutInt8Bytes, 0>(a, s);
   if (a.gemm_n % 8 != 0)
     return launch_tile<BM, BN, WM, WN, KG, GS, kLaneTap, kOcc, kGroups, kOutInt32, 0>(a, s);
   if (int64_t(a.gemm_m) * a.gemm_n * 4 > kStreamOutputBytes)
@@ -494,10 +499,6 @@ int launch_gemm32(const ConvArgs &args, const GemmPlan &p, void *stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   ConvArgs a = args;
   a.m_step = p.bm;
-  if (a.q_y && a.gemm_n % 4 != 0) {
-    set_error("gemm32: int8 output needs N % 4 == 0");
-    return I8CONV_BAD_ARGUMENT;
-  }
   switch (p.bm * 1000 + p.bn) {
     case 64064:
       if (p.kg == 4) return launch_out<64, 64, 2, 2, 4, 2, true, 4, 1>(a, s);

@@ -80,10 +80,12 @@ __device__ __forceinline__ Requant32 requant32_params(int32_t mult, int32_t shif
 }
 
 // Four pixels px .. px + 3 of a lane's channel (a block's elements 4 g ..)
-// requantized to int8 (n % 4 == 0, window 4-byte aligned): the lane packs
-// their bytes, and the quad's transpose turns them into one pixel's four
-// channels per lane, a 4-byte store; a pixel's 32 channels go out as one
-// 32-byte piece.
+// requantized to int8.  Where n % 4 == 0 and the window is 4-byte aligned the
+// lane packs their bytes, and the quad's transpose turns them into one pixel's
+// four channels per lane, a 4-byte store; a pixel's 32 channels go out as one
+// 32-byte piece.  kBytes (any n, any alignment): the same pieces, a byte per
+// lane and store.
+template <bool kBytes>
 __device__ __forceinline__ void store_quad_int8(v4i acc, const Requant32 &r, int32_t zp,
                                                 __amdgpu_buffer_rsrc_t out, int rows, int px,
                                                 int oc0, int n, int lane) {
@@ -92,6 +94,16 @@ __device__ __forceinline__ void store_quad_int8(v4i acc, const Requant32 &r, int
   for (int e = 0; e < 4; ++e)
     y[e] = uint32_t(r.odd ? requant1_odd(acc[e], r.o.mo, r.o.k, r.o.sh)
                           : requant1(acc[e], r.mult, r.shift, zp));
+  if constexpr (kBytes) {
+    const int oc = oc0 + (lane & 31);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      __builtin_amdgcn_raw_buffer_store_b8(
+          uint8_t(y[e]), out,
+          px + e < rows && oc < n ? uint32_t(px + e) * uint32_t(n) + uint32_t(oc) : kOutOfRange, 0,
+          0);
+    return;
+  }
   const uint32_t lo = __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0400u);
   const uint32_t hi = __builtin_amdgcn_perm(y[3], y[2], 0x0c0c0400u);
   const uint32_t v = quad_transpose(__builtin_amdgcn_perm(hi, lo, 0x05040100u), lane);
@@ -101,13 +113,14 @@ __device__ __forceinline__ void store_quad_int8(v4i acc, const Requant32 &r, int
 }
 
 // One 32 x 32 block of a wave requantized to int8.
+template <bool kBytes = false>
 __device__ __forceinline__ void store_block32_int8(const v16i &acc, const Requant32 &r, int32_t zp,
                                                    __amdgpu_buffer_rsrc_t out, int rows, int px0,
                                                    int oc0, int n, int lane) {
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const v4i v = {acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
-    store_quad_int8(v, r, zp, out, rows, px0 + 4 * (lane >> 5) + 8 * g, oc0, n, lane);
+    store_quad_int8<kBytes>(v, r, zp, out, rows, px0 + 4 * (lane >> 5) + 8 * g, oc0, n, lane);
   }
 }
 

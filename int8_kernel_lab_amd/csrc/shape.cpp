@@ -185,6 +185,25 @@ int64_t staged_tiles(const i8conv_shape &s, const i8conv_geometry &g) {
   return ceil_div(g.gemm_m, p.bm) * ceil_div(g.gemm_n, p.bn);
 }
 
+static void set_gemm32(const i8conv_geometry &g, GemmPlan &p, int bm, int bn) {
+  const int64_t tiles = ceil_div(g.gemm_m, bm) * ceil_div(g.gemm_n, bn);
+  p.m32 = true;
+  p.bm = p.m_step = bm;
+  p.bn = bn;
+  if (bm == 64 && tiles <= 512 && p.stages >= 6) p.kg = p.stages >= 24 && tiles <= 256 ? 4 : 2;
+}
+
+// The 32 x 32 x 32 MFMA kernel's tile for any channel count, or none (below).
+static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
+  auto tiles = [&](int bm, int bn) { return ceil_div(g.gemm_m, bm) * ceil_div(g.gemm_n, bn); };
+  if (g.gemm_n > 64 && tiles(128, 128) >= 256)
+    set_gemm32(g, p, 128, 128);
+  else if (tiles(128, 64) >= 512)
+    set_gemm32(g, p, 128, 64);
+  else if (g.gemm_n > 64 || p.stages >= 6 || tiles(64, 64) > 256)
+    set_gemm32(g, p, 64, 64);
+}
+
 // Which kernel runs a generic layer, and on which tile (microseconds per
 // back-to-back launch on one MI355X, before -> after unless said otherwise).
 // C % 128 != 0: the 32 x 32 x 32 MFMA kernel instead of the register-staged
@@ -220,27 +239,23 @@ GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
   }
   if (!gemm32_eligible(s, g)) return p;
   auto tiles = [&](int bm, int bn) { return ceil_div(g.gemm_m, bm) * ceil_div(g.gemm_n, bn); };
-  int bm = 0, bn = 0;
-  if (p.dma) {
-    if (g.gemm_n > 128 && p.stages >= 8 && tiles(256, 256) >= 512)
-      bm = bn = 256;
-    else if (tiles(p.bm, p.bn) < 128)
-      bm = bn = 64;
-  } else if (g.gemm_n > 64 && tiles(128, 128) >= 256) {
-    bm = bn = 128;
-  } else if (tiles(128, 64) >= 512) {
-    bm = 128, bn = 64;
-  } else if (g.gemm_n > 64 || p.stages >= 6 || tiles(64, 64) > 256) {
-    bm = bn = 64;
-  }
-  if (bm == 64 && tiles(64, 64) <= 512 && p.stages >= 6)
-    p.kg = p.stages >= 24 && tiles(64, 64) <= 256 ? 4 : 2;
-  if (bm > 0) {
-    p.m32 = true;
-    p.bm = bm;
-    p.bn = bn;
-    p.m_step = bm;
-  }
+  if (!p.dma)
+    gemm32_tile(g, p);
+  else if (g.gemm_n > 128 && p.stages >= 8 && tiles(256, 256) >= 512)
+    set_gemm32(g, p, 256, 256);
+  else if (tiles(p.bm, p.bn) < 128)
+    set_gemm32(g, p, 64, 64);
+  return p;
+}
+
+// The 32 x 32 x 32 MFMA kernel's plan for int8 output in byte stores, where
+// the generic kernel's own plan cannot requantize (the pipelined kernel with N
+// % 4 != 0 or a misaligned output).
+GemmPlan plan_gemm32(const i8conv_shape &s, const i8conv_geometry &g) {
+  GemmPlan p = plan_generic(s, g);
+  if (p.m32 || !gemm32_eligible(s, g)) return p;
+  p.pw = false;
+  gemm32_tile(g, p);
   return p;
 }
 

@@ -94,3 +94,44 @@ def test_gemm32_output_at_four_bytes(name):
     poison = np.uint32(0xA5A5A5A5).view(np.int32)
     assert raw[0] == poison and np.all(raw[count + 1:] == poison)
     assert_bit_exact(raw[1:count + 1].reshape(shape.output_shape), oracle.conv(shape, x, w, b), name)
+
+
+BYTE_CASES = {
+    # byte stores of int8: channel tails in each tile and wave grouping, a
+    # pixel tail, more tiles than workgroups, and layers whose int32 output
+    # the pipelined kernel computes
+    "64_k67": lab.ConvShape(1, 13, 11, 80, 67, 3, 3, 1, 1, 1, 1, 1, 1),
+    "64_k95_two_groups": lab.ConvShape(1, 14, 13, 144, 95, 3, 3, 1, 1, 1, 1, 1, 1),
+    "64_k33_four_groups": lab.ConvShape(1, 17, 19, 368, 33, 3, 3, 1, 1, 1, 1, 1, 1),
+    "128x64_k63": lab.ConvShape(5, 115, 119, 48, 63, 3, 1, 1, 0, 1, 1, 1, 1),
+    "128x128_k94": lab.ConvShape(3, 137, 131, 32, 94, 3, 3, 1, 1, 1, 1, 1, 1),
+    "128x128_k255_again": lab.ConvShape(1, 205, 203, 48, 255, 1, 3, 0, 1, 1, 1, 1, 1),
+    "pipelined_k101": lab.ConvShape(2, 101, 97, 128, 101, 3, 3, 1, 1, 2, 2, 1, 1),
+    "pipelined_k130": lab.ConvShape(4, 64, 67, 384, 130, 1, 1, 0, 0, 1, 1, 1, 1),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(BYTE_CASES))
+@pytest.mark.parametrize("off", [0, 3])
+def test_gemm32_int8_byte_stores(name, off):
+    shape = BYTE_CASES[name]
+    if lab.dispatch(shape) != "generic":
+        pytest.skip("another kernel's layer")
+    x, w, b = lab.make_case_data(shape, seed=35)
+    mult, shift = _qparams(shape.k, seed=36)
+    expected = oracle.requantize(oracle.conv(shape, x, w, b), mult, shift, 7)
+    count, need = shape.output_elements, lab.requant_workspace_bytes(shape)
+    bufs = [lab.DeviceBuffer.from_array(a) for a in (x, w, b, mult, shift)]
+    yb, ws = lab.DeviceBuffer(count + 16), lab.DeviceBuffer(max(need, 1))
+    try:
+        yb.fill(0x5A)
+        say(f"[gpu] int8 byte stores, {name} at +{off} bytes")
+        lab.launch_requant(shape, *bufs[:5], 7, yb.ptr + off, ws, need)
+        lab.synchronize()
+        raw = yb.download(np.int8, count + 16)
+    finally:
+        for buf in bufs + [yb, ws]:
+            buf.close()
+    assert (raw[:off] == 0x5A).all() and (raw[off + count:] == 0x5A).all()
+    np.testing.assert_array_equal(raw[off:off + count].reshape(shape.output_shape), expected)
