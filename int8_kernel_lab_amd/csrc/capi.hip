@@ -626,7 +626,9 @@ RequantRoute requant_route(const i8conv_shape &s, const i8conv_geometry &g) {
       pointwise_requant_supported(s.c, int(g.gemm_n)))
     return kRqPointwise;
   if (id == I8CONV_KERNEL_SPLITK && g.gemm_n % 4 == 0) return kRqSplitK;
-  if (id == I8CONV_KERNEL_GENERIC && g.gemm_n % 4 == 0 && plan_generic(s, g).dma) return kRqGemm;
+  if (id == I8CONV_KERNEL_GENERIC && g.gemm_n % 4 == 0 && plan_generic(s, g).dma &&
+      !dispatch_patch_layer(s))
+    return kRqGemm;
   return kRqUnfused;
 }
 
@@ -752,26 +754,31 @@ int i8conv_launch_requant(const i8conv_shape *shape, const int8_t *input, const 
   // workspace alone (16 x 224x224, 32 -> 64 7x7 stride 2: 101 us through the
   // int32 workspace and the pass, 35 us; in byte stores where N % 4 != 0: 5 x
   // 120x55, 192 -> 389 1x1: 90 and 22; 4 x 94x94, 256 -> 269: 47 and 16).
-  if (id == I8CONV_KERNEL_GENERIC) {
-    const GemmPlan p = plan_gemm32(*shape, g);
-    if (p.m32) {
+  // Layers of the other kernels without such an epilogue take it too: one
+  // launch instead of two, whose calls take the host longer than the GPU (24 x
+  // 22x22 dilated 64 -> 64: 15.7 us a call before, 8.5 now).
+  PatchPlan pp;
+  const bool row = id == I8CONV_KERNEL_HALO && plan_halo(*shape, g, &pp) && pp.row;
+  if (id != I8CONV_KERNEL_SPLITK && !row) {
+    const bool vec = g.gemm_n % 4 == 0 && requant_route_aligned(kRqGemm, bias, mult, shift, output);
+    const GemmPlan own = plan_generic(*shape, g);
+    const bool pipelined = own.dma && !own.m32 && !own.pw && vec;
+    const GemmPlan p = pipelined ? own : plan_gemm32(*shape, g);
+    if (pipelined || p.m32) {
       ConvArgs args = make_args(*shape, g, input, filter, bias, nullptr);
       args.q_mult = mult;
       args.q_shift = shift;
       args.q_zp = zero_point;
       args.q_y = output;
-      return launch_gemm32(args, p, stream);
+      return launch_gemm(args, p, stream);
     }
   }
   // The row kernel likewise (32 x 56x56, 64 -> 64: 10.5 + 8.1 us with the
   // pass).
-  if (id == I8CONV_KERNEL_HALO) {
-    PatchPlan pp;
-    if (plan_halo(*shape, g, &pp) && pp.row && !pp.streamed) {
-      const ConvArgs args = make_args(*shape, g, input, filter, bias, nullptr);
-      const RequantArgs q{mult, shift, zero_point, output};
-      return launch_row(args, pp, stream, &q);
-    }
+  if (row && !pp.streamed) {
+    const ConvArgs args = make_args(*shape, g, input, filter, bias, nullptr);
+    const RequantArgs q{mult, shift, zero_point, output};
+    return launch_row(args, pp, stream, &q);
   }
   int32_t *acc = static_cast<int32_t *>(workspace);
   void *conv_ws = static_cast<char *>(workspace) + acc_bytes;

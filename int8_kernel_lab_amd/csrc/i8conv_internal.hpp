@@ -152,6 +152,10 @@ bool plan_strip(const i8conv_shape &s, const i8conv_geometry &g, PatchPlan *p);
 
 // Dispatch policy (policy.cpp): an eligible kernel id, or -1 for a bad shape.
 int dispatch(const i8conv_shape &s);
+// Generic layers whose int8 launch asks for the int32 workspace all the same
+// (and leaves it alone): small grids of stride-1 spatial filters, which halo
+// and strip plans also cover and which callers have always sized it for
+bool dispatch_patch_layer(const i8conv_shape &s);
 
 ConvArgs make_args(const i8conv_shape &s, const i8conv_geometry &g,
                    const int8_t *x, const int8_t *w, const int32_t *bias,

@@ -229,7 +229,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
   };
   // per-channel parameters of the tile at tile_n into parameter slot `slot`
   auto copy_params = [&](int slot) {
-    if (wave_id * 64 < BN) {
+    if (wave_id * 64 + lane < BN) {
       const uint32_t bytes = uint32_t(a.gemm_n) * 4u;
       const uint32_t off = uint32_t(tile_n + wave_id * 64 + lane) * 4u;
       const uint32_t dst = lds_params + uint32_t(slot * kParamBytes) + uint32_t(wave_id) * 256u;
@@ -504,6 +504,7 @@ int launch_gemm32(const ConvArgs &args, const GemmPlan &p, void *stream) {
       if (p.kg == 4) return launch_out<64, 64, 2, 2, 4, 2, true, 4, 1>(a, s);
       if (p.kg == 2) return launch_out<64, 64, 2, 2, 2, 2, true, 4, 2>(a, s);
       return launch_out<64, 64, 2, 2, 1, 2, true, 4, 4>(a, s);
+    case 128032: return launch_out<128, 32, 4, 1, 1, 1, true, 3, 3>(a, s);
     case 128064: return launch_out<128, 64, 2, 2, 1, 1, true, 3, 3>(a, s);
     // four waves of 64 x 64: eight of 32 x 64 spill at four waves per SIMD (7 x
     // 196x196, 80 -> 209 1x3: 72 us, 48 with four; 256x256, 64 -> 255: 23.6, 21)

@@ -13,14 +13,13 @@
 //      batch 1: it won all of them; at 24 tiles and 18 stages the generic
 //      GEMM won, 15.0 vs 15.7 us, and on a 32x32 3x3 layer of 9 stages the
 //      halo kernel, 9.3 vs 11.0 us);
-//   3. the pipelined generic GEMM (C % 128 == 0) when its grid has at least
-//      128 tiles: large layers of any filter (it beat every halo/strip plan
-//      from 28x28 x 32 images up to 256x256 x 16, stride 1 or 2, 3x3 or 5x5,
-//      dilated or not);
-//      Likewise the 32 x 32 x 32 MFMA GEMM (C % 128 != 0) wherever it has a
-//      plan: it beat the halo and strip kernels on every such layer (1x3, 64
-//      -> 128: 14.2 against 22.3 us; 256x256, 64 -> 63, 69, 255: 9.3, 11.1,
-//      21 against 16.4, 19.2, 43; dilated 64 -> 128: 5.3 against 6.3);
+//   3. the generic GEMM wherever it runs its pipelined form (C % 128 == 0) or
+//      the 32 x 32 x 32 MFMA one: they beat every halo and strip plan without
+//      row streaming (C % 128 == 0: 3 x 44x44, 512 -> 160 3x1: 25.6 -> 8.3;
+//      36x36, 512 -> 256 3x3: 45.9 -> 16.1; 2 x 40x40 dilated 256 -> 192: 27.7
+//      -> 10.0; 4 x 60x30, 128 -> 64 1x3: 7.9 -> 4.5; others: 1x3, 64 -> 128:
+//      22.3 -> 14.2; 256x256, 64 -> 63, 69, 255: 16.4, 19.2, 43 -> 9.3, 11.1,
+//      21; dilated 64 -> 128: 6.3 -> 5.3);
 //   4. otherwise an input-reuse kernel for a stride-1 spatial filter
 //      (r*s > 1): halo when eligible, else strip (small dilated layers,
 //      asymmetric 1x3/3x1, C = 64 layers wider than the row kernel's four
@@ -36,7 +35,11 @@
 namespace i8conv {
 
 namespace {
-int dispatch_uncached(const i8conv_shape &s);
+struct Choice {
+  int id;
+  bool patch;  // dispatch_patch_layer
+};
+Choice dispatch_uncached(const i8conv_shape &s);
 
 // The policy is a pure function of the shape, and its planners search
 // (the resident-rows plan of a 64x64 dilated layer takes ~50 us of host
@@ -45,7 +48,7 @@ int dispatch_uncached(const i8conv_shape &s);
 // cost a lookup.
 struct DispatchEntry {
   i8conv_shape shape;
-  int id;
+  Choice choice;
   bool used;
 };
 constexpr size_t kDispatchCache = 64;
@@ -58,41 +61,46 @@ size_t shape_slot(const i8conv_shape &s) {
   for (size_t i = 0; i < sizeof(s) / sizeof(int); ++i) h = (h ^ uint32_t(f[i])) * 16777619u;
   return h % kDispatchCache;
 }
-}  // namespace
 
-int dispatch(const i8conv_shape &s) {
+Choice lookup(const i8conv_shape &s) {
   static_assert(sizeof(i8conv_shape) == 13 * sizeof(int), "shape fields are 13 ints");
   const size_t slot = shape_slot(s);
   {
     std::lock_guard<std::mutex> lock(g_dispatch_mutex);
     const DispatchEntry &e = g_dispatch_cache[slot];
-    if (e.used && std::memcmp(&e.shape, &s, sizeof(s)) == 0) return e.id;
+    if (e.used && std::memcmp(&e.shape, &s, sizeof(s)) == 0) return e.choice;
   }
-  const int id = dispatch_uncached(s);
+  const Choice choice = dispatch_uncached(s);
   std::lock_guard<std::mutex> lock(g_dispatch_mutex);
-  g_dispatch_cache[slot] = DispatchEntry{s, id, true};
-  return id;
+  g_dispatch_cache[slot] = DispatchEntry{s, choice, true};
+  return choice;
 }
+}  // namespace
+
+int dispatch(const i8conv_shape &s) { return lookup(s).id; }
+
+bool dispatch_patch_layer(const i8conv_shape &s) { return lookup(s).patch; }
 
 namespace {
-int dispatch_uncached(const i8conv_shape &s) {
+Choice dispatch_uncached(const i8conv_shape &s) {
   i8conv_geometry g;
-  if (derive(s, &g) != I8CONV_OK) return -1;
+  if (derive(s, &g) != I8CONV_OK) return {-1, false};
   PatchPlan pp;
   const bool halo = plan_halo(s, g, &pp);
-  if (halo && pp.row) return I8CONV_KERNEL_HALO;
+  if (halo && pp.row) return {I8CONV_KERNEL_HALO, false};
   const GemmPlan gp = plan_generic(s, g);
   const int64_t tiles = staged_tiles(s, g);
   const bool spatial = int64_t(s.r) * s.s > 1;
   if (tiles <= 16 && (gp.stages >= 16 || (!spatial && gp.stages >= 8)))
-    return I8CONV_KERNEL_SPLITK;
-  if (gp.m32 && !gp.dma) return I8CONV_KERNEL_GENERIC;
-  if (gp.dma && tiles >= 128) return I8CONV_KERNEL_GENERIC;
-  if (spatial && s.stride_h == 1 && s.stride_w == 1) {
-    if (halo) return I8CONV_KERNEL_HALO;
-    if (plan_strip(s, g, &pp)) return I8CONV_KERNEL_STRIP;
+    return {I8CONV_KERNEL_SPLITK, false};
+  const bool reuse = spatial && s.stride_h == 1 && s.stride_w == 1;
+  const bool patch = reuse && gp.dma && tiles < 128 && (halo || plan_strip(s, g, &pp));
+  if (gp.m32 || gp.dma) return {I8CONV_KERNEL_GENERIC, patch};
+  if (reuse) {
+    if (halo) return {I8CONV_KERNEL_HALO, false};
+    if (plan_strip(s, g, &pp)) return {I8CONV_KERNEL_STRIP, false};
   }
-  return I8CONV_KERNEL_GENERIC;
+  return {I8CONV_KERNEL_GENERIC, false};
 }
 }  // namespace
 

@@ -190,16 +190,19 @@ static void set_gemm32(const i8conv_geometry &g, GemmPlan &p, int bm, int bn) {
   p.m32 = true;
   p.bm = p.m_step = bm;
   p.bn = bn;
-  if (bm == 64 && tiles <= 512 && p.stages >= 6) p.kg = p.stages >= 24 && tiles <= 256 ? 4 : 2;
+  if (bm == 64 && p.stages >= 6 && tiles <= (p.stages >= 8 ? 1152 : 512))
+    p.kg = p.stages >= 24 && tiles <= 256 ? 4 : 2;
 }
 
 // The 32 x 32 x 32 MFMA kernel's tile for any channel count, or none (below).
 static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
   auto tiles = [&](int bm, int bn) { return ceil_div(g.gemm_m, bm) * ceil_div(g.gemm_n, bn); };
-  if (g.gemm_n > 64 && tiles(128, 128) >= 256)
+  if (g.gemm_n > 64 && p.stages >= 8 && tiles(64, 64) <= 1152)
+    set_gemm32(g, p, 64, 64);
+  else if (g.gemm_n > 64 && tiles(128, 128) >= 256)
     set_gemm32(g, p, 128, 128);
   else if (tiles(128, 64) >= 512)
-    set_gemm32(g, p, 128, 64);
+    set_gemm32(g, p, 128, g.gemm_n <= 32 ? 32 : 64);
   else if (g.gemm_n > 64 || p.stages >= 6 || tiles(64, 64) > 256)
     set_gemm32(g, p, 64, 64);
 }
@@ -211,8 +214,13 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
 //   * 128 x 128, two workgroups per unit, for N > 64 with at least 256 tiles
 //     (256x256, 64 -> 255 3x3: 43 -> 21; 7 x 196x196, 80 -> 209 1x3: 202 ->
 //     48; 16 x 224x224, 32 -> 96 4x4 stride 4: 15.8 -> 8.6, 64 x 64: 10.0);
+//     But at most 1152 tiles of 64 x 64 and eight or more stages: those with
+//     two groups of waves (2 x 238x25, 400 -> 288 3x3: 41 -> 30; 22 x 40x40,
+//     400 -> 96 1x3: 19.5 -> 15.4, int8 25.4 -> 17.4);
 //   * 128 x 64, three per unit, with at least 512 tiles (16 x 224x224, 32 ->
-//     64 7x7 stride 2: 101 -> 35; 256x256, 64 -> 63: 16.4 -> 9.3);
+//     64 7x7 stride 2: 101 -> 35; 256x256, 64 -> 63: 16.4 -> 9.3), 128 x 32
+//     for at most 32 channels (30 x 97x108, 32 -> 32 7x7 stride 2: 128 x 64
+//     18.0 -> 15.6; 16 x 56x56, 96 -> 32: 8.0 -> 7.3);
 //   * 64 x 64, four per unit, below that (416x416, 32 -> 64 3x3 stride 2: 7.3
 //     -> 5.9, 128 x 64: 7.6).  With at most two tiles per unit a stage's
 //     latency counts, not its throughput: then groups of waves share a tile's
@@ -225,8 +233,14 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
 //     than six stages and one round of 64-pixel tiles (2 x 30x30, 48 -> 64
 //     3x3: 5.5 against 6.0).
 // C % 128 == 0: the pipelined kernel, except
-//   * grids of fewer than 128 of its tiles, which leave half the units idle:
-//     64 x 64 (52x52, 256 -> 512 3x3 stride 2: 12.7 -> 7.9 with two groups);
+//   * at most 128 tiles of 64 x 64, six to 18 stages: 64 x 64 (52x52, 256 ->
+//     512 3x3 stride 2: 10.0 -> 7.3 with two groups; 2 x 64x64, 128 -> 64: 7.0
+//     -> 5.9).  More tiles or stages stay (2 x 40x40, 256 -> 192, 150 tiles:
+//     10.0 against 12.1; 36x36, 512 -> 256, 36 stages: 16.1 against 18.4), but
+//     for grids so small that the policy splits their reduction;
+//   * three or four stages and a last channel tile that is not whole: 128 x 64
+//     from 512 tiles on (64 x 28x28, 384 -> 192 1x1: 19.0 -> 12.3; 53 x 62x62,
+//     512 -> 288: 103 -> 94; two stages, 32 x 56x56, 256 -> 160: 24.7, 25.4);
 //   * at least two rounds of 256 x 256 tiles: a third fewer copied bytes per
 //     operation (16 x 256x256, 256 -> 256 3x3: 780 -> 706; 5x5 stride 2 with
 //     int8 output: 484 -> 457).
@@ -243,19 +257,22 @@ GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
     gemm32_tile(g, p);
   else if (g.gemm_n > 128 && p.stages >= 8 && tiles(256, 256) >= 512)
     set_gemm32(g, p, 256, 256);
-  else if (tiles(p.bm, p.bn) < 128)
+  else if (p.stages >= 3 && p.stages <= 4 && g.gemm_n % 128 != 0 && tiles(128, 64) >= 512)
+    set_gemm32(g, p, 128, 64);
+  else if (p.stages >= 6 && tiles(64, 64) <= 128 && (p.stages <= 18 || tiles(p.bm, p.bn) <= 16))
     set_gemm32(g, p, 64, 64);
   return p;
 }
 
 // The 32 x 32 x 32 MFMA kernel's plan for int8 output in byte stores, where
-// the generic kernel's own plan cannot requantize (the pipelined kernel with N
-// % 4 != 0 or a misaligned output).
+// the dispatched kernel cannot requantize (the pipelined kernel with N % 4 != 0
+// or a misaligned output, the register-staged, halo and strip kernels).
 GemmPlan plan_gemm32(const i8conv_shape &s, const i8conv_geometry &g) {
   GemmPlan p = plan_generic(s, g);
   if (p.m32 || !gemm32_eligible(s, g)) return p;
   p.pw = false;
   gemm32_tile(g, p);
+  if (!p.m32) set_gemm32(g, p, 64, 64);
   return p;
 }
 
@@ -422,13 +439,13 @@ bool plan_row(const i8conv_shape &s, const i8conv_geometry &g, PatchPlan *p) {
       break;
     }
   }
+  if (!found) return false;
   // 128 channels in 64-channel slices: the form with copy waves when it fits
-  if (found && s.c == 128 && p->bn == 64 && rowpass_nfr(g.out_w) != 0 &&
-      p->rows - 2 <= rowpass_max_rows(rowpass_nfr(g.out_w)) &&
-      rowpass_lds_bytes(s.w + 2 * s.pad_w, p->rows - 2) <= size_t(kLdsBudget) &&
-      g.output_elements * 4 <= INT32_MAX)
-    p->streamed = true;
-  return found;
+  p->streamed = s.c == 128 && p->bn == 64 && rowpass_nfr(g.out_w) != 0 &&
+                p->rows - 2 <= rowpass_max_rows(rowpass_nfr(g.out_w)) &&
+                rowpass_lds_bytes(s.w + 2 * s.pad_w, p->rows - 2) <= size_t(kLdsBudget) &&
+                g.output_elements * 4 <= INT32_MAX;
+  return true;
 }
 
 bool finish_patch_plan(const i8conv_shape &s, const i8conv_geometry &g,

@@ -34,7 +34,10 @@ CASES = {
     "64_k128": ("64px x 64oc", lab.ConvShape(18, 31, 33, 32, 36, 2, 2, 0, 0, 1, 1, 1, 1)),
     # 128 x 64: C = 32 and 48, odd channel counts, padding wider than the image
     "128x64_c32_k63": ("128px x 64oc", lab.ConvShape(5, 121, 119, 32, 63, 3, 3, 1, 1, 1, 1, 1, 1)),
-    "128x64_c48_k4": ("128px x 64oc", lab.ConvShape(1, 250, 263, 48, 4, 7, 7, 3, 3, 1, 1, 1, 1)),
+    # 128 x 32: at most 32 channels, also of pixel rows past the image
+    "128x32_c48_k4": ("128px x 32oc", lab.ConvShape(1, 250, 263, 48, 4, 7, 7, 3, 3, 1, 1, 1, 1)),
+    "128x32_c32_k32": ("128px x 32oc", lab.ConvShape(3, 151, 149, 32, 32, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "128x64_c48_k36": ("128px x 64oc", lab.ConvShape(1, 250, 263, 48, 36, 5, 5, 3, 3, 1, 1, 1, 1)),
     # 128 x 128: N = 65 and 255 (one, then two channel tiles), 1x3 dilated
     "128_k65": ("128px x 128oc", lab.ConvShape(2, 129, 130, 64, 65, 3, 3, 1, 1, 1, 1, 1, 1)),
     "128_k255": ("128px x 128oc", lab.ConvShape(1, 130, 131, 64, 255, 1, 3, 0, 2, 1, 1, 1, 2)),
@@ -102,10 +105,12 @@ BYTE_CASES = {
     # the pipelined kernel computes
     "64_k67": lab.ConvShape(1, 13, 11, 80, 67, 3, 3, 1, 1, 1, 1, 1, 1),
     "64_k95_two_groups": lab.ConvShape(1, 14, 13, 144, 95, 3, 3, 1, 1, 1, 1, 1, 1),
-    "64_k33_four_groups": lab.ConvShape(1, 17, 19, 368, 33, 3, 3, 1, 1, 1, 1, 1, 1),
+    "64_k33_four_groups": lab.ConvShape(2, 27, 25, 368, 33, 3, 3, 1, 1, 1, 1, 1, 1),
     "128x64_k63": lab.ConvShape(5, 115, 119, 48, 63, 3, 1, 1, 0, 1, 1, 1, 1),
+    "128x32_k31": lab.ConvShape(2, 187, 185, 48, 31, 1, 3, 0, 1, 1, 1, 1, 1),
     "128x128_k94": lab.ConvShape(3, 137, 131, 32, 94, 3, 3, 1, 1, 1, 1, 1, 1),
     "128x128_k255_again": lab.ConvShape(1, 205, 203, 48, 255, 1, 3, 0, 1, 1, 1, 1, 1),
+    "64_k30_halo_layer": lab.ConvShape(3, 22, 21, 64, 30, 3, 3, 2, 2, 1, 1, 2, 2),
     "pipelined_k101": lab.ConvShape(2, 101, 97, 128, 101, 3, 3, 1, 1, 2, 2, 1, 1),
     "pipelined_k130": lab.ConvShape(4, 64, 67, 384, 130, 1, 1, 0, 0, 1, 1, 1, 1),
 }
@@ -116,8 +121,6 @@ BYTE_CASES = {
 @pytest.mark.parametrize("off", [0, 3])
 def test_gemm32_int8_byte_stores(name, off):
     shape = BYTE_CASES[name]
-    if lab.dispatch(shape) != "generic":
-        pytest.skip("another kernel's layer")
     x, w, b = lab.make_case_data(shape, seed=35)
     mult, shift = _qparams(shape.k, seed=36)
     expected = oracle.requantize(oracle.conv(shape, x, w, b), mult, shift, 7)
