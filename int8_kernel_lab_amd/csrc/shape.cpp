@@ -445,6 +445,30 @@ bool plan_row(const i8conv_shape &s, const i8conv_geometry &g, PatchPlan *p) {
                 p->rows - 2 <= rowpass_max_rows(rowpass_nfr(g.out_w)) &&
                 rowpass_lds_bytes(s.w + 2 * s.pad_w, p->rows - 2) <= size_t(kLdsBudget) &&
                 g.output_elements * 4 <= INT32_MAX;
+  // A grid of one round and a bit (273 workgroups) takes fewer blocks per
+  // image, so that it is one round, where a block's input rows then grow by at
+  // most a quarter, or by half where two blocks do not fit a unit's LDS (us per
+  // launch before -> after): 21 x 36x36, 64 -> 64: 8.6 -> 5.3 (same rows); 37 x
+  // 20x20, 256 -> 64: 15.5 -> 9.7 (5 -> 6); 9 x 50x50, 64 -> 192: 14.3 -> 8.3
+  // (7 -> 8); 13 x 30x30, 128 -> 416, 125 KB of LDS: 20.3 -> 13.3 (12 -> 17); 25
+  // x 24x24, 64 -> 256, 72 KB, would take 14 rows instead of 10: 8.4 -> 8.9,
+  // int8 9.7 -> 13.4.
+  const int64_t per_block = int64_t(s.n) * p->tiles_n;
+  const int64_t fewer = 256 / per_block;
+  if (!p->streamed && per_block * p->ranges > 256 && fewer >= 1 && fewer < p->ranges) {
+    const int64_t slot = int64_t(halo_ring_slot_bytes(p->bn / 64));
+    const int64_t rows = ceil_div(g.out_h, fewer) + 2;
+    const int64_t input_lds = kHaloBiasLds + rows * row.row_bytes;
+    const int64_t ring = std::min<int64_t>({kHaloRing, chunks, (kLdsBudget - input_lds) / slot});
+    const int64_t now = kHaloBiasLds + p->rows * row.row_bytes + p->ring * slot;
+    if (input_lds < kLdsBudget && ring >= 1 &&
+        4 * rows <= (2 * now > kLdsBudget ? 6 : 5) * int64_t(p->rows)) {
+      p->ranges = int(fewer);
+      p->rows = int(rows);
+      p->ring = int(ring);
+      p->stage_pixels = int(rows * (s.w + 2 * s.pad_w));
+    }
+  }
   return true;
 }
 

@@ -7,6 +7,7 @@ import pytest
 import int8_kernel_lab_amd as lab
 from oracle import oracle
 from tests.conftest import say
+from tests.test_gpu_parity import assert_bit_exact, run_kernel
 from tests.test_requant import _qparams
 
 CASES = {
@@ -38,3 +39,32 @@ def test_row_requant_bit_exact(name, form):
     got = lab.conv2d_requant(x, w, b, mult, shift, -6, shape)
     exp = oracle.requantize(oracle.conv(shape, x, w, b), mult, shift, -6)
     np.testing.assert_array_equal(got, exp)
+
+
+ONE_ROUND = {
+    # grids of just over 256 workgroups: fewer blocks per image, uneven ones
+    # among them, one and two channel slices
+    "c64_k64_12_blocks": (lab.ConvShape(21, 35, 36, 64, 64, 3, 3, 1, 1, 1, 1, 1, 1), "12 row blocks"),
+    "c64_k192_9_blocks": (lab.ConvShape(9, 50, 50, 64, 192, 3, 3, 1, 1, 1, 1, 1, 1), "9 row blocks"),
+    "c128_k416_2_blocks": (lab.ConvShape(13, 29, 30, 128, 416, 3, 3, 1, 1, 1, 1, 1, 1), "2 row blocks"),
+    "c256_k60_6_blocks": (lab.ConvShape(37, 20, 20, 256, 60, 3, 3, 1, 1, 1, 1, 1, 1), "6 row blocks"),
+}
+
+
+@pytest.mark.parametrize("name", sorted(ONE_ROUND))
+def test_row_plan_of_one_round(name):
+    shape, blocks = ONE_ROUND[name]
+    assert blocks in lab.describe("halo", shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(ONE_ROUND))
+def test_row_one_round_bit_exact(name):
+    shape = ONE_ROUND[name][0]
+    x, w, b = lab.make_case_data(shape, seed=44)
+    say(f"[gpu] row kernel {name} {shape}")
+    acc = oracle.conv(shape, x, w, b)
+    assert_bit_exact(run_kernel("halo", shape, x, w, b), acc, name)
+    mult, shift = _qparams(shape.k, seed=45)
+    np.testing.assert_array_equal(lab.conv2d_requant(x, w, b, mult, shift, 4, shape),
+                                  oracle.requantize(acc, mult, shift, 4))
