@@ -172,10 +172,10 @@ int i8conv_launch_noalloc(int id, const i8conv_shape *shape, const int8_t *input
 int i8conv_requantize(const int32_t *acc, int64_t pixels, int32_t channels,
                       const int32_t *mult, const int32_t *shift,
                       int32_t zero_point, int8_t *output, void *stream);
-/* 1 when the dispatched kernel for `shape` requantizes in its own epilogue
- * (no int32 tensor is written), 0 when the convolution goes through an
- * int32 workspace and a requantizing pass.  Fused: the row kernel with
- * copy waves; the generic kernel's pointwise streaming form (1x1 stride-1
+/* 1 when an int8 launch of `shape` needs no int32 workspace, 0 when it asks
+ * for one (the kernels that have a requantizing epilogue all the same leave it
+ * alone, the others write int32 there and a requantizing pass follows).
+ * Fused: the row kernel with copy waves; the generic kernel's pointwise streaming form (1x1 stride-1
  * unpadded layers with output-channel slices of 64 or 128), when bias,
  * mult, shift and output are 16-byte aligned; split-K's second pass (N % 4
  * == 0), when bias, mult and shift are 16-byte aligned; the pipelined GEMM's

@@ -5,9 +5,8 @@
 // (requant1 in i8conv_device.hpp).  An HBM-bound elementwise pass: each
 // thread reads 16 bytes of int32 (four channels of one pixel) and writes
 // their four int8 values as one dword; a scalar form covers N % 4 != 0.
-// The row kernel with copy waves applies the same function in its epilogue
-// instead (kernel_rowpass.hip); every other kernel's output goes through
-// this pass.
+// The convolution kernels apply the same function in their epilogues instead;
+// this pass serves i8conv_requantize and split-K layers with N % 4 != 0.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
