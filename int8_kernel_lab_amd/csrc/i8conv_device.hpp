@@ -372,6 +372,30 @@ __device__ __forceinline__ v4i mfma16(v4i a, v4i b, v4i c) {
 
 #endif  // __HIPCC__
 
+// The tiles of a persistent workgroup: first, first + step, ... below last.
+// Workgroup b runs on XCD b % 8, and each XCD walks a contiguous run of tiles
+// (neighbours share input rows and filters in its L2).  The runs' lengths
+// differ by at most one, in the same order as the XCDs' workgroup counts: no
+// workgroup gets more than ceil(tiles / workgroups) tiles where the grid is
+// one round of them or a multiple of 8 workgroups.  (Runs split at tiles * xcd
+// / 8 instead leave a workgroup two tiles in a row on a one-round grid that is
+// no multiple of 8: 4 x 28x28, 192 -> 192 3x3, 147 tiles: 10.6 us, 7.0 so; 7 x
+// 38x38, 288 -> 32, 158 tiles: 13.7 and 8.4.)
+struct TileRun {
+  int first, last, step;
+};
+I8_HD inline TileRun xcd_tile_run(int tiles, int workgroups, int block) {
+  const int xcds = workgroups >= 8 ? 8 : 1;
+  const int xcd = block % xcds;
+  TileRun r;
+  r.step = (workgroups - xcd + xcds - 1) / xcds;  // workgroups on this XCD
+  const int each = tiles / xcds, more = tiles % xcds;
+  const int begin = xcd * each + (xcd < more ? xcd : more);
+  r.first = begin + block / xcds;
+  r.last = begin + each + (xcd < more ? 1 : 0);
+  return r;
+}
+
 // LDS bank rule for ds_read_b128 on gfx950, measured with the LDS probe
 // (kernel_probe.hip): a wave's read runs at full rate when every 32
 // consecutive lanes address distinct 16-byte units modulo 512 bytes and

@@ -252,15 +252,9 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
     }
   };
 
-  // workgroup b runs on XCD b % 8: each XCD walks a contiguous run of tiles
-  const int G = int(gridDim.x);
-  const int xcds = G >= 8 ? 8 : 1;
-  const int xcd = int(blockIdx.x) % xcds;
-  const int step = (G - xcd + xcds - 1) / xcds;  // workgroups on this XCD
-  const int first = int(int64_t(tiles) * xcd / xcds);
-  const int last = int(int64_t(tiles) * (xcd + 1) / xcds);
-  int t = first + int(blockIdx.x) / xcds;
-  if (t >= last) return;
+  const TileRun run = xcd_tile_run(tiles, int(gridDim.x), int(blockIdx.x));
+  int t = run.first;
+  if (t >= run.last) return;
 
   // fragment read offsets in a stage buffer: row 32 i + lane % 32 of the
   // wave's filter (or pixel) rows, chunk 2 ks + lane / 32
@@ -363,8 +357,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
     }
 
     const int out_m = tile_m, out_n = tile_n, out_end = m_end;
-    t += step;
-    const bool again = t < last;
+    t += run.step;
+    const bool again = t < run.last;
     if constexpr (KG > 1) {
       // each wave's sums go to its 4 KB of the first stage buffers (every
       // wave has read its last stage), four elements per 1 KB; then group g

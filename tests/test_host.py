@@ -75,6 +75,16 @@ def test_lds_layouts_are_conflict_free(tmp_path):
     assert out.stdout.startswith("ok ")
 
 
+def test_persistent_grids_walk_each_tile_once_and_evenly(tmp_path):
+    exe = tmp_path / "tile_run_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", CSRC, "-I", os.path.join(ROOT, "include"),
+                    os.path.join(ROOT, "tests", "tile_run_check.cpp"), "-o", str(exe)],
+                   check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert out.stdout.startswith("ok ")
+
+
 # ---- workload tables (gen_case.py:15-36) ------------------------------------
 
 def test_workload_loader_errors(tmp_path):
