@@ -380,6 +380,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
       if constexpr (kByte)
         r = requant32_params(*reinterpret_cast<const int *>(pq + BN * 4),
                              *reinterpret_cast<const int *>(pq + BN * 8), a.q_zp);
+      const uint32_t base = quad_int8_base<kOut == kOutInt8Bytes>(oc0, a.gemm_n, lane);
 #pragma unroll
       for (int u = 0; u < 4 / KG; ++u) {
         const int q = group + KG * u;
@@ -390,7 +391,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
         if constexpr (kByte) {
           const auto yr = make_rsrc(a.q_y + size_t(out_m) * size_t(a.gemm_n),
                                     uint32_t(rows) * uint32_t(a.gemm_n));
-          store_quad_int8<kOut == kOutInt8Bytes>(v, r, a.q_zp, yr, rows, px0 + 8 * q, oc0, a.gemm_n, lane);
+          if (__builtin_expect(r.odd, 1))
+            store_quad_int8<kOut == kOutInt8Bytes, true>(v, r, a.q_zp, yr, base, wm * TM + 8 * q,
+                                                         a.gemm_n, lane);
+          else
+            store_quad_int8<kOut == kOutInt8Bytes, false>(v, r, a.q_zp, yr, base, wm * TM + 8 * q,
+                                                          a.gemm_n, lane);
         } else {
           const auto yr = make_rsrc(a.y + size_t(out_m) * size_t(a.gemm_n),
                                     uint32_t(rows) * uint32_t(a.gemm_n) * 4u);
@@ -432,10 +438,11 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
         const int8_t *const pq = pr + (wn * TN + 32 * i + (lane & 31)) * 4;
         const Requant32 r = requant32_params(*reinterpret_cast<const int *>(pq + BN * 4),
                                              *reinterpret_cast<const int *>(pq + BN * 8), a.q_zp);
+        const uint32_t base = quad_int8_base<kOut == kOutInt8Bytes>(oc0 + 32 * i, a.gemm_n, lane);
 #pragma unroll
         for (int j = 0; j < FM; ++j)
-          store_block32_int8<kOut == kOutInt8Bytes>(acc[i][j], r, a.q_zp, yr, rows, px0 + 32 * j,
-                                                    oc0 + 32 * i, a.gemm_n, lane);
+          requant_block32<kOut == kOutInt8Bytes>(acc[i][j], r, a.q_zp, yr, base, px0 + 32 * j,
+                                                 a.gemm_n, lane);
       }
     }
     if (!again) return;

@@ -30,7 +30,8 @@
 //     output but 17 % slower with int8, whose requantization then runs on
 //     half the waves).  128 x 128: four MFMA waves of 64 x 64 and four copy
 //     waves (32 x 14x14, 512 -> 512: 20.5 us; eight MFMA waves of 64 x 32,
-//     which read half as much again from LDS, 21.5);
+//     which read half as much again from LDS, 21.5), with int8 output eight,
+//     which share the requantization (launch_gemm_dma);
 //   * an MFMA wave reads the fragments of the next k-step between the MFMAs of
 //     the current one, across the stage barrier too.  Against the 16 x 16 x
 //     64 form that read a stage's fragments and then ran its MFMAs (us per
@@ -348,12 +349,12 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
       const Requant32 r =
           requant32_params(int32_t(__builtin_amdgcn_raw_buffer_load_b32(mr, off, 0, 0)),
                            int32_t(__builtin_amdgcn_raw_buffer_load_b32(sr, off, 0, 0)), a.q_zp);
+      const uint32_t base = quad_int8_base<false>(oc0 + 32 * i, a.gemm_n, lane);
 #pragma unroll
       for (int j = 0; j < FM; ++j) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][j][e] = int(uint32_t(acc[i][j][e]) + bias);
-        store_block32_int8(acc[i][j], r, a.q_zp, yr, rows, px0 + 32 * j, oc0 + 32 * i, a.gemm_n,
-                           lane);
+        requant_block32<false>(acc[i][j], r, a.q_zp, yr, base, px0 + 32 * j, a.gemm_n, lane);
       }
     }
     return;
@@ -387,14 +388,16 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
     store_tile32<0>(acc, yr, rows, px0, oc0, a.gemm_n, lane);
 }
 
-template <int BM, int BN, int WM, int WN, int NCW = 0>
+template <int BM, int BN, int WM, int WN, int NCW = 0, bool kSplits = true>
 int launch_tile(const ConvArgs &a, int splits, hipStream_t stream) {
   const int tiles = int(((int64_t(a.gemm_m) + a.m_step - 1) / a.m_step) * ((a.gemm_n + BN - 1) / BN));
   const int stages = a.gemm_k / kStageBytes;
   const int ring = std::min(kRing, splits > 1 ? a.stages_per_split : stages);
   const size_t lds = size_t(ring) * size_t(BM + BN) * kStageBytes;
-  auto kern = splits > 1 ? gemm_dma_kernel<BM, BN, WM, WN, true, NCW>
-                         : gemm_dma_kernel<BM, BN, WM, WN, false, NCW>;
+  auto kern = gemm_dma_kernel<BM, BN, WM, WN, false, NCW>;
+  if constexpr (kSplits) {
+    if (splits > 1) kern = gemm_dma_kernel<BM, BN, WM, WN, true, NCW>;
+  }
   static LdsLimit limits[2];
   if (const int rc = limits[splits > 1].raise(kern, lds); rc != I8CONV_OK) return rc;
   I8_LAUNCH(kern, dim3(unsigned(tiles), unsigned(splits)), dim3(64 * (WM * WN + NCW)),
@@ -449,7 +452,12 @@ int launch_gemm_dma(const ConvArgs &args, const GemmPlan &p, int splits, void *s
   switch (p.bm * 1000 + p.bn) {
     case 128064: return launch_tile<128, 64, 2, 2>(a, splits, s);
     case 128128:
-      return spec ? launch_tile<128, 128, 2, 2, 4>(a, splits, s) : launch_tile<128, 128, 2, 4>(a, splits, s);
+      if (!spec) return launch_tile<128, 128, 2, 4>(a, splits, s);
+      // int8: eight MFMA waves of 64 x 32, which share the requantization (7 x
+      // 11x14, 512 -> 128 1x1: 6.5 us with four, 6.1 with eight; 4 x 79x79, 256
+      // -> 80 1x3, exact multipliers: 8.3 and 7.9)
+      if (a.q_y) return launch_tile<128, 128, 2, 4, 4, false>(a, splits, s);
+      return launch_tile<128, 128, 2, 2, 4>(a, splits, s);
     case 256064: return launch_tile<256, 64, 4, 2>(a, splits, s);
     case 256128: return launch_tile<256, 128, 4, 2, 8>(a, splits, s);
   }

@@ -79,49 +79,76 @@ __device__ __forceinline__ Requant32 requant32_params(int32_t mult, int32_t shif
   return r;
 }
 
-// Four pixels px .. px + 3 of a lane's channel (a block's elements 4 g ..)
-// requantized to int8.  Where n % 4 == 0 and the window is 4-byte aligned the
-// lane packs their bytes, and the quad's transpose turns them into one pixel's
-// four channels per lane, a 4-byte store; a pixel's 32 channels go out as one
-// 32-byte piece.  kBytes (any n, any alignment): the same pieces, a byte per
-// lane and store.
+// Four pixels of a lane's channel (a block's elements 4 g ..) requantized to
+// int8, the first of them pixel px of the window.  Where n % 4 == 0 and the
+// window is 4-byte aligned the lane packs their bytes, and the quad's
+// transpose turns them into one pixel's four channels per lane, a 4-byte
+// store; a pixel's 32 channels go out as one 32-byte piece.  kBytes (any n,
+// any alignment): the same pieces, a byte per lane and store.
+//
+// `base` is the byte of the lane's first store at px == 0 (quad_int8_base),
+// out of range for channels past n; pixels past the window's last row fall out
+// of its bounds by themselves, so a store costs one add instead of a
+// multiplication and two compares.
 template <bool kBytes>
+__device__ __forceinline__ uint32_t quad_int8_base(int oc0, int n, int lane) {
+  const int px = 4 * (lane >> 5) + (kBytes ? 0 : lane & 3);
+  const int oc = oc0 + (lane & (kBytes ? 31 : 28));
+  return oc < n ? uint32_t(px) * uint32_t(n) + uint32_t(oc) : kOutOfRange;
+}
+template <bool kBytes, bool kOdd>
 __device__ __forceinline__ void store_quad_int8(v4i acc, const Requant32 &r, int32_t zp,
-                                                __amdgpu_buffer_rsrc_t out, int rows, int px,
-                                                int oc0, int n, int lane) {
+                                                __amdgpu_buffer_rsrc_t out, uint32_t base, int px,
+                                                int n, int lane) {
   uint32_t y[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
-    y[e] = uint32_t(r.odd ? requant1_odd(acc[e], r.o.mo, r.o.k, r.o.sh)
-                          : requant1(acc[e], r.mult, r.shift, zp));
+  for (int e = 0; e < 4; ++e) {
+    y[e] = uint32_t(kOdd ? requant1_odd(acc[e], r.o.mo, r.o.k, r.o.sh)
+                         : requant1(acc[e], r.mult, r.shift, zp));
+  }
+  const uint32_t off = base + uint32_t(px) * uint32_t(n);
   if constexpr (kBytes) {
-    const int oc = oc0 + (lane & 31);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      __builtin_amdgcn_raw_buffer_store_b8(
-          uint8_t(y[e]), out,
-          px + e < rows && oc < n ? uint32_t(px + e) * uint32_t(n) + uint32_t(oc) : kOutOfRange, 0,
-          0);
+      __builtin_amdgcn_raw_buffer_store_b8(uint8_t(y[e]), out, off + uint32_t(e) * uint32_t(n), 0, 0);
     return;
   }
   const uint32_t lo = __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0400u);
   const uint32_t hi = __builtin_amdgcn_perm(y[3], y[2], 0x0c0c0400u);
   const uint32_t v = quad_transpose(__builtin_amdgcn_perm(hi, lo, 0x05040100u), lane);
-  const int p = px + (lane & 3), oc = oc0 + (lane & 28);
-  __builtin_amdgcn_raw_buffer_store_b32(
-      v, out, p < rows && oc < n ? uint32_t(p) * uint32_t(n) + uint32_t(oc) : kOutOfRange, 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b32(v, out, off, 0, 0);
 }
 
-// One 32 x 32 block of a wave requantized to int8.
-template <bool kBytes = false>
+// One 32 x 32 block of a wave requantized to int8, px0 its first pixel.
+template <bool kBytes, bool kOdd>
 __device__ __forceinline__ void store_block32_int8(const v16i &acc, const Requant32 &r, int32_t zp,
-                                                   __amdgpu_buffer_rsrc_t out, int rows, int px0,
-                                                   int oc0, int n, int lane) {
+                                                   __amdgpu_buffer_rsrc_t out, uint32_t base,
+                                                   int px0, int n, int lane) {
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const v4i v = {acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
-    store_quad_int8<kBytes>(v, r, zp, out, rows, px0 + 4 * (lane >> 5) + 8 * g, oc0, n, lane);
+    store_quad_int8<kBytes, kOdd>(v, r, zp, out, base, px0 + 8 * g, n, lane);
   }
+}
+
+// The odd-multiplier form and the exact one apart, chosen once per block: the
+// first is then short straight-line code and the exact form's 64-bit products
+// lie out of its way.  With both in the code of every four values, fetching
+// that code, once per launch, took a microsecond (us per launch of the
+// pipelined GEMM: its 16 x 16 MFMA form, this one with both together, apart;
+// 4 x 79x79, 256 -> 96 1x3: 7.8, 8.7, 6.7; 7 x 11x14, 512 -> 128 1x1: 6.9, 8.7,
+// 6.1; 4 x 52x52, 256 -> 72: 5.5, 6.3, 5.2; exact form, 16 x 28x28, 512 -> 384:
+// 14.6, 20.4, 12.7).  Chosen for a wave's blocks of 32 channels together the
+// exact form spills where four waves share a SIMD (256 x 128 tile, 8 x 64x64,
+// 256 -> 256: 25.3, 28.3 so).
+template <bool kBytes>
+__device__ __forceinline__ void requant_block32(const v16i &acc, const Requant32 &r, int32_t zp,
+                                                __amdgpu_buffer_rsrc_t out, uint32_t base, int px0,
+                                                int n, int lane) {
+  if (__builtin_expect(r.odd, 1))
+    store_block32_int8<kBytes, true>(acc, r, zp, out, base, px0, n, lane);
+  else
+    store_block32_int8<kBytes, false>(acc, r, zp, out, base, px0, n, lane);
 }
 
 #endif  // __HIPCC__

@@ -138,3 +138,51 @@ def test_gemm32_int8_byte_stores(name, off):
             buf.close()
     assert (raw[:off] == 0x5A).all() and (raw[off + count:] == 0x5A).all()
     np.testing.assert_array_equal(raw[off:off + count].reshape(shape.output_shape), expected)
+
+
+PIPELINED = {
+    # the pipelined kernel's requantizing epilogue on each of its tiles: with
+    # and without copy waves, channel tails inside a 32-channel block and past
+    # one, pixel tails, tiles that store fewer rows than they have
+    "128x128_k100": ("128px x 128oc, grid 74x1, 18 k-stages, 4 copy waves",
+                     lab.ConvShape(2, 71, 66, 256, 100, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "128x128_k384_rows": ("128px x 128oc (96px stored), grid 149x3, 4 k-stages, 4 copy waves",
+                          lab.ConvShape(1, 121, 118, 512, 384, 1, 1, 0, 0, 1, 1, 1, 1)),
+    "128x128_two_stages": ("128px x 128oc, grid 74x2, 2 k-stages",
+                           lab.ConvShape(2, 71, 66, 256, 132, 1, 1, 0, 0, 1, 1, 1, 1)),
+    "128x64_k60": ("128px x 64oc, grid 74x1, 3 k-stages",
+                   lab.ConvShape(2, 71, 66, 128, 60, 1, 3, 0, 1, 1, 1, 1, 1)),
+    "256x64_k36": ("256px x 64oc, grid 193x1, 5 k-stages",
+                   lab.ConvShape(1, 222, 222, 128, 36, 5, 1, 2, 0, 1, 1, 1, 1)),
+    "256x128_k76": ("256px x 128oc, grid 193x1, 5 k-stages, 8 copy waves",
+                    lab.ConvShape(1, 222, 222, 128, 76, 5, 1, 2, 0, 1, 1, 1, 1)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(PIPELINED))
+def test_pipelined_kernel_runs_these_layers(name):
+    tile, shape = PIPELINED[name]
+    assert f"pipelined tile {tile}" in lab.describe("generic", shape)
+    assert lab.dispatch(shape) == "generic"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(PIPELINED))
+def test_pipelined_requant_bit_exact(name):
+    _, shape = PIPELINED[name]
+    x, w, b = lab.make_case_data(shape, seed=51)
+    acc = oracle.conv(shape, x, w, b)
+    rng = np.random.default_rng(52)
+    odd = ((rng.integers(2 ** 29, 2 ** 30, size=shape.k) * 2 + 1).astype(np.int32),
+           rng.integers(44, 47, size=shape.k).astype(np.int32))
+    # shifts below 33: no channel in the odd-multiplier form's domain
+    exact = (rng.integers(100, 200, size=shape.k).astype(np.int32),
+             np.full(shape.k, 22, np.int32))
+    mixed = (odd[0].copy(), odd[1].copy())
+    mixed[0][shape.k - 1], mixed[1][shape.k - 1] = exact[0][0], exact[1][0]
+    for form, (mult, shift) in (("odd", odd), ("exact", exact), ("mixed", mixed)):
+        say(f"[gpu] pipelined requant {name} {form}")
+        got = lab.conv2d_requant(x, w, b, mult, shift, 11, shape)
+        exp = oracle.requantize(acc, mult, shift, 11)
+        assert len(np.unique(exp)) > 50
+        np.testing.assert_array_equal(got, exp, err_msg=form)
