@@ -242,8 +242,22 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
 //     from 512 tiles on (64 x 28x28, 384 -> 192 1x1: 19.0 -> 12.3; 53 x 62x62,
 //     512 -> 288: 103 -> 94; two stages, 32 x 56x56, 256 -> 160: 24.7, 25.4);
 //   * at least two rounds of 256 x 256 tiles: a third fewer copied bytes per
-//     operation (16 x 256x256, 256 -> 256 3x3: 780 -> 706; 5x5 stride 2 with
-//     int8 output: 484 -> 457).
+//     operation (16 x 256x256, 256 -> 256 3x3: 718 -> 614; 5x5 stride 2 with
+//     int8 output: 411 -> 376).  Not where they compute more than 8/7 of the
+//     channel columns that 128-wide tiles do (128-wide, 256-wide: 4 x 128x140
+//     dilated, 256 -> 288: 71, 95, int8 67, 90; 8 x 128x128, 128 -> 260: 74,
+//     85; 512x128, 256 -> 640: 104, 109; 256 -> 1152: 181, 177), nor, from 16
+//     stages on, where more than an eighth of the rounds would be empty
+//     (520x128, 512 -> 512, 520 tiles: 166, 186; 850x128, 256 -> 512, 850
+//     tiles: 140, 145; with nine stages int8 gains what int32 loses: 1200x128,
+//     128 -> 256, 600 tiles: 78.6, 69.5 and 67.7, 71.1).
+static bool wide_tiles(const i8conv_geometry &g, int stages) {
+  const int64_t tiles_n = ceil_div(g.gemm_n, 256), narrow_n = ceil_div(g.gemm_n, 128);
+  const int64_t tiles = ceil_div(g.gemm_m, 256) * tiles_n, rounds = ceil_div(tiles, 256);
+  return stages >= 8 && tiles >= 512 && 7 * 2 * tiles_n <= 8 * narrow_n &&
+         (stages < 16 || 8 * tiles >= 7 * 256 * rounds);
+}
+
 GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
   GemmPlan p = plan_staged(s, g);
   if (pointwise_eligible(s, g)) {
@@ -255,7 +269,7 @@ GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
   auto tiles = [&](int bm, int bn) { return ceil_div(g.gemm_m, bm) * ceil_div(g.gemm_n, bn); };
   if (!p.dma)
     gemm32_tile(g, p);
-  else if (g.gemm_n > 128 && p.stages >= 8 && tiles(256, 256) >= 512)
+  else if (wide_tiles(g, p.stages))
     set_gemm32(g, p, 256, 256);
   else if (p.stages >= 3 && p.stages <= 4 && g.gemm_n % 128 != 0 && tiles(128, 64) >= 512)
     set_gemm32(g, p, 128, 64);

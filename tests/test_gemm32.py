@@ -53,6 +53,22 @@ def test_gemm32_runs_these_layers(name):
     assert f"32x32 MFMA tile {tile}" in lab.describe("generic", shape)
 
 
+@pytest.mark.parametrize("n,hw,c,k,r,wide", [
+    # 256-wide tiles where they compute at most 8/7 of the columns that 128-wide
+    # ones do
+    (1, 512, 128, 129, 3, True), (1, 512, 128, 256, 3, True), (1, 512, 128, 385, 3, True),
+    (1, 512, 128, 257, 3, False), (1, 512, 128, 384, 3, False), (1, 512, 128, 128, 3, False),
+    (1, 512, 128, 640, 3, False), (1, 512, 128, 896, 3, True),
+    # rounds of 256: 1024 tiles are four; 520 leave most of a third empty,
+    # which only short reductions make up for
+    (1, 512, 256, 256, 3, True), (1, 364, 256, 256, 3, False), (1, 364, 128, 256, 3, True),
+    # 960 tiles: 15/16 of four rounds
+    (15, 128, 256, 256, 3, True)])
+def test_256_wide_tiles_where_they_pay(n, hw, c, k, r, wide):
+    shape = lab.ConvShape(n, hw, hw, c, k, r, r, r // 2, r // 2, 1, 1, 1, 1)
+    assert ("256px x 256oc" in lab.describe("generic", shape)) == wide
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_gemm32_bit_exact(name):
