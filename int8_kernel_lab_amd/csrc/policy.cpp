@@ -13,19 +13,26 @@
 //      batch 1: it won all of them; at 24 tiles and 18 stages the generic
 //      GEMM won, 15.0 vs 15.7 us, and on a 32x32 3x3 layer of 9 stages the
 //      halo kernel, 9.3 vs 11.0 us);
-//   3. the generic GEMM wherever it runs its pipelined form (C % 128 == 0) or
-//      the 32 x 32 x 32 MFMA one: they beat every halo and strip plan without
-//      row streaming (C % 128 == 0: 3 x 44x44, 512 -> 160 3x1: 25.6 -> 8.3;
-//      36x36, 512 -> 256 3x3: 45.9 -> 16.1; 2 x 40x40 dilated 256 -> 192: 27.7
+//   3. the resident-rows form of the halo kernel where each of its workgroups
+//      has one fragment of 16 pixels, a filter slice of at most 72 KB and at
+//      most 28 KB of input rows: the generic kernel's smallest grids are slower
+//      there, by less the more input a workgroup copies first (3 x 9x9, 192 ->
+//      96 1x3, 9 KB: 4.5 against 5.0 us; 2 x 24x24, 192 -> 160 1x3, 13 KB: 4.7,
+//      5.1; 1 x 15x15, 128 -> 64 dilated 2, 19 KB: 5.4, 5.6; level at 25 to 30 KB;
+//      1 x 38x38, 192 -> 128 3x1, 32 KB: 5.3, 5.1);
+//   4. the generic GEMM wherever it runs its pipelined form (C % 128 == 0) or
+//      the 32 x 32 x 32 MFMA one: they beat every other halo and strip plan
+//      without row streaming (C % 128 == 0: 3 x 44x44, 512 -> 160 3x1: 25.6 ->
+//      8.3; 36x36, 512 -> 256 3x3: 45.9 -> 16.1; 2 x 40x40 dilated 256 -> 192: 27.7
 //      -> 10.0; 4 x 60x30, 128 -> 64 1x3: 7.9 -> 4.5; others: 1x3, 64 -> 128:
 //      22.3 -> 14.2; 256x256, 64 -> 63, 69, 255: 16.4, 19.2, 43 -> 9.3, 11.1,
 //      21; dilated 64 -> 128: 6.3 -> 5.3);
-//   4. otherwise an input-reuse kernel for a stride-1 spatial filter
+//   5. otherwise an input-reuse kernel for a stride-1 spatial filter
 //      (r*s > 1): halo when eligible, else strip (small dilated layers,
 //      asymmetric 1x3/3x1, C = 64 layers wider than the row kernel's four
 //      fragments); at stride 2 the generic GEMM beat the halo kernel on
 //      every such layer (15.0 vs 18.0 us at 52x52, C = 256);
-//   5. otherwise the generic implicit GEMM (1x1 layers, strided layers,
+//   6. otherwise the generic implicit GEMM (1x1 layers, strided layers,
 //      C % 64 != 0).
 #include <cstring>
 #include <mutex>
@@ -94,6 +101,11 @@ Choice dispatch_uncached(const i8conv_shape &s) {
   if (tiles <= 16 && (gp.stages >= 16 || (!spatial && gp.stages >= 8)))
     return {I8CONV_KERNEL_SPLITK, false};
   const bool reuse = spatial && s.stride_h == 1 && s.stride_w == 1;
+  if (halo && reuse && pp.resident && pp.frags_m == 1 &&
+      int64_t(pp.bn) * g.gemm_k <= 72 * 1024 &&
+      pp.rows * halo_row_layout(int64_t(s.w) + 2 * s.pad_w, s.c, kHaloPadUnits).row_bytes <=
+          28 * 1024)
+    return {I8CONV_KERNEL_HALO, false};
   const bool patch = reuse && gp.dma && tiles < 128 && (halo || plan_strip(s, g, &pp));
   if (gp.m32 || gp.dma) return {I8CONV_KERNEL_GENERIC, patch};
   if (reuse) {

@@ -168,6 +168,20 @@ def test_baseline_eligibility_and_dispatch(name, baseline_cases):
     assert lab.dispatch(shape) == chosen
 
 
+@pytest.mark.parametrize("fields,chosen", [
+    # one 16-pixel fragment per workgroup and few input rows: resident rows
+    ((3, 9, 9, 192, 96, 1, 3, 0, 1, 1, 1, 1, 1), "halo"),
+    ((2, 24, 24, 192, 160, 1, 3, 0, 1, 1, 1, 1, 1), "halo"),
+    ((2, 18, 18, 64, 128, 3, 3, 2, 2, 1, 1, 2, 2), "halo"),
+    ((1, 15, 15, 128, 64, 3, 3, 2, 2, 1, 1, 2, 2), "halo"),
+    # 32 KB of them; a filter slice of 144 KB; two fragments per workgroup
+    ((1, 38, 38, 192, 128, 3, 1, 1, 0, 1, 1, 1, 1), "generic"),
+    ((1, 15, 15, 128, 96, 3, 3, 2, 2, 1, 1, 2, 2), "generic"),
+    ((1, 56, 56, 192, 256, 1, 3, 0, 1, 1, 1, 1, 1), "generic")])
+def test_small_resident_row_grids_keep_the_halo_kernel(fields, chosen):
+    assert lab.dispatch(lab.ConvShape(*fields)) == chosen
+
+
 @pytest.mark.parametrize("name,shape", sorted(all_shapes().items()), ids=lambda v: str(v))
 def test_dispatch_returns_an_eligible_kernel_with_its_workspace(name, shape):
     chosen = lab.dispatch(shape)
