@@ -203,7 +203,8 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
     set_gemm32(g, p, 128, 128);
   else if (tiles(128, 64) >= 512)
     set_gemm32(g, p, 128, g.gemm_n <= 32 ? 32 : 64);
-  else if (g.gemm_n > 64 || p.stages >= 6 || tiles(64, 64) > 256)
+  else if (g.gemm_n > 64 || p.stages >= 6 ||
+           (tiles(64, 64) > 256 && (g.gemm_n > 32 || p.stages > 3)))
     set_gemm32(g, p, 64, 64);
 }
 
@@ -231,16 +232,20 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
 //     four are slower than two, 11.4);
 //   * the register-staged kernel keeps layers of at most 64 channels, fewer
 //     than six stages and one round of 64-pixel tiles (2 x 30x30, 48 -> 64
-//     3x3: 5.5 against 6.0).
+//     3x3: 5.5 against 6.0), and those of at most 32 channels and three stages
+//     that are too small for 128 x 32: half of a 64 x 64 tile is then dead
+//     (200x200, 32 -> 32 1x1: 4.4, 5.2; 248x248, 32 -> 32 3x3: 6.3, 6.9; five
+//     stages, 352x352, 64 -> 32 3x3 stride 2: 6.9, 6.2).
 // C % 128 == 0: the pipelined kernel, except
 //   * at most 128 tiles of 64 x 64, six to 18 stages: 64 x 64 (52x52, 256 ->
 //     512 3x3 stride 2: 10.0 -> 7.3 with two groups; 2 x 64x64, 128 -> 64: 7.0
 //     -> 5.9).  More tiles or stages stay (2 x 40x40, 256 -> 192, 150 tiles:
 //     10.0 against 12.1; 36x36, 512 -> 256, 36 stages: 16.1 against 18.4), but
 //     for grids so small that the policy splits their reduction;
-//   * three or four stages and a last channel tile that is not whole: 128 x 64
+//   * three or four stages and N no multiple of 128, up to 64 too: 128 x 64
 //     from 512 tiles on (64 x 28x28, 384 -> 192 1x1: 19.0 -> 12.3; 53 x 62x62,
-//     512 -> 288: 103 -> 94; two stages, 32 x 56x56, 256 -> 160: 24.7, 25.4);
+//     512 -> 288: 103 -> 94; 30 x 60x60, 384 -> 64: 14.6 -> 12.5; 20 x 60x60,
+//     128 -> 64 1x3: 10.8 -> 8.1; two stages, 32 x 56x56, 256 -> 160: 24.7, 25.4);
 //   * at least two rounds of 256 x 256 tiles: a third fewer copied bytes per
 //     operation (16 x 256x256, 256 -> 256 3x3: 718 -> 614; 5x5 stride 2 with
 //     int8 output: 411 -> 376).  Not where they compute more than 8/7 of the
