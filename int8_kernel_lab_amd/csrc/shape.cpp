@@ -201,7 +201,7 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
     set_gemm32(g, p, 64, 64);
   else if (g.gemm_n > 64 && tiles(128, 128) >= 256)
     set_gemm32(g, p, 128, 128);
-  else if (tiles(128, 64) >= 512)
+  else if (tiles(128, 64) >= (g.gemm_n <= 32 ? 256 : 512))
     set_gemm32(g, p, 128, g.gemm_n <= 32 ? 32 : 64);
   else if (g.gemm_n > 64 || p.stages >= 6 ||
            (tiles(64, 64) > 256 && (g.gemm_n > 32 || p.stages > 3)))
@@ -221,7 +221,10 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
 //   * 128 x 64, three per unit, with at least 512 tiles (16 x 224x224, 32 ->
 //     64 7x7 stride 2: 101 -> 35; 256x256, 64 -> 63: 16.4 -> 9.3), 128 x 32
 //     for at most 32 channels (30 x 97x108, 32 -> 32 7x7 stride 2: 128 x 64
-//     18.0 -> 15.6; 16 x 56x56, 96 -> 32: 8.0 -> 7.3);
+//     18.0 -> 15.6; 16 x 56x56, 96 -> 32: 8.0 -> 7.3), from 256 tiles on: half
+//     of a 64 x 64 tile would be dead (register-staged, 64 x 64, 128 x 32:
+//     248x248, 160 -> 32 3x3: 13.8, 14.4, 10.4; 223x223, 48 -> 32 3x3: 6.9,
+//     7.4, 5.9; 184x184, 48 -> 32: 6.2, 6.4, 5.6);
 //   * 64 x 64, four per unit, below that (416x416, 32 -> 64 3x3 stride 2: 7.3
 //     -> 5.9, 128 x 64: 7.6).  With at most two tiles per unit a stage's
 //     latency counts, not its throughput: then groups of waves share a tile's
@@ -233,9 +236,9 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
 //   * the register-staged kernel keeps layers of at most 64 channels, fewer
 //     than six stages and one round of 64-pixel tiles (2 x 30x30, 48 -> 64
 //     3x3: 5.5 against 6.0), and those of at most 32 channels and three stages
-//     that are too small for 128 x 32: half of a 64 x 64 tile is then dead
-//     (200x200, 32 -> 32 1x1: 4.4, 5.2; 248x248, 32 -> 32 3x3: 6.3, 6.9; five
-//     stages, 352x352, 64 -> 32 3x3 stride 2: 6.9, 6.2).
+//     that are too small for 128 x 32 (130x130, 32 -> 32 1x1: 3.8, 4.1; 176x176,
+//     32 -> 32 3x3: 5.1, 5.3; five stages, 352x352, 64 -> 32 3x3 stride 2: 6.9,
+//     6.2).
 // C % 128 == 0: the pipelined kernel, except
 //   * at most 128 tiles of 64 x 64, six to 18 stages: 64 x 64 (52x52, 256 ->
 //     512 3x3 stride 2: 10.0 -> 7.3 with two groups; 2 x 64x64, 128 -> 64: 7.0

@@ -70,12 +70,12 @@ def test_256_wide_tiles_where_they_pay(n, hw, c, k, r, wide):
 
 
 @pytest.mark.parametrize("hw,c,k,r,tile", [
-    # at most 32 channels and three stages: register-staged up to where 128 x 32
-    # tiles take over; more channels or stages: 64 x 64
-    (200, 32, 32, 1, "register-staged"), (248, 32, 32, 3, "register-staged"),
-    (200, 32, 33, 1, "32x32 MFMA tile 64px x 64oc"), (248, 48, 32, 3, "32x32 MFMA tile 64px x 64oc"),
-    (260, 32, 32, 3, "32x32 MFMA tile 128px x 32oc"),
-    (120, 32, 64, 1, "register-staged")])
+    # at most 32 channels: 128 x 32 from 256 tiles on, below that
+    # register-staged up to three stages; more channels or stages: 64 x 64
+    (181, 32, 32, 1, "32x32 MFMA tile 128px x 32oc"), (181, 160, 32, 3, "32x32 MFMA tile 128px x 32oc"),
+    (180, 32, 32, 1, "register-staged"), (180, 32, 32, 3, "register-staged"),
+    (180, 48, 32, 3, "32x32 MFMA tile 64px x 64oc"), (180, 32, 33, 1, "32x32 MFMA tile 64px x 64oc"),
+    (181, 32, 33, 1, "32x32 MFMA tile 64px x 64oc"), (120, 32, 64, 1, "register-staged")])
 def test_narrow_short_layers(hw, c, k, r, tile):
     shape = lab.ConvShape(1, hw, hw, c, k, r, r, r // 2, r // 2, 1, 1, 1, 1)
     assert tile in lab.describe("generic", shape)
