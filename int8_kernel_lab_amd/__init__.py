@@ -48,8 +48,14 @@ SHAPE_FIELDS = ("n", "h", "w", "c", "k", "r", "s", "pad_h", "pad_w",
                 "stride_h", "stride_w", "dilation_h", "dilation_w")
 
 
+class _CRefSlot:
+    """Holds ConvShape's C struct beside its __dict__, which stays its fields'."""
+
+    __slots__ = ("_ref",)
+
+
 @dataclass(frozen=True)
-class ConvShape:
+class ConvShape(_CRefSlot):
     """Convolution geometry; the 13 ConvShape template parameters."""
 
     n: int
@@ -73,14 +79,14 @@ class ConvShape:
         """byref() of a C struct of this (immutable) shape, built once: a
         launch then spends 0.1 us of host time on it instead of 1.9.  Read
         only; c_struct() is the one to hand out."""
-        ref = self.__dict__.get("_ref")
+        ref = getattr(self, "_ref", None)
         if ref is None:
             ref = ctypes.byref(self.c_struct())
             object.__setattr__(self, "_ref", ref)
         return ref
 
-    def __getstate__(self):
-        return {f: getattr(self, f) for f in SHAPE_FIELDS}
+    def __getstate__(self):  # not the C struct: it points into this process
+        return self.__dict__
 
     def geometry(self) -> _lib.CGeometry:
         """Derived sizes; ValueError where the reference's static_asserts

@@ -3,8 +3,11 @@ division, the workload-table readers, the C++ driver's command line and the
 sweep script's argument handling.  No GPU is touched: every driver run below
 exits on an argument or table error before its first HIP call.
 """
+import copy
 import ctypes
+import dataclasses
 import os
+import pickle
 import subprocess
 import sys
 
@@ -49,6 +52,27 @@ def test_generator_order_and_ranges():
     xr, _, br = lab.make_case_data(shape, seed=99, value_range=(-4, 4), bias_range=(-31, 31))
     assert xr.min() >= -4 and xr.max() <= 4 and br.min() >= -31 and br.max() <= 31
     assert set(np.unique(xr).tolist()) == set(range(-4, 5))
+
+
+# ---- shapes -------------------------------------------------------------------
+
+@dataclasses.dataclass(frozen=True)
+class NamedShape(lab.ConvShape):
+    name: str = ""
+
+
+def test_a_shape_stays_its_fields_after_a_launch():
+    for shape in (lab.ConvShape(1, 8, 8, 16, 8, 3, 3, 1, 1),
+                  NamedShape(1, 8, 8, 16, 8, 3, 3, 1, 1, name="stem")):
+        fields = dict(vars(shape))
+        with pytest.raises(lab.I8ConvError):  # refused before any GPU call
+            lab.launch("generic", shape, None, None, None, None)
+        assert vars(shape) == fields
+        assert type(shape)(**vars(shape)) == shape
+        for other in (pickle.loads(pickle.dumps(shape)), copy.copy(shape), copy.deepcopy(shape)):
+            assert other == shape and vars(other) == fields
+            assert other._c_ref() is not shape._c_ref()
+            assert other.geometry().gemm_k == shape.geometry().gemm_k
 
 
 # ---- exact division used by every kernel's index math -------------------------
