@@ -172,23 +172,27 @@ int i8conv_launch_noalloc(int id, const i8conv_shape *shape, const int8_t *input
 int i8conv_requantize(const int32_t *acc, int64_t pixels, int32_t channels,
                       const int32_t *mult, const int32_t *shift,
                       int32_t zero_point, int8_t *output, void *stream);
-/* 1 when an int8 launch of `shape` needs no int32 workspace, 0 when it asks
- * for one (the kernels that have a requantizing epilogue all the same leave it
- * alone, the others write int32 there and a requantizing pass follows).
- * Fused: the row kernel with copy waves; the generic kernel's pointwise streaming form (1x1 stride-1
- * unpadded layers with output-channel slices of 64 or 128), when bias,
- * mult, shift and output are 16-byte aligned; split-K's second pass (N % 4
- * == 0), when bias, mult and shift are 16-byte aligned; the pipelined GEMM's
- * epilogue (N % 4 == 0), when mult and shift are 16-byte aligned.  With
- * other pointers the launch takes the unfused way, whose workspace is the
- * int32 output plus the kernel's own. */
+/* Whether i8conv_launch_requant runs `shape` without an int32 workspace.
+ * 1: the row kernel with copy waves; the generic kernel's pointwise streaming
+ * form (1x1 stride-1 unpadded layers with output-channel slices of 64 or 128),
+ * when bias, mult, shift and output are 16-byte aligned; split-K's second pass
+ * (N % 4 == 0), when bias, mult and shift are 16-byte aligned; the generic
+ * GEMM where C % 128 == 0 and N % 4 == 0 (but for small grids of stride-1
+ * spatial filters), when mult and shift are 16-byte aligned.  With other
+ * pointers such a launch asks for the workspace too.
+ * 0: the launch asks for an int32 workspace of the whole output and is refused
+ * without it.  Most of these kernels requantize in their epilogue all the same
+ * and leave it alone; the convolution is written there, and a requantizing
+ * pass follows, for split-K with N % 4 != 0 or unaligned pointers, for an
+ * output that overlaps the input, filter or bias, and beyond the sizes of the
+ * 32 x 32 MFMA kernel (2^20 output channels, 2^30 pixels).
+ * Where this is 1 the output must not overlap the other tensors. */
 int i8conv_requant_fused(const i8conv_shape *shape);
-/* Workspace i8conv_launch_requant needs: the dispatched kernel's own (split-K's
- * partial sums; nothing for the other kernels), plus the int32 output
- * (256-byte aligned) when the requantization is not fused. */
+/* Workspace i8conv_launch_requant asks for: the dispatched kernel's own
+ * (split-K's partial sums; nothing for the other kernels), plus the int32
+ * output (256-byte aligned) where i8conv_requant_fused is 0. */
 size_t i8conv_requant_workspace_bytes(const i8conv_shape *shape);
-/* The dispatched convolution with int8 output: fused epilogue or
- * convolution into the workspace + requantizing pass.  Allocates nothing. */
+/* The dispatched convolution with int8 output, as above.  Allocates nothing. */
 int i8conv_launch_requant(const i8conv_shape *shape, const int8_t *input,
                           const int8_t *filter, const int32_t *bias,
                           const int32_t *mult, const int32_t *shift,

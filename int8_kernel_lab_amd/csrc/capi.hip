@@ -648,6 +648,10 @@ bool requant_route_aligned(RequantRoute r, const int32_t *bias, const int32_t *m
   }
 }
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
+bool overlap(const void *a, int64_t a_bytes, const void *b, int64_t b_bytes) {
+  const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x < y + uintptr_t(b_bytes) && y < x + uintptr_t(a_bytes);
+}
 }  // namespace
 
 int i8conv_requantize(const int32_t *acc, int64_t pixels, int32_t channels,
@@ -750,6 +754,13 @@ int i8conv_launch_requant(const i8conv_shape *shape, const int8_t *input, const 
                    : std::string()));
     return I8CONV_WORKSPACE_TOO_SMALL;
   }
+  // A layer run in place (its int8 output over its input, or over the filter or
+  // bias) goes through the workspace: the convolution then has read all of them
+  // before the pass writes the first byte, where an epilogue would write rows
+  // that other workgroups still read.
+  const bool in_place = overlap(output, g.output_elements, input, g.input_elements) ||
+                        overlap(output, g.output_elements, filter, g.filter_elements) ||
+                        overlap(output, g.output_elements, bias, 4 * int64_t(g.gemm_n));
   // The 32 x 32 x 32 MFMA kernel requantizes in its epilogue and leaves the
   // workspace alone (16 x 224x224, 32 -> 64 7x7 stride 2: 101 us through the
   // int32 workspace and the pass, 35 us; in byte stores where N % 4 != 0: 5 x
@@ -759,7 +770,7 @@ int i8conv_launch_requant(const i8conv_shape *shape, const int8_t *input, const 
   // 22x22 dilated 64 -> 64: 15.7 us a call before, 8.5 now).
   PatchPlan pp;
   const bool row = id == I8CONV_KERNEL_HALO && plan_halo(*shape, g, &pp) && pp.row;
-  if (id != I8CONV_KERNEL_SPLITK && !row) {
+  if (id != I8CONV_KERNEL_SPLITK && !row && !in_place) {
     const bool vec = g.gemm_n % 4 == 0 && requant_route_aligned(kRqGemm, bias, mult, shift, output);
     const GemmPlan own = plan_generic(*shape, g);
     const bool pipelined = own.dma && !own.m32 && !own.pw && vec;
@@ -775,7 +786,7 @@ int i8conv_launch_requant(const i8conv_shape *shape, const int8_t *input, const 
   }
   // The row kernel likewise (32 x 56x56, 64 -> 64: 10.5 + 8.1 us with the
   // pass).
-  if (row && !pp.streamed) {
+  if (row && !pp.streamed && !in_place) {
     const ConvArgs args = make_args(*shape, g, input, filter, bias, nullptr);
     const RequantArgs q{mult, shift, zero_point, output};
     return launch_row(args, pp, stream, &q);

@@ -540,3 +540,38 @@ def test_kernel_requant_function_matches_oracle_on_host(tmp_path):
         assert got[i, 0] == want, (i, acc[i], mult[i], shift[i], zp[i], got[i], want)
         assert got[i, 1] == want, ("short", i, acc[i], mult[i], shift[i], zp[i], got[i], want)
         assert got[i, 2] == want, ("odd", i, acc[i], mult[i], shift[i], zp[i], got[i], want)
+
+
+IN_PLACE = {
+    # layers that ask for the int32 workspace: the row kernel, the 32 x 32 MFMA
+    # kernel (also for N % 4 != 0), the halo and the register-staged kernel
+    "row": lab.ConvShape(4, 30, 28, 64, 64, 3, 3, 1, 1, 1, 1, 1, 1),
+    "gemm32_c96": lab.ConvShape(6, 33, 31, 96, 96, 3, 3, 1, 1, 1, 1, 1, 1),
+    "gemm32_k83": lab.ConvShape(5, 40, 37, 96, 83, 1, 3, 0, 1, 1, 1, 1, 1),
+    "halo": lab.ConvShape(3, 17, 15, 64, 64, 3, 3, 2, 2, 1, 1, 2, 2),
+    "register_staged": lab.ConvShape(2, 30, 30, 48, 48, 3, 3, 1, 1, 1, 1, 1, 1),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(IN_PLACE))
+def test_requant_in_place_bit_exact(name):
+    # the int8 output over the input: the convolution reads all of it first
+    from tests.conftest import say
+    shape = IN_PLACE[name]
+    assert not lab.requant_fused(shape)
+    x, w, b = lab.make_case_data(shape, seed=61)
+    mult, shift = _qparams(shape.k, seed=62)
+    exp = oracle.requantize(oracle.conv(shape, x, w, b), mult, shift, 2)
+    need = lab.requant_workspace_bytes(shape)
+    bufs = [lab.DeviceBuffer.from_array(a) for a in (x, w, b, mult, shift)]
+    ws = lab.DeviceBuffer(need)
+    try:
+        say(f"[gpu] requantized launch in place, {name}")
+        lab.launch_requant(shape, *bufs, 2, bufs[0].ptr, ws, need)
+        lab.synchronize()
+        got = bufs[0].download(np.int8, exp.size).reshape(exp.shape)
+    finally:
+        for buf in bufs + [ws]:
+            buf.close()
+    np.testing.assert_array_equal(got, exp)
