@@ -35,6 +35,7 @@ namespace i8conv {
 constexpr int kThreads = 256;      // 4 wave64 per workgroup
 constexpr int kStageBytes = 128;   // k-bytes per LDS stage of the GEMM kernels
 constexpr int kLdsBudget = 160 * 1024;
+constexpr int kWideChannels = 1 << 20;  // more output channels than these: GemmPlan::wide
 
 void set_error(const std::string &message);
 
@@ -93,6 +94,8 @@ struct GemmPlan {
   // c % 128 == 0: the LDS-DMA pipelined kernel (kernel_gemm_dma.hip), else
   // the register-staged one (kernel_gemm.hip)
   bool dma = false;
+  // ... on 128 x 128 tiles with 64-bit output addresses: N > kWideChannels
+  bool wide = false;
   // generic only: the 32 x 32 x 32 MFMA kernel (kernel_gemm32.hip) runs the
   // layer, on bm x bn tiles; kg groups of waves share a tile's reduction
   bool m32 = false;

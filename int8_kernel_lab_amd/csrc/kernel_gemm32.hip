@@ -492,7 +492,7 @@ int launch_out(const ConvArgs &a, hipStream_t s) {
 bool gemm32_eligible(const i8conv_shape &s, const i8conv_geometry &g) {
   // 32-bit tile, tap and k arithmetic, and a tile's output window below 2 GiB
   return int64_t(s.r) * s.dilation_h <= (1 << 28) && int64_t(s.s) * s.dilation_w <= (1 << 28) &&
-         g.gemm_m <= (1 << 30) && g.gemm_k <= (1 << 30) && g.gemm_n <= (1 << 20) &&
+         g.gemm_m <= (1 << 30) && g.gemm_k <= (1 << 30) && g.gemm_n <= kWideChannels &&
          ((g.gemm_m + 63) / 64) * ((int64_t(g.gemm_n) + 63) / 64) <= INT32_MAX;
 }
 

@@ -78,7 +78,10 @@ __device__ __forceinline__ void with_live_frags(int live, Run &run) {
 // copies, so an MFMA wave never stalls on a copy issue.  The two roles run
 // separate loops with the same one barrier per stage, so neither role's
 // registers are live in the other's loop.
-template <int BM, int BN, int WM, int WN, bool kSplit, int NCW>
+//
+// kWide: more than kWideChannels output channels, where a tile's output window
+// can pass 2 GiB: element stores at 64-bit addresses.
+template <int BM, int BN, int WM, int WN, bool kSplit, int NCW, bool kWide>
 __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs a) {
   constexpr int NMW = WM * WN;             // MFMA waves
   constexpr int NW = NCW > 0 ? NCW : NMW;  // copy waves
@@ -336,6 +339,30 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
   // store.
   const int rows = m_end - tile_m;
   const int px0 = wm * TMW, oc0 = tile_n + wn * TNW;
+  if constexpr (kWide) {
+    int32_t *const y =
+        kSplit ? a.partial + size_t(blockIdx.y) * size_t(a.gemm_m) * size_t(a.gemm_n) : a.y;
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+      const int oc = oc0 + 32 * i + (lane & 31);
+      if (oc >= a.gemm_n) continue;
+      const uint32_t bias = kSplit ? 0u : uint32_t(a.bias[oc]);
+#pragma unroll
+      for (int j = 0; j < FM; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int px = px0 + 32 * j + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+          if (px >= rows) continue;
+          const size_t at = size_t(tile_m + px) * size_t(a.gemm_n) + size_t(oc);
+          const int32_t v = int32_t(uint32_t(acc[i][j][e]) + bias);
+          if (!kSplit && a.q_y)
+            a.q_y[at] = int8_t(requant1(v, a.q_mult[oc], a.q_shift[oc], a.q_zp));
+          else
+            y[at] = v;
+        }
+    }
+    return;
+  }
   if (!kSplit && a.q_y) {
     const auto yr = make_rsrc(a.q_y + size_t(tile_m) * size_t(a.gemm_n),
                               uint32_t(rows) * uint32_t(a.gemm_n));
@@ -388,15 +415,15 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
     store_tile32<0>(acc, yr, rows, px0, oc0, a.gemm_n, lane);
 }
 
-template <int BM, int BN, int WM, int WN, int NCW = 0, bool kSplits = true>
+template <int BM, int BN, int WM, int WN, int NCW = 0, bool kSplits = true, bool kWide = false>
 int launch_tile(const ConvArgs &a, int splits, hipStream_t stream) {
   const int tiles = int(((int64_t(a.gemm_m) + a.m_step - 1) / a.m_step) * ((a.gemm_n + BN - 1) / BN));
   const int stages = a.gemm_k / kStageBytes;
   const int ring = std::min(kRing, splits > 1 ? a.stages_per_split : stages);
   const size_t lds = size_t(ring) * size_t(BM + BN) * kStageBytes;
-  auto kern = gemm_dma_kernel<BM, BN, WM, WN, false, NCW>;
+  auto kern = gemm_dma_kernel<BM, BN, WM, WN, false, NCW, kWide>;
   if constexpr (kSplits) {
-    if (splits > 1) kern = gemm_dma_kernel<BM, BN, WM, WN, true, NCW>;
+    if (splits > 1) kern = gemm_dma_kernel<BM, BN, WM, WN, true, NCW, kWide>;
   }
   static LdsLimit limits[2];
   if (const int rc = limits[splits > 1].raise(kern, lds); rc != I8CONV_OK) return rc;
@@ -427,6 +454,7 @@ int gemm_dma_copy_waves(const GemmPlan &p) {
   // anyway, and the split roles only add a barrier hop per stage.
   // The planner picks 256 x 128 only for more than four k-stages.
   const int per_workgroup = p.splits > 1 ? p.stages_per_split : p.stages;
+  if (p.wide) return 0;
   if (p.bm == 256 && p.bn == 128) return 8;
   return p.bm == 128 && p.bn == 128 && per_workgroup >= 4 ? 4 : 0;
 }
@@ -439,12 +467,18 @@ int launch_gemm_dma(const ConvArgs &args, const GemmPlan &p, int splits, void *s
   // one tap, a stage range per split, a tile it was built for, and LDS rows
   // the ring can hold
   const int stages = a.gemm_k / kStageBytes;
-  if (a.c % kStageBytes != 0 || a.gemm_n > (1 << 20) || a.gemm_k % kStageBytes != 0 || stages < 1 ||
+  if (a.c % kStageBytes != 0 || (a.gemm_n > kWideChannels) != p.wide || a.gemm_k % kStageBytes != 0 || stages < 1 ||
       (splits > 1 && (a.stages_per_split < 1 || int64_t(splits - 1) * a.stages_per_split >= stages)) ||
       !gemm_dma_tile_supported(p.bm, p.bn) || a.m_step % 16 != 0 || a.m_step > p.bm ||
       a.m_step < 16 ||
       size_t(kRing) * size_t(p.bm + p.bn) * kStageBytes > size_t(kLdsBudget)) {
     set_error("pipelined gemm plan out of range");
+    return I8CONV_BAD_ARGUMENT;
+  }
+  if (p.wide) {
+    if (p.bm == 128 && p.bn == 128)
+      return launch_tile<128, 128, 2, 4, 0, true, true>(a, splits, s);
+    set_error("unsupported pipelined gemm tile");
     return I8CONV_BAD_ARGUMENT;
   }
   // copy waves on the wide tiles when the workgroup has k-stages enough

@@ -75,11 +75,8 @@ bool gemm_tile_supported(int bm, int bn) {
 }
 
 // The LDS-DMA pipelined kernel (kernel_gemm_dma.hip) needs every 128-byte
-// k-stage inside one filter tap: c % 128 == 0, and a tile's output window
-// below 2 GiB.
-static bool dma_eligible(const i8conv_shape &s) {
-  return s.c % kStageBytes == 0 && s.k <= (1 << 20);
-}
+// k-stage inside one filter tap: c % 128 == 0.
+static bool dma_eligible(const i8conv_shape &s) { return s.c % kStageBytes == 0; }
 
 // Generic tile choice.  Pipelined kernel: 128 output channels per tile
 // (64 when N <= 64), and 256 pixels when that still gives the grid about
@@ -162,7 +159,8 @@ static GemmPlan plan_staged(const i8conv_shape &s, const i8conv_geometry &g) {
     p.dma = true;
     p.bn = g.gemm_n <= 64 ? 64 : 128;
     const int64_t tiles_n = ceil_div(g.gemm_n, p.bn);
-    p.bm = p.stages > 4 && ceil_div(g.gemm_m, 256) * tiles_n >= 192 ? 256 : 128;
+    p.wide = g.gemm_n > kWideChannels;
+    p.bm = !p.wide && p.stages > 4 && ceil_div(g.gemm_m, 256) * tiles_n >= 192 ? 256 : 128;
     p.m_step = gemm_dma_step(g.gemm_m, tiles_n, p.bm, p.bn);
     return p;
   }
@@ -318,6 +316,7 @@ GemmPlan plan_splitk(const i8conv_shape &s, const i8conv_geometry &g) {
   }
   p.dma = dma_eligible(s);
   if (p.dma) {
+    p.wide = g.gemm_n > kWideChannels;
     p.bn = g.gemm_n <= 64 ? 64 : 128;
     p.bm = 128;
   } else {

@@ -214,3 +214,29 @@ def test_pipelined_requant_bit_exact(name):
         exp = oracle.requantize(acc, mult, shift, 11)
         assert len(np.unique(exp)) > 50
         np.testing.assert_array_equal(got, exp, err_msg=form)
+
+
+# more than 2^20 output channels, C % 128 == 0: past the buffer windows of the
+# other forms (a pixel row of this output is 4 MB)
+VERY_WIDE = lab.ConvShape(1, 3, 3, 256, (1 << 20) + 4, 1, 1)
+
+
+def test_very_wide_layers_stay_on_the_pipelined_kernel():
+    assert "pipelined tile 128px x 128oc (80px stored), grid 1x8193" in lab.describe("generic", VERY_WIDE)
+    assert lab.dispatch(VERY_WIDE) == "generic"
+    assert lab.requant_fused(VERY_WIDE) and lab.requant_workspace_bytes(VERY_WIDE) == 0
+    assert "pipelined" in lab.describe("splitk", VERY_WIDE)
+
+
+@pytest.mark.gpu
+def test_very_wide_layers_bit_exact():
+    shape = VERY_WIDE
+    x, w, b = lab.make_case_data(shape, seed=71)
+    acc = oracle.conv(shape, x, w, b)
+    for kernel in ("generic", "splitk"):
+        say(f"[gpu] {kernel} on {shape}")
+        assert_bit_exact(run_kernel(kernel, shape, x, w, b), acc, kernel)
+    mult, shift = _qparams(shape.k, seed=72)
+    say("[gpu] requantized")
+    got = lab.conv2d_requant(x, w, b, mult, shift, -1, shape)
+    np.testing.assert_array_equal(got, oracle.requantize(acc, mult, shift, -1))
