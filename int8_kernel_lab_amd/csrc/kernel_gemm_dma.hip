@@ -403,6 +403,19 @@ __global__ __launch_bounds__(64 * (WM * WN + NCW)) void gemm_dma_kernel(ConvArgs
   }
   const auto yr = make_rsrc(out + size_t(tile_m) * size_t(a.gemm_n),
                             uint32_t(rows) * uint32_t(a.gemm_n) * 4u);
+  // Partial sums of the 64-channel tiles: short walks, where a quarter of the
+  // stores counts for more than the code of the transposes (3 x 19x19, 256 ->
+  // 48 dilated: 7.9 us in 4-byte stores, 7.7 so; two 128-channel tiles: no
+  // difference on average, 3 x 27x27, 1024 -> 128 1x1: 6.9, 7.3).
+  if constexpr (kSplit && BN == 64) {
+    if ((a.gemm_n & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+      if (sector_pitch(a.gemm_n))
+        store_tile32_x4<kStoreThrough>(acc, yr, rows, px0, oc0, a.gemm_n, lane);
+      else
+        store_tile32_x4<0>(acc, yr, rows, px0, oc0, a.gemm_n, lane);
+      return;
+    }
+  }
   // Outputs beyond 128 MiB: evict-first.  Written through, such outputs ran
   // up to 1.75x slower (16x256x256x256 1x1: 220 -> 388 us; 268 MB and up all
   // lost), while every output of the baseline layers (0.8-51 MB) gains from

@@ -62,6 +62,53 @@ __device__ __forceinline__ void store_tile32(const v16i (&acc)[FN][FM], __amdgpu
     }
 }
 
+// 4 x 4 transpose of dwords over the four lanes of a quad: lane k of the quad
+// ends with element k of lanes 0, 1, 2, 3.
+__device__ __forceinline__ v4i quad_transpose4(v4i a, int lane) {
+  const bool odd = lane & 1, high = lane & 2;
+  v4i b, c;
+#pragma unroll
+  for (int e = 0; e < 4; e += 2) {  // across lane bit 0: quad_perm 1 0 3 2
+    const int up = __builtin_amdgcn_update_dpp(0, a[e + 1], 0xb1, 0xf, 0xf, false);
+    const int down = __builtin_amdgcn_update_dpp(0, a[e], 0xb1, 0xf, 0xf, false);
+    b[e] = odd ? up : a[e];
+    b[e + 1] = odd ? a[e + 1] : down;
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {  // across lane bit 1: quad_perm 2 3 0 1
+    const int up = __builtin_amdgcn_update_dpp(0, b[e + 2], 0x4e, 0xf, 0xf, false);
+    const int down = __builtin_amdgcn_update_dpp(0, b[e], 0x4e, 0xf, 0xf, false);
+    c[e] = high ? up : b[e];
+    c[e + 2] = high ? b[e + 2] : down;
+  }
+  return c;
+}
+
+// store_tile32 in 16-byte stores (n % 4 == 0, window 16-byte aligned): a quad's
+// transpose gives each lane four channels of one pixel, and a store writes
+// eight whole 128-byte pieces.
+template <int kPolicy, int FM, int FN>
+__device__ __forceinline__ void store_tile32_x4(const v16i (&acc)[FN][FM], __amdgpu_buffer_rsrc_t out,
+                                                int rows, int px0, int oc0, int n, int lane) {
+  const uint32_t pitch = uint32_t(n) * 4u;
+  const int px = px0 + 4 * (lane >> 5) + (lane & 3), oc = oc0 + (lane & 28);
+#pragma unroll
+  for (int j = 0; j < FM; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int p = px + 32 * j + 8 * g;
+      const uint32_t off = uint32_t(p) * pitch + uint32_t(oc) * 4u;
+#pragma unroll
+      for (int i = 0; i < FN; ++i) {
+        const v4i v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
+                       acc[i][j][4 * g + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(
+            quad_transpose4(v, lane), out,
+            p < rows && oc + 32 * i < n ? off + 128u * i : kOutOfRange, 0, kPolicy);
+      }
+    }
+}
+
 // One channel's requantization constants for the blocks of a wave: the
 // odd-multiplier form where all of the wave's lanes allow it, else the exact
 // one.
