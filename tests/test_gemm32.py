@@ -19,14 +19,16 @@ CASES = {
     "64_c16_5x3": ("64px x 64oc", lab.ConvShape(3, 19, 23, 16, 68, 5, 3, 2, 0, 2, 1, 1, 2)),
     "64_c384_s2": ("64px x 64oc", lab.ConvShape(2, 23, 21, 384, 132, 3, 3, 1, 1, 2, 2, 1, 1)),
     # groups of waves on a tile's stages: two (7 and 15 stages: the second
-    # group's last one past the reduction), four (25 and 26 stages), with a
-    # second tile for some workgroups
+    # group's last one past the reduction), four (25 and 26 stages); one round
+    # of tiles, and with two groups a second tile for some workgroups (512)
     "64_g2_c96": ("64px x 64oc, grid 4x2, 7 k-stages, 2 wave groups",
                   lab.ConvShape(1, 15, 14, 96, 72, 3, 3, 1, 1, 1, 1, 1, 1)),
     "64_g2_c208_k33": ("64px x 64oc, grid 38x1, 15 k-stages, 2 wave groups",
                        lab.ConvShape(3, 27, 30, 208, 33, 3, 3, 1, 1, 1, 1, 1, 1)),
     "64_g2_450_tiles": ("64px x 64oc, grid 225x2, 6 k-stages, 2 wave groups",
                         lab.ConvShape(10, 40, 36, 80, 100, 3, 3, 1, 1, 1, 1, 1, 1)),
+    "64_g2_632_tiles": ("64px x 64oc, grid 316x2, 8 k-stages, 2 wave groups",
+                        lab.ConvShape(6, 58, 58, 112, 100, 3, 3, 1, 1, 1, 1, 1, 1)),
     "64_g4_c352": ("64px x 64oc, grid 4x2, 25 k-stages, 4 wave groups",
                    lab.ConvShape(2, 11, 10, 352, 68, 3, 3, 1, 1, 1, 1, 1, 1)),
     "64_g4_c656_5x1": ("64px x 64oc, grid 6x3, 26 k-stages, 4 wave groups",
@@ -34,15 +36,29 @@ CASES = {
     "64_k128": ("64px x 64oc", lab.ConvShape(18, 31, 33, 32, 36, 2, 2, 0, 0, 1, 1, 1, 1)),
     # 128 x 64: C = 32 and 48, odd channel counts, padding wider than the image
     "128x64_c32_k63": ("128px x 64oc", lab.ConvShape(5, 121, 119, 32, 63, 3, 3, 1, 1, 1, 1, 1, 1)),
-    # 128 x 32: at most 32 channels, also of pixel rows past the image
+    # ... more tiles than the 768 workgroups
+    "128x64_k40_851_tiles": ("128px x 64oc, grid 851x1",
+                             lab.ConvShape(1, 330, 330, 32, 40, 3, 3, 1, 1, 1, 1, 1, 1)),
+    # 128 x 32: at most 32 channels, also of pixel rows past the image; more
+    # tiles than workgroups
+    "128x32_k20_851_tiles": ("128px x 32oc, grid 851x1",
+                             lab.ConvShape(1, 330, 330, 32, 20, 3, 3, 1, 1, 1, 1, 1, 1)),
     "128x32_c48_k4": ("128px x 32oc", lab.ConvShape(1, 250, 263, 48, 4, 7, 7, 3, 3, 1, 1, 1, 1)),
     "128x32_c32_k32": ("128px x 32oc", lab.ConvShape(3, 151, 149, 32, 32, 3, 3, 1, 1, 1, 1, 1, 1)),
     "128x64_c48_k36": ("128px x 64oc", lab.ConvShape(1, 250, 263, 48, 36, 5, 5, 3, 3, 1, 1, 1, 1)),
     # 128 x 128: N = 65 and 255 (one, then two channel tiles), 1x3 dilated
     "128_k65": ("128px x 128oc", lab.ConvShape(2, 129, 130, 64, 65, 3, 3, 1, 1, 1, 1, 1, 1)),
     "128_k255": ("128px x 128oc", lab.ConvShape(1, 130, 131, 64, 255, 1, 3, 0, 2, 1, 1, 1, 2)),
+    "128_k250_652_tiles": ("128px x 128oc, grid 326x2",
+                           lab.ConvShape(1, 205, 203, 48, 250, 1, 3, 0, 1, 1, 1, 1, 1)),
     "128_k260": ("128px x 128oc", lab.ConvShape(1, 123, 125, 112, 260, 1, 1, 0, 0, 1, 1, 1, 1)),
-    # 256 x 256: 514 tiles (two full rounds and a partial one), N = 132
+    # 256 x 256: 514 tiles (two full rounds and a partial one), N = 132; three
+    # channel chunks of a 1x3 filter and a stride-2 layer, both with a pixel
+    # tail and N = 388 (a second channel tile of which half is dead)
+    "256_c384_1x3_k388": ("256px x 256oc, grid 256x2, 9 k-stages",
+                          lab.ConvShape(1, 255, 257, 384, 388, 1, 3, 0, 1, 1, 1, 1, 1)),
+    "256_s2_k388": ("256px x 256oc, grid 256x2, 9 k-stages",
+                    lab.ConvShape(1, 509, 513, 128, 388, 3, 3, 1, 1, 2, 2, 1, 1)),
     "256_k132": ("256px x 256oc", lab.ConvShape(2, 256, 257, 128, 132, 3, 3, 1, 1, 1, 1, 1, 1)),
 }
 
@@ -138,10 +154,15 @@ BYTE_CASES = {
     "128x32_k31": lab.ConvShape(2, 187, 185, 48, 31, 1, 3, 0, 1, 1, 1, 1, 1),
     "128x128_k94": lab.ConvShape(3, 137, 131, 32, 94, 3, 3, 1, 1, 1, 1, 1, 1),
     "128x128_k255_again": lab.ConvShape(1, 205, 203, 48, 255, 1, 3, 0, 1, 1, 1, 1, 1),
+    "256_k255": lab.ConvShape(1, 363, 361, 128, 255, 3, 3, 1, 1, 1, 1, 1, 1),
     "64_k30_halo_layer": lab.ConvShape(3, 22, 21, 64, 30, 3, 3, 2, 2, 1, 1, 2, 2),
     "pipelined_k101": lab.ConvShape(2, 101, 97, 128, 101, 3, 3, 1, 1, 2, 2, 1, 1),
     "pipelined_k130": lab.ConvShape(4, 64, 67, 384, 130, 1, 1, 0, 0, 1, 1, 1, 1),
 }
+
+
+def test_gemm32_byte_stores_on_256_wide_tiles():
+    assert "32x32 MFMA tile 256px x 256oc, grid 512x1" in lab.describe("generic", BYTE_CASES["256_k255"])
 
 
 @pytest.mark.gpu
@@ -240,3 +261,16 @@ def test_very_wide_layers_bit_exact():
     say("[gpu] requantized")
     got = lab.conv2d_requant(x, w, b, mult, shift, -1, shape)
     np.testing.assert_array_equal(got, oracle.requantize(acc, mult, shift, -1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [64, 60, 36, 24, 63])
+def test_splitk_64_channel_tiles_bit_exact(k):
+    # partial sums in 16-byte stores (whole sectors, ordinary, a tail inside a
+    # 32-channel block), in 4-byte stores (N % 4 != 0); a pixel tail; the last
+    # split shorter than the others
+    shape = lab.ConvShape(1, 17, 13, 384, k, 3, 3, 2, 2, 1, 1, 2, 2)
+    assert "splitk pipelined tile 128px x 64oc" in lab.describe("splitk", shape)
+    x, w, b = lab.make_case_data(shape, seed=81)
+    say(f"[gpu] splitk on {shape}")
+    assert_bit_exact(run_kernel("splitk", shape, x, w, b), oracle.conv(shape, x, w, b), f"k{k}")

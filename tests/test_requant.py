@@ -116,12 +116,12 @@ def test_requant_fused_where_the_dispatched_kernel_requantizes():
     # the pipelined GEMM's epilogue and split-K's second pass
     for name in ("cfg3_down_3x3_s2", "cfg5b_dilated", "cfg5a_deep_k"):
         assert lab.requant_fused(_baseline(name)), name
-    # the row kernel without copy waves (C = 64) has no requantizing epilogue
+    # the row kernel without copy waves (C = 64) asks for the int32 workspace
     assert not lab.requant_fused(_baseline("cfg1_smoke"))
     # pointwise slices of 32 channels (C = 512) have no requantizing
     # instance: the pipelined GEMM (C % 128 == 0) requantizes in its
     # epilogue instead; slices of 256 (C = 64, N = 256) or 32 channels with
-    # C = 64 go unfused (the register-staged GEMM has no such epilogue)
+    # C = 64 ask for the int32 workspace
     wide = lab.ConvShape(1, 8, 8, 512, 64, 1, 1, 0, 0, 1, 1, 1, 1)
     assert lab.requant_fused(wide) and lab.requant_workspace_bytes(wide) == 0
     for shape in (lab.ConvShape(1, 8, 8, 64, 256, 1, 1, 0, 0, 1, 1, 1, 1),
@@ -138,7 +138,7 @@ def test_requant_workspace_sizes():
     # split-K's second pass requantizes: only the partial sums
     s5 = _baseline("cfg5a_deep_k")
     assert lab.requant_workspace_bytes(s5) == lab.workspace_bytes("splitk", s5)
-    # unfused (the C = 64 row kernel): the int32 output, 256-byte aligned
+    # the C = 64 row kernel: the int32 output, 256-byte aligned
     s1 = _baseline("cfg1_smoke")
     acc = (s1.output_elements * 4 + 255) // 256 * 256
     assert lab.requant_workspace_bytes(s1) == acc + lab.workspace_bytes(lab.dispatch(s1), s1)
@@ -147,13 +147,12 @@ def test_requant_workspace_sizes():
 def test_requant_launch_errors_without_gpu():
     s3 = _baseline("cfg3_down_3x3_s2")
     fake = 1 << 20  # never dereferenced: the checks fail before any launch
-    # unfused (the C = 64 row kernel) without a workspace
+    # the C = 64 row kernel without the workspace it asks for
     with pytest.raises(lab.I8ConvError) as e:
         lab.launch_requant(_baseline("cfg1_smoke"), fake, fake, fake, fake, fake, 0, fake, None, 0)
     assert e.value.status == _lib.WORKSPACE_TOO_SMALL
-    # the pipelined GEMM fuses only with 16-byte aligned mult and shift: a
-    # multiplier array at +4 bytes takes the unfused way, which needs the
-    # int32 workspace
+    # the pipelined GEMM does without the int32 workspace only with 16-byte
+    # aligned mult and shift: a multiplier array at +4 bytes asks for it
     with pytest.raises(lab.I8ConvError, match="16-byte aligned") as e:
         lab.launch_requant(s3, fake, fake, fake, fake + 4, fake, 0, fake, None, 0)
     assert e.value.status == _lib.WORKSPACE_TOO_SMALL
@@ -168,8 +167,8 @@ def test_requant_launch_errors_without_gpu():
     with pytest.raises(lab.I8ConvError) as e:
         lab.requantize(fake, 10, 0, fake, fake, 0, fake)
     assert e.value.status == _lib.BAD_ARGUMENT
-    # the pointwise form fuses only with 16-byte aligned bias, mult, shift
-    # and output; an output at +4 bytes needs the unfused workspace
+    # the pointwise form requantizes only with 16-byte aligned bias, mult,
+    # shift and output; an output at +4 bytes asks for the int32 workspace
     s4a = _baseline("cfg4a_pointwise_1x1")
     with pytest.raises(lab.I8ConvError, match="16-byte aligned") as e:
         lab.launch_requant(s4a, fake, fake, fake, fake, fake, 0, fake + 4, None, 0)
@@ -283,7 +282,7 @@ GEMM_RQ = {
     # the pipelined GEMM's requantizing epilogue (C % 128 == 0, N % 4 == 0):
     # a 1x1 layer whose pointwise form has no requantizing instance (C =
     # 512); a stride-2 layer with a 4-channel tail past 128; C = 64 takes the
-    # register-staged GEMM and the int32 pass
+    # 32 x 32 MFMA kernel's epilogue instead of the register-staged GEMM's pass
     "c512_1x1_k64": lab.ConvShape(1, 9, 9, 512, 64, 1, 1, 0, 0, 1, 1, 1, 1),
     "s2_k132": lab.ConvShape(8, 28, 28, 128, 132, 3, 3, 1, 1, 2, 2, 1, 1),
     "c64_s2_pass": lab.ConvShape(2, 16, 16, 64, 64, 3, 3, 1, 1, 2, 2, 1, 1),
@@ -386,9 +385,9 @@ def test_pointwise_requant_odd_form_bit_exact(name, mixed):
 
 
 @pytest.mark.gpu
-def test_pointwise_requant_unaligned_output_takes_the_unfused_path():
-    # output at +4 bytes: the convolution into the int32 workspace and the
-    # requantizing pass, bit-exact, nothing written outside the output
+def test_pointwise_requant_unaligned_output():
+    # output at +4 bytes: not the pointwise form but the 32 x 32 MFMA kernel's
+    # epilogue, bit-exact, nothing written outside the output
     from tests.conftest import say
     shape = POINTWISE_RQ["c64_k128"]
     x, w, b = lab.make_case_data(shape, seed=13)
