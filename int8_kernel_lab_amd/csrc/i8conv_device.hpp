@@ -87,9 +87,10 @@ struct ConvArgs {
   // pipelined GEMM: pixel rows a tile stores (its tile height, or fewer:
   // the tile's last rows then read as zeros and are not stored)
   int m_step;
-  // pipelined GEMM only: requantized int8 output from its epilogue when
-  // q_y != nullptr (y unused), with per-channel multipliers and shifts
-  // (16-byte aligned, N % 4 == 0) and the zero point
+  // pipelined and 32 x 32 MFMA GEMM: requantized int8 output from their
+  // epilogue when q_y != nullptr (y unused), with per-channel multipliers and
+  // shifts and the zero point; the pipelined one needs N % 4 == 0 and a 4-byte
+  // aligned q_y (any where N > kWideChannels), the other takes any
   const int32_t *q_mult;
   const int32_t *q_shift;
   int32_t q_zp;

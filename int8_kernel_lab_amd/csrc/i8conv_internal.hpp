@@ -155,9 +155,10 @@ bool plan_strip(const i8conv_shape &s, const i8conv_geometry &g, PatchPlan *p);
 
 // Dispatch policy (policy.cpp): an eligible kernel id, or -1 for a bad shape.
 int dispatch(const i8conv_shape &s);
-// Generic layers whose int8 launch asks for the int32 workspace all the same
-// (and leaves it alone): small grids of stride-1 spatial filters, which halo
-// and strip plans also cover and which callers have always sized it for
+// Generic layers whose int8 launch asks for the int32 workspace all the same:
+// small grids of stride-1 spatial filters, which halo and strip plans also
+// cover and which callers have always sized it for.  Only an output that
+// overlaps the input, filter or bias uses it.
 bool dispatch_patch_layer(const i8conv_shape &s);
 
 ConvArgs make_args(const i8conv_shape &s, const i8conv_geometry &g,
@@ -175,7 +176,7 @@ int launch_splitk(const ConvArgs &a, const GemmPlan &p, void *workspace,
 // kernel_gemm_dma.hip; splits > 1 writes partial sums to a.partial
 int launch_gemm_dma(const ConvArgs &a, const GemmPlan &p, int splits, void *stream);
 // kernel_gemm32.hip: whether a layer's sizes fit it, and its launch (int8
-// output when a.q_y is set: N % 4 == 0 and a 4-byte aligned q_y)
+// output when a.q_y is set, any N and alignment)
 bool gemm32_eligible(const i8conv_shape &s, const i8conv_geometry &g);
 int launch_gemm32(const ConvArgs &a, const GemmPlan &p, void *stream);
 // kernel_pointwise.hip: C and N with an instance (C in {64, 128, 256,

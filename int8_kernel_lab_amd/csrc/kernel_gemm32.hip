@@ -14,17 +14,17 @@
 //   * v_mfma_i32_32x32x32 does the operations of two 16 x 16 x 64 with half
 //     the operand reads: on random operands, all SIMDs busy, it sustains 3.45
 //     POP/s against 2.8 (the shader clock follows the power drawn);
-//   * k-stages of 128 bytes per row come by LDS-DMA (R stage buffers, one
+//   * k-stages of 128 bytes per row come by LDS-DMA (two stage buffers, one
 //     barrier per stage).  A 128-byte row is a whole L2 line: the same copies
 //     in 64-byte halves land at 70 instead of 130 GB/s per compute unit;
 //   * with kLaneTap each lane decomposes its own 16-byte chunk's k into tap
 //     and channel, so a stage may span taps (C % 128 != 0); otherwise a stage
 //     lies inside one tap and the channel chunk is the outer loop, the taps
 //     the inner one;
-//   * workgroups are persistent: the next tile's first R stages are copied
+//   * workgroups are persistent: the next tile's first stages are copied
 //     before the tile's stores go out.  Small tiles share a compute unit two
 //     to four at a time, which hides their copy issue and LDS latency better
-//     than more stage buffers did (R = 2, 4, 6, 9 within 8 %);
+//     than more than two stage buffers did (4, 6 and 9 within 8 %);
 //   * int8 output: each lane requantizes its channel (parameters read once
 //     per tile), and the four lanes of a quad turn their bytes into one
 //     pixel's four channels per lane; other channel counts and alignments
@@ -47,6 +47,7 @@ namespace {
 template <int N>
 using Set = std::integral_constant<int, N>;
 
+constexpr int kStageBuffers = 2;  // per group of waves
 
 // What the epilogue writes: int32, or requantized int8 in 4-byte stores (N % 4
 // == 0, output 4-byte aligned) or byte stores (any N).
@@ -55,19 +56,6 @@ enum OutKind { kOutInt32, kOutInt8, kOutInt8Bytes };
 template <int N>
 __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// at most `stages` stages of CPW copies outstanding (0 <= stages <= MOST)
-template <int CPW, int MOST>
-__device__ __forceinline__ void wait_stages(int stages) {
-  if constexpr (MOST == 0) {
-    wait_vm<0>();
-  } else {
-    if (stages >= MOST)
-      wait_vm<(CPW * MOST < 63 ? CPW * MOST : 63)>();
-    else
-      wait_stages<CPW, MOST - 1>(stages);
-  }
 }
 
 __device__ __forceinline__ void barrier_lds() {
@@ -79,12 +67,12 @@ __device__ __forceinline__ void barrier_lds() {
 // BM pixels x BN channels over WM x WN waves; KG groups of such waves, each
 // with stage buffers of its own, take the k-stages in turn (group g the
 // stages g, g + KG, ...) and add their sums up through LDS at the end;
-// fragments read GS k-steps of 32 bytes at a time; R stage buffers per group;
-// kOcc waves per SIMD.
-template <int BM, int BN, int WM, int WN, int KG, int GS, int R, bool kLaneTap, int kOut,
-          int kPolicy, int kOcc>
+// fragments read GS k-steps of 32 bytes at a time; kOcc waves per SIMD.
+template <int BM, int BN, int WM, int WN, int KG, int GS, bool kLaneTap, int kOut, int kPolicy,
+          int kOcc>
 __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArgs a, int tiles) {
   constexpr int P = kStageBytes;             // bytes per LDS row: one k-stage
+  constexpr int R = kStageBuffers;
   constexpr int KS = P / 32;                 // k-steps per stage
   constexpr int kWaves = WM * WN;
   constexpr int TM = BM / WM, TN = BN / WN;  // pixels and channels per wave
@@ -270,10 +258,13 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
   bool pend = false;  // ST stores of the previous tile follow the prologue's copies
   prologue(slot);
   for (;;) {
+    // the first stage has landed
     if (pend)
       wait_vm<(ST < 63 ? ST : 63)>();
+    else if (stages > 1)
+      wait_vm<CPW>();
     else
-      wait_stages<CPW, R - 1>(min(R, stages) - 1);
+      wait_vm<0>();
     barrier_lds();
 
     v16i acc[FN][FM];
@@ -306,7 +297,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
     for (int q = 0; q < kReads; ++q) read(Set<0>{}, bufs, 0, q);
 
     int ring = 0;
-    auto stage = [&](auto first, int s) {
+    auto stage = [&](int s) {
       const int next = ring + 1 == R ? 0 : ring + 1;
       const int8_t *const buf = bufs + ring * kTile;
       const int8_t *const nbuf = bufs + next * kTile;
@@ -316,8 +307,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
       auto part = [&](auto set, auto last, int pt) {
         if (last.value) {
           // every wave has read all of stage s, and stage s + 1 has landed
-          if (s + 1 < stages && !(pend && s + 1 < R))
-            wait_stages<CPW, R - 2>(min(R - 2, stages - 2 - s));
+          if (s + 1 < stages && !(pend && s + 1 < R)) wait_vm<0>();
           barrier_lds();
         }
 #pragma unroll
@@ -335,26 +325,16 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
           __builtin_amdgcn_sched_barrier(0);
         }
       };
-      if constexpr (NP == 1) {
-        part(first, std::true_type{}, 0);
-      } else {
-        static_assert(NP % 2 == 0, "one set per stage, or an even number");
-        part(Set<0>{}, std::false_type{}, 0);
-        if constexpr (NP == 4) {
-          part(Set<1>{}, std::false_type{}, 1);
-          part(Set<0>{}, std::false_type{}, 2);
-        }
-        part(Set<1>{}, std::true_type{}, NP - 1);
+      static_assert(NP == 2 || NP == 4, "an even number of sets per stage");
+      part(Set<0>{}, std::false_type{}, 0);
+      if constexpr (NP == 4) {
+        part(Set<1>{}, std::false_type{}, 1);
+        part(Set<0>{}, std::false_type{}, 2);
       }
+      part(Set<1>{}, std::true_type{}, NP - 1);
       ring = next;
     };
-    for (int s = 0; s < stages; ++s) {
-      stage(Set<0>{}, s);
-      if constexpr (NP == 1) {
-        if (++s == stages) break;
-        stage(Set<1>{}, s);
-      }
-    }
+    for (int s = 0; s < stages; ++s) stage(s);
 
     const int out_m = tile_m, out_n = tile_n, out_end = m_end;
     t += run.step;
@@ -454,10 +434,9 @@ __global__ __launch_bounds__(64 * WM * WN * KG, kOcc) void gemm32_kernel(ConvArg
 template <int BM, int BN, int WM, int WN, int KG, int GS, bool kLaneTap, int kOcc, int kGroups,
           int kOut, int kPolicy>
 int launch_tile(const ConvArgs &a, hipStream_t stream) {
-  constexpr int R = 2;
-  auto kern = gemm32_kernel<BM, BN, WM, WN, KG, GS, R, kLaneTap, kOut, kPolicy, kOcc>;
+  auto kern = gemm32_kernel<BM, BN, WM, WN, KG, GS, kLaneTap, kOut, kPolicy, kOcc>;
   const size_t lds =
-      size_t(KG) * R * (BM + BN) * kStageBytes + 2 * (kOut == kOutInt32 ? 1 : 3) * BN * 4;
+      size_t(KG) * kStageBuffers * (BM + BN) * kStageBytes + 2 * (kOut == kOutInt32 ? 1 : 3) * BN * 4;
   const int tiles = int(((int64_t(a.gemm_m) + BM - 1) / BM) * ((a.gemm_n + BN - 1) / BN));
   static LdsLimit limit;
   if (const int rc = limit.raise(kern, lds); rc != I8CONV_OK) return rc;
