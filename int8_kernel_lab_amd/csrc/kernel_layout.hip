@@ -49,9 +49,10 @@ constexpr int kTileRowBytes = 128;
 constexpr int kDwordTile = 64;  // dwords per side of a dword tile
 constexpr int kShortSide = 16;   // shorter sides than this: an element per thread
 constexpr int kShortMost = 512;  // longest short side of the short-row and short-column forms
-// Dword transposes of at least so many bytes store evict-first (32 x 56x56 x
-// 128: 15.8 us, written through 19.3; 256 channels: 36.3, 37.8), smaller ones
-// through (32 x 14x14 x 512: 5.6 us, evict-first 6.5).
+// Dword transposes between 16-byte rows of at least so many bytes store
+// evict-first (32 x 56x56 x 128: 15.8 us, written through 19.3; 256 channels:
+// 36.3, 37.8), smaller ones through (32 x 14x14 x 512: 5.6 us, evict-first
+// 6.5); those of any length store ordinarily.
 constexpr int64_t kStreamTransposeBytes = 32 << 20;
 
 __device__ __forceinline__ int byte_tile_row(int i) { return 32 * i + 8 * (i >> 4); }
@@ -92,9 +93,8 @@ __device__ __forceinline__ v4i load16_any(const int8_t *src, int64_t off, int64_
 // values), and only a last tile of fewer than 16 rows stores single bytes.
 template <int kSub, bool kAny>
 __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *src, int8_t *dst,
-                                                                  int64_t batch, int rows,
-                                                                  int cols, int tiles_r,
-                                                                  int tiles_c) {
+                                                                  int rows, int cols, int tiles_r,
+                                                                  int tiles_c, int64_t batch) {
   constexpr int T = kTileRowBytes;
   constexpr int kTileDw = 32 * T + 8 * (T / 16);  // one 128 x 128 tile
   __shared__ __align__(16) uint32_t tile[kSub * kTileDw];
@@ -109,10 +109,6 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
   const int r0 = tr * T, c0 = tc * T * kSub;
   // read: tile row i = source row r0 + i, bytes [c0, c0 + 128 kSub); piece
   // pc of the row goes to tile pc / 8
-  auto place = [&](int idx, v4i v) {
-    const int i = idx / (8 * kSub), pc = idx % (8 * kSub);
-    *reinterpret_cast<v4i *>(&tile[(pc >> 3) * kTileDw + byte_tile_row(i) + 4 * (pc & 7)]) = v;
-  };
   if constexpr (kAny) {
     // every load before the first LDS write: left to itself the compiler waits
     // for each (16 x 256 x 45x45: 5.5 against 6.7 us)
@@ -127,12 +123,18 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
                   : v4i{0, 0, 0, 0};
     }
 #pragma unroll
-    for (int u = 0; u < 4 * kSub; ++u) place(int(threadIdx.x) + u * kThreads, in[u]);
+    for (int u = 0; u < 4 * kSub; ++u) {
+      const int idx = int(threadIdx.x) + u * kThreads;
+      const int i = idx / (8 * kSub), pc = idx % (8 * kSub);
+      *reinterpret_cast<v4i *>(&tile[(pc >> 3) * kTileDw + byte_tile_row(i) + 4 * (pc & 7)]) = in[u];
+    }
   } else {
     for (int idx = threadIdx.x; idx < T * 8 * kSub; idx += kThreads) {
-      const uint32_t row = uint32_t(r0 + idx / (8 * kSub)), cb = uint32_t(c0 + idx % (8 * kSub) * 16);
-      place(idx, load16(sr, row < uint32_t(rows) && cb < uint32_t(cols) ? row * uint32_t(cols) + cb
-                                                                       : kOutOfRange));
+      const int i = idx / (8 * kSub), pc = idx % (8 * kSub);
+      const uint32_t cb = uint32_t(c0 + pc * 16);
+      const bool ok = r0 + i < rows && cb < uint32_t(cols);
+      *reinterpret_cast<v4i *>(&tile[(pc >> 3) * kTileDw + byte_tile_row(i) + 4 * (pc & 7)]) =
+          load16(sr, ok ? uint32_t(r0 + i) * uint32_t(cols) + cb : kOutOfRange);
     }
   }
   __syncthreads();
@@ -186,9 +188,8 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
 // a last tile of fewer than four.
 template <bool kAny, int kPolicy>
 __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t *src, int8_t *dst,
-                                                                   int64_t batch, int rows,
-                                                                   int cols, int tiles_r,
-                                                                   int tiles_c) {
+                                                                   int rows, int cols, int tiles_r,
+                                                                   int tiles_c, int64_t batch) {
   constexpr int T = kDwordTile, kPitch = T + 1;
   __shared__ uint32_t tile[T * kPitch];
   const int per_mat = tiles_r * tiles_c;
@@ -417,12 +418,14 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
     const int sub = esize == 1 && cols >= 2 * T ? 2 : 1;
     const int tiles_c = (cols + sub * T - 1) / (sub * T);
     const int64_t blocks = batch * tiles_r * tiles_c;  // < 2^31: checked by the caller
-    auto kern = esize != 1 ? (total * 4 >= kStreamTransposeBytes
-                                  ? transpose_dwords_tiled<kAny, kStoreStream>
-                                  : transpose_dwords_tiled<kAny, kStoreThrough>)
-                           : sub == 2 ? transpose_bytes_tiled<2, kAny> : transpose_bytes_tiled<1, kAny>;
-    hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kThreads), 0, s, in, out, batch, rows,
-                       cols, tiles_r, tiles_c);
+    auto kern = sub == 2 ? transpose_bytes_tiled<2, kAny> : transpose_bytes_tiled<1, kAny>;
+    if (esize != 1) {
+      kern = transpose_dwords_tiled<kAny, kAny ? 0 : kStoreThrough>;
+      if (!kAny && total * 4 >= kStreamTransposeBytes)
+        kern = transpose_dwords_tiled<kAny, kAny ? 0 : kStoreStream>;
+    }
+    hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kThreads), 0, s, in, out, rows, cols,
+                       tiles_r, tiles_c, batch);
     return launch_status("transpose launch");
   };
   if (aligned16 && rows16 && cols16) return tiled(std::false_type{});
