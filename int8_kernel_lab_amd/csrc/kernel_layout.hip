@@ -87,10 +87,11 @@ __device__ __forceinline__ v4i load16_any(const int8_t *src, int64_t off, int64_
   return v;
 }
 
-// kAny: rows, columns and bases of any length and alignment.  Pieces then
-// start at any byte; a column's last 16 rows are stored by a lane that starts
-// early enough to end with them (some bytes are written twice, with the same
-// values), and only a last tile of fewer than 16 rows stores single bytes.
+// kAny: at least 16 rows and columns, of any length, and bases of any
+// alignment.  Pieces then start at any byte; a column's last 16 rows are stored
+// by a lane that starts early enough to end with them, and a last tile of fewer
+// than 16 rows starts early too (some bytes are written twice, with the same
+// values; single byte stores for such a tile: 4 x 513 x 19x19: 6.6 us, 4.0 so).
 template <int kSub, bool kAny>
 __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *src, int8_t *dst,
                                                                   int rows, int cols, int tiles_r,
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
   const size_t mat_bytes = size_t(rows) * size_t(cols);  // < 2^31: checked at launch
   const auto sr = make_rsrc(src + size_t(mat) * mat_bytes, uint32_t(mat_bytes));
   const auto dr = make_rsrc(dst + size_t(mat) * mat_bytes, uint32_t(mat_bytes));
-  const int r0 = tr * T, c0 = tc * T * kSub;
+  const int r0 = kAny ? min(tr * T, rows - 16) : tr * T, c0 = tc * T * kSub;
   // read: tile row i = source row r0 + i, bytes [c0, c0 + 128 kSub); piece
   // pc of the row goes to tile pc / 8
   if constexpr (kAny) {
@@ -144,9 +145,7 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
   const int cg = threadIdx.x >> 3, rg = threadIdx.x & 7;
   int i0 = 16 * rg;
   if (r0 + i0 >= rows) return;  // !kAny: rows % 16 == 0, a row group is whole or absent
-  const int live = min(T, rows - r0);
-  if (kAny && i0 + 16 > live) i0 = max(0, live - 16);
-  const int n = kAny ? min(16, live - i0) : 16;  // < 16 only in a tile of fewer rows
+  if constexpr (kAny) i0 = min(i0, rows - r0 - 16);
 #pragma unroll
   for (int sub = 0; sub < kSub; ++sub) {
     uint32_t out[4][4];  // [column][4-row group]
@@ -165,14 +164,8 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
       if (col >= cols) continue;
       const v4i v{int32_t(out[c][0]), int32_t(out[c][1]), int32_t(out[c][2]), int32_t(out[c][3])};
       if constexpr (kAny) {
-        int8_t *const d = dst + int64_t(mat) * int64_t(mat_bytes) + int64_t(col) * rows + r0 + i0;
-        if (n == 16) {
-          __builtin_memcpy(d, &v, 16);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 15; ++e)
-            if (e < n) d[e] = int8_t(uint32_t(v[e >> 2]) >> (8 * (e & 3)));
-        }
+        __builtin_memcpy(dst + int64_t(mat) * int64_t(mat_bytes) + int64_t(col) * rows + r0 + i0,
+                         &v, 16);
       } else {
         __builtin_amdgcn_raw_buffer_store_b128(
             v, dr, uint32_t(col) * uint32_t(rows) + uint32_t(r0 + i0), 0, kStoreThrough);
@@ -184,8 +177,8 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
 // Dwords: 64 x 64 tiles, so that both sides move in 256-byte pieces and each
 // lane has four 16-byte loads in flight.  A 65-dword pitch puts the 16 pieces
 // x 4 rows of a wave's LDS accesses in 64 distinct banks on both sides.  kAny
-// as above: a lane's four rows end with the tile's last row, single dwords in
-// a last tile of fewer than four.
+// as above: a lane's four rows end with the tile's last row, and a last tile of
+// fewer than four starts early.
 template <bool kAny, int kPolicy>
 __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t *src, int8_t *dst,
                                                                    int rows, int cols, int tiles_r,
@@ -200,7 +193,7 @@ __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t 
   const size_t mat_bytes = size_t(rows) * size_t(cols) * 4;  // < 2^31: checked at launch
   const auto sr = make_rsrc(src + size_t(mat) * mat_bytes, uint32_t(mat_bytes));
   const auto dr = make_rsrc(dst + size_t(mat) * mat_bytes, uint32_t(mat_bytes));
-  const int r0 = tr * T, c0 = tc * T;
+  const int r0 = kAny ? min(tr * T, rows - 4) : tr * T, c0 = tc * T;
   const uint32_t row_bytes = uint32_t(cols) * 4;
   const int piece = threadIdx.x & 15, line = threadIdx.x >> 4;
   // read: tile row i = source row r0 + i, bytes [c0*4, c0*4 + 256)
@@ -228,9 +221,7 @@ __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t 
   const uint32_t out_row_bytes = uint32_t(rows) * 4;
   int i0 = piece * 4;
   if (r0 + i0 >= rows) return;
-  const int live = min(T, rows - r0);
-  if (kAny && i0 + 4 > live) i0 = max(0, live - 4);
-  const int n = kAny ? min(4, live - i0) : 4;  // < 4 only in a tile of fewer rows
+  if constexpr (kAny) i0 = min(i0, rows - r0 - 4);
 #pragma unroll
   for (int u = 0; u < T / 16; ++u) {
     const int j = line + 16 * u, c = c0 + j;
@@ -239,17 +230,8 @@ __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t 
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = int32_t(tile[(i0 + e) * kPitch + j]);
     if constexpr (kAny) {
-      int8_t *const d = dst + int64_t(mat) * int64_t(mat_bytes) + int64_t(c) * out_row_bytes +
-                        int64_t(r0 + i0) * 4;
-      if (n == 4) {
-        __builtin_memcpy(d, &v, 16);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 3; ++e) {
-          const int32_t x = v[e];
-          if (e < n) __builtin_memcpy(d + 4 * e, &x, 4);
-        }
-      }
+      __builtin_memcpy(dst + int64_t(mat) * int64_t(mat_bytes) + int64_t(c) * out_row_bytes +
+                           int64_t(r0 + i0) * 4, &v, 16);
     } else {
       __builtin_amdgcn_raw_buffer_store_b128(
           v, dr, uint32_t(c) * out_row_bytes + uint32_t(r0 + i0) * 4, 0, kPolicy);

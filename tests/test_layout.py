@@ -169,3 +169,36 @@ def test_transposes_between_unaligned_tensors_bit_exact(off):
     assert (out[:off] == 0x5A).all() and (out[off + x.size:] == 0x5A).all()
     src.close()
     dst.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("n,rows,cols", [
+    # large enough for tiles of any length on both sides: last tiles of one row,
+    # of fewer rows than a lane stores and of just enough, of one column; one
+    # tile of rows; few columns.  The last one: elements
+    (1, 16, 24577), (2, 513, 523), (1, 257, 2049), (3, 143, 1401), (1, 1025, 401), (2, 399, 1023),
+    (1, 24577, 17), (3, 131, 1001), (1, 385, 639)])
+def test_tiled_transposes_of_any_length_bit_exact(n, rows, cols, off):
+    from tests.conftest import say
+    rng = np.random.default_rng(rows + cols)
+    for dtype in (np.int8, np.int32):
+        say(f"[gpu] tiled transposes {n}x{rows}x{cols} {dtype.__name__} at +{off}")
+        x = rng.integers(-128, 128, size=(n, rows, cols), dtype=np.int64).astype(dtype)
+        pad = off // x.itemsize
+        src, dst = lab.DeviceBuffer(x.nbytes + 16), lab.DeviceBuffer(x.nbytes + 16)
+        try:
+            src.upload(np.concatenate([np.zeros(pad, dtype), x.reshape(-1),
+                                       np.zeros(16 // x.itemsize - pad, dtype)]))
+            dst.fill(0x5A)
+            transpose = lab.nchw_to_nhwc if dtype == np.int8 else lab.nhwk_to_nkhw
+            dims = (rows, 1, cols) if dtype == np.int8 else (1, rows, cols)
+            transpose(src.ptr + off, dst.ptr + off, n, *dims)
+            lab.synchronize()
+            raw = dst.download(np.int8, x.nbytes + 16)
+        finally:
+            src.close()
+            dst.close()
+        got = raw[off:off + x.nbytes].view(dtype).reshape(n, cols, rows)
+        np.testing.assert_array_equal(got, x.transpose(0, 2, 1))
+        assert (raw[:off] == 0x5A).all() and (raw[off + x.nbytes:] == 0x5A).all()
