@@ -17,8 +17,15 @@
 // x 45x37 x 128: 6.1, tiled 4.3).  Everything else runs the tiled form with
 // pieces at any byte: an element per thread, its writes scattered, took 62 us
 // for 16 x 45x45 x 256 dwords (12 tiled, 5.5 TB/s), 298 for 32 x 448 x 63x63
-// bytes (30 tiled).  Tensors with a side below 16 elements keep the
-// element-per-thread form.
+// bytes (30 tiled).
+//
+// An element per thread keeps tensors with a side below 16 elements, and the
+// smallest ones, where a tile's two passes take longer than the scattered
+// writes: bytes up to 384 K elements where rows are the shorter side or have
+// fewer than 32 elements (1 x 513 x 7x7: 2.5 us, tiled 3.3; 2 x 50 x 45x45: 3.1,
+// 3.8; 4 x 50 x 45x45, 405 K: 4.0, 3.8; 4 x 63x63 x 17: 3.0, 3.5), 224 K otherwise
+// (2 x 45x45 x 50: 3.2, 3.3; 4 x 36x38 x 50, 274 K: 3.6, 3.3), dwords up to 192 K
+// (45x45 x 50: 2.8, 3.1; 2 x 45x45 x 50: 3.5, 3.2).
 //
 // Bytes: each lane takes 16 rows x 4 columns of the tile, reads them as 16
 // dwords (4 columns of a row each), turns every 4 x 4 byte block around with
@@ -48,7 +55,9 @@ namespace {
 constexpr int kTileRowBytes = 128;
 constexpr int kDwordTile = 64;  // dwords per side of a dword tile
 constexpr int kShortSide = 16;   // shorter sides than this: an element per thread
-constexpr int kShortMost = 512;  // longest short side of the short-row and short-column forms
+// longest short side of the short-row and short-column forms, and of small
+// tensors (16 x 520 x 4x4: 2.8 us, tiled 3.1; 3 x 700 x 8x10: 3.7, tiled 3.1)
+constexpr int kShortMost = 512, kShortMostSmall = 576;
 // Dword transposes between 16-byte rows of at least so many bytes store
 // evict-first (32 x 56x56 x 128: 15.8 us, written through 19.3; 256 channels:
 // 36.3, 37.8), smaller ones through (32 x 14x14 x 512: 5.6 us, evict-first
@@ -391,6 +400,10 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
   const bool cols16 = (int64_t(cols) * esize) % 16 == 0;
   const auto *in = static_cast<const int8_t *>(src);
   auto *out = static_cast<int8_t *>(dst);
+  const bool small = total < (esize == 4 ? 192 : rows < cols || cols < 32 ? 384 : 224) << 10;
+  const int short_most = small ? kShortMostSmall : kShortMost;
+  const bool short_rows = rows16 && int64_t(cols) * esize * 16 <= kShortLds;
+  const bool short_cols = cols16 && int64_t(rows) * esize * 16 <= kShortLds;
   auto tiled = [&](auto any) {
     constexpr bool kAny = decltype(any)::value;
     const int T = esize == 1 ? kTileRowBytes : kDwordTile;
@@ -411,7 +424,7 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
     return launch_status("transpose launch");
   };
   if (aligned16 && rows16 && cols16) return tiled(std::false_type{});
-  if (aligned16 && rows16 && cols <= kShortMost && int64_t(cols) * esize * 16 <= kShortLds) {
+  if (aligned16 && short_rows && cols <= short_most) {
     const int R = int(std::min<int64_t>(128, kShortLds / (int64_t(cols) * esize) / 16 * 16));
     const int tiles = (rows + R - 1) / R;
     const int64_t blocks = batch * tiles;
@@ -423,7 +436,7 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
                          out, rows, cols, R, tiles);
     return launch_status("transpose launch");
   }
-  if (aligned16 && cols16 && rows <= kShortMost && int64_t(rows) * esize * 16 <= kShortLds) {
+  if (aligned16 && short_cols && rows <= short_most) {
     const int wb = int(std::min<int64_t>(kTileRowBytes, kShortLds / (int64_t(rows) * esize) / 16 * 16));
     const int W = wb / esize;
     const int tiles = (cols + W - 1) / W;
@@ -436,7 +449,8 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
                          out, rows, cols, W, tiles);
     return launch_status("transpose launch");
   }
-  if (rows >= kShortSide && cols >= kShortSide) return tiled(std::true_type{});
+  if (rows >= kShortSide && cols >= kShortSide && (!small || (aligned16 && (short_rows || short_cols))))
+    return tiled(std::true_type{});
   const unsigned blocks = unsigned(std::min<int64_t>((total + kThreads - 1) / kThreads, 1 << 20));
   if (esize == 1)
     hipLaunchKernelGGL(transpose_elements<int8_t>, dim3(blocks), dim3(kThreads), 0, s,
