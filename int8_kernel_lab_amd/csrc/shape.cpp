@@ -238,11 +238,12 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
 //     32 -> 32 3x3: 5.1, 5.3; five stages, 352x352, 64 -> 32 3x3 stride 2: 6.9,
 //     6.2).
 // C % 128 == 0: the pipelined kernel, except
-//   * at most 128 tiles of 64 x 64, six to 18 stages: 64 x 64 (52x52, 256 ->
-//     512 3x3 stride 2: 10.0 -> 7.3 with two groups; 2 x 64x64, 128 -> 64: 7.0
-//     -> 5.9).  More tiles or stages stay (2 x 40x40, 256 -> 192, 150 tiles:
-//     10.0 against 12.1; 36x36, 512 -> 256, 36 stages: 16.1 against 18.4), but
-//     for grids so small that the policy splits their reduction;
+//   * at most one tile of 64 x 64 per unit and six stages or more: 64 x 64
+//     (pipelined, 64 x 64: 52x52, 256 -> 512 3x3 stride 2: 10.0, 7.5; 2 x 40x40,
+//     256 -> 192, 150 tiles: 10.1, 7.7; 36x36, 512 -> 256, 36 stages: 16.0,
+//     11.2; 2 x 128x128, 384 -> 72 stride 2, 256 tiles, int8: 14.0, 11.6; beyond
+//     that two rounds: 2 x 134x134, 256 -> 72 dilated, 282 tiles: 10.3, 11.1;
+//     180x180, 128 -> 256 stride 2, 508 tiles: 7.6, 8.6);
 //   * three or four stages and N no multiple of 128, up to 64 too: 128 x 64
 //     from 512 tiles on (64 x 28x28, 384 -> 192 1x1: 19.0 -> 12.3; 53 x 62x62,
 //     512 -> 288: 103 -> 94; 30 x 60x60, 384 -> 64: 14.6 -> 12.5; 20 x 60x60,
@@ -279,7 +280,7 @@ GemmPlan plan_generic(const i8conv_shape &s, const i8conv_geometry &g) {
     set_gemm32(g, p, 256, 256);
   else if (p.stages >= 3 && p.stages <= 4 && g.gemm_n % 128 != 0 && tiles(128, 64) >= 512)
     set_gemm32(g, p, 128, 64);
-  else if (p.stages >= 6 && tiles(64, 64) <= 128 && (p.stages <= 18 || tiles(p.bm, p.bn) <= 16))
+  else if (p.stages >= 6 && tiles(64, 64) <= 256)
     set_gemm32(g, p, 64, 64);
   return p;
 }

@@ -33,6 +33,9 @@ CASES = {
                    lab.ConvShape(2, 11, 10, 352, 68, 3, 3, 1, 1, 1, 1, 1, 1)),
     "64_g4_c656_5x1": ("64px x 64oc, grid 6x3, 26 k-stages, 4 wave groups",
                        lab.ConvShape(5, 9, 8, 656, 132, 5, 1, 2, 0, 1, 1, 1, 1)),
+    # ... and of a layer that the pipelined kernel would run on 22 tiles
+    "64_g4_c512_k132": ("64px x 64oc, grid 21x3, 36 k-stages, 4 wave groups",
+                        lab.ConvShape(1, 35, 37, 512, 132, 3, 3, 1, 1, 1, 1, 1, 1)),
     "64_k128": ("64px x 64oc", lab.ConvShape(18, 31, 33, 32, 36, 2, 2, 0, 0, 1, 1, 1, 1)),
     # 128 x 64: C = 32 and 48, odd channel counts, padding wider than the image
     "128x64_c32_k63": ("128px x 64oc", lab.ConvShape(5, 121, 119, 32, 63, 3, 3, 1, 1, 1, 1, 1, 1)),
@@ -67,6 +70,15 @@ CASES = {
 def test_gemm32_runs_these_layers(name):
     tile, shape = CASES[name]
     assert f"32x32 MFMA tile {tile}" in lab.describe("generic", shape)
+
+
+@pytest.mark.parametrize("n,hw,c,k,r,small", [
+    # one 64 x 64 tile per compute unit at most, from six stages on
+    (1, 128, 256, 64, 3, True), (1, 129, 256, 64, 3, False), (2, 40, 256, 192, 3, True),
+    (1, 36, 512, 256, 3, True), (1, 36, 512, 256, 1, False), (1, 36, 768, 256, 1, True)])
+def test_64_wide_tiles_of_deep_layers_in_one_round(n, hw, c, k, r, small):
+    s = lab.ConvShape(n, hw, hw, c, k, r, r, r // 2, r // 2, 1, 1, 1, 1)
+    assert ("32x32 MFMA tile 64px x 64oc" in lab.describe("generic", s)) == small
 
 
 @pytest.mark.parametrize("n,hw,c,k,r,wide", [
