@@ -195,7 +195,7 @@ static void set_gemm32(const i8conv_geometry &g, GemmPlan &p, int bm, int bn) {
 // The 32 x 32 x 32 MFMA kernel's tile for any channel count, or none (below).
 static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
   auto tiles = [&](int bm, int bn) { return ceil_div(g.gemm_m, bm) * ceil_div(g.gemm_n, bn); };
-  if (g.gemm_n > 64 && p.stages >= 8 && tiles(64, 64) <= 1152)
+  if (g.gemm_n > 64 && p.stages >= 8 && tiles(64, 64) <= 896)
     set_gemm32(g, p, 64, 64);
   else if (g.gemm_n > 64 && tiles(128, 128) >= 256)
     set_gemm32(g, p, 128, 128);
@@ -213,9 +213,12 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
 //   * 128 x 128, two workgroups per unit, for N > 64 with at least 256 tiles
 //     (256x256, 64 -> 255 3x3: 43 -> 21; 7 x 196x196, 80 -> 209 1x3: 202 ->
 //     48; 16 x 224x224, 32 -> 96 4x4 stride 4: 15.8 -> 8.6, 64 x 64: 10.0);
-//     But at most 1152 tiles of 64 x 64 and eight or more stages: those with
-//     two groups of waves (2 x 238x25, 400 -> 288 3x3: 41 -> 30; 22 x 40x40,
-//     400 -> 96 1x3: 19.5 -> 15.4, int8 25.4 -> 17.4);
+//     But at most 896 tiles of 64 x 64, 1.75 rounds, and eight or more stages:
+//     those with two groups of waves, as they leave fewer dead columns (64 x 64,
+//     128 x 128: 130x130, 224 -> 160 3x3, 795 tiles: 17.2, 17.9; 4 x 135x135,
+//     400 -> 160 5x5 stride 2, 867, int8: 68.1, 70.8; 2 x 238x25, 400 -> 288
+//     3x3, 930: 29.4, 28.3; 8 x 64x64, 160 -> 72 3x3, 1024, int8: 15.4, 12.2;
+//     22 x 40x40, 400 -> 96 1x3, 1100: 15.8, 14.6, int8 16.8, 15.0);
 //   * 128 x 64, three per unit, with at least 512 tiles (16 x 224x224, 32 ->
 //     64 7x7 stride 2: 101 -> 35; 256x256, 64 -> 63: 16.4 -> 9.3), 128 x 32
 //     for at most 32 channels (30 x 97x108, 32 -> 32 7x7 stride 2: 128 x 64
@@ -226,11 +229,12 @@ static void gemm32_tile(const i8conv_geometry &g, GemmPlan &p) {
 //   * 64 x 64, four per unit, below that (416x416, 32 -> 64 3x3 stride 2: 7.3
 //     -> 5.9, 128 x 64: 7.6).  With at most two tiles per unit a stage's
 //     latency counts, not its throughput: then groups of waves share a tile's
-//     stages, two of them from six stages on (4 x 28x28, 192 -> 192 3x3, 14
-//     stages: 19.9 -> 13.1 -> 10.6; 7 x 38x38, 288 -> 32, 21 stages: 17.8 ->
-//     14.2), four from 24 stages on and at most one tile per unit (193x34,
-//     432 -> 96, 31 stages: one group 26.1, two 18.6, four 17.3; at 14 stages
-//     four are slower than two, 11.4);
+//     stages (one group, two, four): two of them from six stages on (2 x
+//     118x118, 96 -> 72 3x3 stride 2, 7 stages: 6.0, 5.6; 4 x 28x28, 192 -> 192
+//     3x3, 14 stages: 8.2, 6.8, 7.6; 7 x 38x38, 288 -> 32, 21 stages: 10.6, 8.4,
+//     8.9; 2 x 70x70, 288 -> 160, 462 tiles: 13.5, 12.4), four from 24 stages on
+//     and at most one tile per unit (193x34, 432 -> 96, 31 stages: 14.2, 10.9,
+//     10.8; 16 x 12x12, 400 -> 192 5x3 stride 2, 47 stages: 19.4, 13.7, 13.0);
 //   * the register-staged kernel keeps layers of at most 64 channels, fewer
 //     than six stages and one round of 64-pixel tiles (2 x 30x30, 48 -> 64
 //     3x3: 5.5 against 6.0), and those of at most 32 channels and three stages

@@ -81,6 +81,15 @@ def test_64_wide_tiles_of_deep_layers_in_one_round(n, hw, c, k, r, small):
     assert ("32x32 MFMA tile 64px x 64oc" in lab.describe("generic", s)) == small
 
 
+@pytest.mark.parametrize("n,hw,c,k,tile", [
+    # at least 256 tiles of 128 x 128: 64 x 64 up to 896 tiles, from eight stages on
+    (1, 130, 224, 160, 64), (4, 56, 160, 288, 128), (8, 64, 160, 72, 128), (4, 57, 160, 320, 128),
+    (1, 130, 96, 160, 128), (1, 128, 224, 160, 64)])
+def test_64_wide_tiles_up_to_two_rounds(n, hw, c, k, tile):
+    s = lab.ConvShape(n, hw, hw, c, k, 3, 3, 1, 1, 1, 1, 1, 1)
+    assert f"32x32 MFMA tile {tile}px x {tile}oc" in lab.describe("generic", s)
+
+
 @pytest.mark.parametrize("n,hw,c,k,r,wide", [
     # 256-wide tiles where they compute at most 8/7 of the columns that 128-wide
     # ones do
