@@ -9,7 +9,7 @@
 // Tiled transposes (16-byte rows on both sides: rows * esize and cols *
 // esize multiples of 16, 16-byte aligned bases): one workgroup per 128 x
 // 128-byte tile (bytes: two tiles side by side where the source rows hold
-// 256 bytes or more) or 64 x 64-dword tile, read as whole source row pieces
+// 256 bytes or more) or 64 x 64- or 32 x 32-dword tile, read as whole source row pieces
 // (16 bytes a lane), staged in LDS and written as whole pieces of the
 // transposed matrix's rows.  With one side of at most 512 elements (any
 // number) and the other's rows whole 16-byte pieces, the short-row and
@@ -60,8 +60,10 @@ constexpr int kShortSide = 16;   // shorter sides than this: an element per thre
 constexpr int kShortMost = 512, kShortMostSmall = 576;
 // Dword transposes between 16-byte rows of at least so many bytes store
 // evict-first (32 x 56x56 x 128: 15.8 us, written through 19.3; 256 channels:
-// 36.3, 37.8), smaller ones through (32 x 14x14 x 512: 5.6 us, evict-first
-// 6.5); those of any length store ordinarily.
+// 36.3, 37.8), smaller ones through (48 x 28x28 x 64: 3.9 us, ordinarily 4.2);
+// those of any length and those whose output pieces share 32-byte sectors and
+// that are as large store ordinarily (47.8 MB, 119 x 14x14x512: 15.0 us, evict-
+// first 19.7).
 constexpr int64_t kStreamTransposeBytes = 32 << 20;
 
 __device__ __forceinline__ int byte_tile_row(int i) { return 32 * i + 8 * (i >> 4); }
@@ -188,11 +190,20 @@ __global__ __launch_bounds__(kThreads) void transpose_bytes_tiled(const int8_t *
 // x 4 rows of a wave's LDS accesses in 64 distinct banks on both sides.  kAny
 // as above: a lane's four rows end with the tile's last row, and a last tile of
 // fewer than four starts early.
-template <bool kAny, int kPolicy>
+//
+// Output rows of more than a tile that are no whole 32-byte sectors (rows % 8
+// != 0: 14 x 14, 62 x 62 pixels): neighbouring pieces share a sector, which only
+// the L2 puts together, so ordinary stores.  32 x 32 tiles then, 128-byte
+// pieces, where the columns fill them and are many (24 sets of tensors in turn,
+// 32, 64 wide, the latter evict-first or written through: 112 x 14x14x1024: 36.0
+// us, 54.8; 68 x 18x18x1024: 35.9, 53.9; 15 x 14x14x512: 4.1, 4.8; 12 x
+// 22x22x256: 4.0, 4.5; but 65 x 22x22x128: 11.4, 10.4), and the 64 wide stay
+// below 256 columns and for partly filled ones (47 x 34x34x60: 7.1, 4.3).
+template <bool kAny, int kPolicy, int T>
 __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t *src, int8_t *dst,
                                                                    int rows, int cols, int tiles_r,
                                                                    int tiles_c, int64_t batch) {
-  constexpr int T = kDwordTile, kPitch = T + 1;
+  constexpr int kPitch = T + 1, kPieces = T / 4, kLines = kThreads / kPieces;
   __shared__ uint32_t tile[T * kPitch];
   const int per_mat = tiles_r * tiles_c;
   const int mat = int(blockIdx.x) / per_mat;
@@ -204,12 +215,12 @@ __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t 
   const auto dr = make_rsrc(dst + size_t(mat) * mat_bytes, uint32_t(mat_bytes));
   const int r0 = kAny ? min(tr * T, rows - 4) : tr * T, c0 = tc * T;
   const uint32_t row_bytes = uint32_t(cols) * 4;
-  const int piece = threadIdx.x & 15, line = threadIdx.x >> 4;
-  // read: tile row i = source row r0 + i, bytes [c0*4, c0*4 + 256)
-  v4i in[T / 16];
+  const int piece = threadIdx.x % kPieces, line = threadIdx.x / kPieces;
+  // read: tile row i = source row r0 + i, bytes [c0*4, c0*4 + 4 T)
+  v4i in[T / kLines];
 #pragma unroll
-  for (int u = 0; u < T / 16; ++u) {
-    const int i = line + 16 * u;
+  for (int u = 0; u < T / kLines; ++u) {
+    const int i = line + kLines * u;
     const uint32_t cb = uint32_t(c0 * 4 + piece * 16);
     const bool ok = r0 + i < rows && cb < row_bytes;
     if constexpr (kAny)
@@ -220,11 +231,11 @@ __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t 
       in[u] = load16(sr, ok ? uint32_t(r0 + i) * row_bytes + cb : kOutOfRange);
   }
 #pragma unroll
-  for (int u = 0; u < T / 16; ++u)
+  for (int u = 0; u < T / kLines; ++u)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) tile[(line + 16 * u) * kPitch + piece * 4 + e] = uint32_t(in[u][e]);
+    for (int e = 0; e < 4; ++e) tile[(line + kLines * u) * kPitch + piece * 4 + e] = uint32_t(in[u][e]);
   __syncthreads();
-  // write: output row j = column c0 + j, bytes [r0*4, r0*4 + 256): the lane
+  // write: output row j = column c0 + j, bytes [r0*4, r0*4 + 4 T): the lane
   // gathers tile rows i0 .. i0 + 3 of column j (!kAny: rows % 4 == 0, the 4
   // rows are all inside the matrix or all outside)
   const uint32_t out_row_bytes = uint32_t(rows) * 4;
@@ -232,8 +243,8 @@ __global__ __launch_bounds__(kThreads) void transpose_dwords_tiled(const int8_t 
   if (r0 + i0 >= rows) return;
   if constexpr (kAny) i0 = min(i0, rows - r0 - 4);
 #pragma unroll
-  for (int u = 0; u < T / 16; ++u) {
-    const int j = line + 16 * u, c = c0 + j;
+  for (int u = 0; u < T / kLines; ++u) {
+    const int j = line + kLines * u, c = c0 + j;
     if (c >= cols) continue;
     v4i v;
 #pragma unroll
@@ -406,7 +417,10 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
   const bool short_cols = cols16 && int64_t(rows) * esize * 16 <= kShortLds;
   auto tiled = [&](auto any) {
     constexpr bool kAny = decltype(any)::value;
-    const int T = esize == 1 ? kTileRowBytes : kDwordTile;
+    // dwords: output pieces that share sectors; small tiles where those are full
+    const bool shared = esize == 4 && rows > kDwordTile && rows % 8 != 0;
+    const bool half = !kAny && shared && cols >= 256 && cols % 32 == 0;
+    const int T = esize == 1 ? kTileRowBytes : half ? 32 : kDwordTile;
     const int tiles_r = (rows + T - 1) / T;
     // bytes: two 128-column tiles per workgroup (256-byte source row pieces)
     // where the source rows are long enough to fill them
@@ -415,9 +429,13 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
     const int64_t blocks = batch * tiles_r * tiles_c;  // < 2^31: checked by the caller
     auto kern = sub == 2 ? transpose_bytes_tiled<2, kAny> : transpose_bytes_tiled<1, kAny>;
     if (esize != 1) {
-      kern = transpose_dwords_tiled<kAny, kAny ? 0 : kStoreThrough>;
-      if (!kAny && total * 4 >= kStreamTransposeBytes)
-        kern = transpose_dwords_tiled<kAny, kAny ? 0 : kStoreStream>;
+      kern = transpose_dwords_tiled<kAny, kAny ? 0 : kStoreThrough, kDwordTile>;
+      if constexpr (!kAny) {
+        if (half) kern = transpose_dwords_tiled<false, 0, 32>;
+        else if (total * 4 >= kStreamTransposeBytes)
+          kern = shared ? transpose_dwords_tiled<false, 0, kDwordTile>
+                        : transpose_dwords_tiled<false, kStoreStream, kDwordTile>;
+      }
     }
     hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kThreads), 0, s, in, out, rows, cols,
                        tiles_r, tiles_c, batch);

@@ -119,6 +119,23 @@ def test_nhwk_to_nkhw_int32_bit_exact(n, h, w, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,h,w,k", [
+    # output rows of 36 to 3844 dwords, most of which are no whole 32-byte sectors: small
+    # tiles (256 columns and more that fill them), large ones below and for
+    # partly filled ones, rows within one tile; with ordinary, write-through
+    # and evict-first stores (from 32 MiB on)
+    (2, 2, 34, 256), (3, 14, 14, 288), (2, 14, 14, 224), (1, 62, 62, 260), (5, 6, 6, 512),
+    (45, 14, 14, 1024), (187, 14, 14, 244), (240, 6, 6, 1024), (11, 28, 28, 1024)])
+def test_nhwk_to_nkhw_shared_sectors_bit_exact(n, h, w, k):
+    from tests.conftest import say
+    rng = np.random.default_rng(n + k)
+    y = rng.integers(-(2 ** 31), 2 ** 31, size=(n, h, w, k), dtype=np.int32)
+    say(f"[gpu] nhwk->nkhw {n}x{h}x{w}x{k}")
+    got = _run_gpu(lab.nhwk_to_nkhw, y, y.size, np.int32, n, h, w, k)
+    np.testing.assert_array_equal(got.reshape(n, k, h, w), y.transpose(0, 3, 1, 2))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,h,w,c,v", [(3, 7, 9, 96, 32), (2, 28, 28, 128, 32), (1, 5, 5, 64, 16),
                                        (2, 3, 3, 128, 64), (256, 3, 3, 128, 32)])
 def test_pack_vect_c_bit_exact(n, h, w, c, v):
