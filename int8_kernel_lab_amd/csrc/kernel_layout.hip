@@ -9,15 +9,15 @@
 // Tiled transposes (16-byte rows on both sides: rows * esize and cols *
 // esize multiples of 16, 16-byte aligned bases): one workgroup per 128 x
 // 128-byte tile (bytes: two tiles side by side where the source rows hold
-// 256 bytes or more) or 64 x 64- or 32 x 32-dword tile, read as whole source row pieces
-// (16 bytes a lane), staged in LDS and written as whole pieces of the
-// transposed matrix's rows.  With one side of at most 512 elements (any
-// number) and the other's rows whole 16-byte pieces, the short-row and
-// short-column forms below run (32 x 21x20 x 256 bytes: 3.9 us, tiled 4.4; 16
-// x 45x37 x 128: 6.1, tiled 4.3).  Everything else runs the tiled form with
-// pieces at any byte: an element per thread, its writes scattered, took 62 us
-// for 16 x 45x45 x 256 dwords (12 tiled, 5.5 TB/s), 298 for 32 x 448 x 63x63
-// bytes (30 tiled).
+// 256 bytes or more) or 64 x 64- or 32 x 32-dword tile, read as whole source
+// row pieces (16 bytes a lane), staged in LDS and written as whole pieces of
+// the transposed matrix's rows.  With one side of at most 512 elements (any
+// number; more where the other side has 16 or 32) and the other's rows whole
+// 16-byte pieces, the short-row and short-column forms below run (32 x 21x20 x
+// 256 bytes: 3.9 us, tiled 4.4; 16 x 45x37 x 128: 6.1, tiled 4.3).  Everything
+// else runs the tiled form with pieces at any byte: an element per thread, its
+// writes scattered, took 62 us for 16 x 45x45 x 256 dwords (12 tiled, 5.5
+// TB/s), 298 for 32 x 448 x 63x63 bytes (30 tiled).
 //
 // An element per thread keeps tensors with a side below 16 elements, and the
 // smallest ones, where a tile's two passes take longer than the scattered
@@ -43,6 +43,8 @@
 // are 16 bytes per lane, pixels consecutive across lanes on both sides.
 #include <hip/hip_runtime.h>
 
+#include <limits.h>
+
 #include <algorithm>
 #include <string>
 #include <type_traits>
@@ -55,9 +57,14 @@ namespace {
 constexpr int kTileRowBytes = 128;
 constexpr int kDwordTile = 64;  // dwords per side of a dword tile
 constexpr int kShortSide = 16;   // shorter sides than this: an element per thread
-// longest short side of the short-row and short-column forms, and of small
-// tensors (16 x 520 x 4x4: 2.8 us, tiled 3.1; 3 x 700 x 8x10: 3.7, tiled 3.1)
+// Longest short side of the short-row and short-column forms, and of small
+// tensors (16 x 520 x 4x4: 2.8 us, tiled 3.1; 3 x 700 x 8x10: 3.7, tiled 3.1).
+// Bytes of which the other side fills no 128-byte tile keep them longer, 16 up
+// to what LDS holds (285 x 45x45 x 16: 5.5 us, tiled 10.0; 16 x 30x30: 3.8,
+// 9.2), 32 up to these (32 x 33x33: 5.8, 7.0; 39x39: 13.5, 12.4; 39x39 x 32:
+// 4.7, 7.1; many sets in turn, 45x45 x 32: 9.5, 8.2; 48 x 23x23: 4.1, 3.9).
 constexpr int kShortMost = 512, kShortMostSmall = 576;
+constexpr int kShortMostRows = 1152, kShortMostCols = 1600;
 // Dword transposes between 16-byte rows of at least so many bytes store
 // evict-first (32 x 56x56 x 128: 15.8 us, written through 19.3; 256 channels:
 // 36.3, 37.8), smaller ones through (48 x 28x28 x 64: 3.9 us, ordinarily 4.2);
@@ -412,7 +419,10 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
   const auto *in = static_cast<const int8_t *>(src);
   auto *out = static_cast<int8_t *>(dst);
   const bool small = total < (esize == 4 ? 192 : rows < cols || cols < 32 ? 384 : 224) << 10;
-  const int short_most = small ? kShortMostSmall : kShortMost;
+  // the longest short side for another side of `other` elements
+  auto short_most = [&](int other, int narrow) {
+    return other <= 16 ? INT_MAX : other <= 32 ? narrow : small ? kShortMostSmall : kShortMost;
+  };
   const bool short_rows = rows16 && int64_t(cols) * esize * 16 <= kShortLds;
   const bool short_cols = cols16 && int64_t(rows) * esize * 16 <= kShortLds;
   auto tiled = [&](auto any) {
@@ -442,7 +452,7 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
     return launch_status("transpose launch");
   };
   if (aligned16 && rows16 && cols16) return tiled(std::false_type{});
-  if (aligned16 && short_rows && cols <= short_most) {
+  if (aligned16 && short_rows && cols <= short_most(rows, kShortMostRows)) {
     const int R = int(std::min<int64_t>(128, kShortLds / (int64_t(cols) * esize) / 16 * 16));
     const int tiles = (rows + R - 1) / R;
     const int64_t blocks = batch * tiles;
@@ -454,7 +464,7 @@ int launch_transpose(const void *src, void *dst, int64_t batch, int rows, int co
                          out, rows, cols, R, tiles);
     return launch_status("transpose launch");
   }
-  if (aligned16 && short_cols && rows <= short_most) {
+  if (aligned16 && short_cols && rows <= short_most(cols, kShortMostCols)) {
     const int wb = int(std::min<int64_t>(kTileRowBytes, kShortLds / (int64_t(rows) * esize) / 16 * 16));
     const int W = wb / esize;
     const int tiles = (cols + W - 1) / W;

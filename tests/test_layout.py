@@ -193,9 +193,11 @@ def test_transposes_between_unaligned_tensors_bit_exact(off):
 @pytest.mark.parametrize("n,rows,cols", [
     # large enough for tiles of any length on both sides: last tiles of one row,
     # of fewer rows than a lane stores and of just enough, of one column; one
-    # tile of rows; few columns.  The last one: elements
+    # tile of rows; few columns.  Long short sides of bytes next to 16 and 32
+    # elements.  The last one: elements
     (1, 16, 24577), (2, 513, 523), (1, 257, 2049), (3, 143, 1401), (1, 1025, 401), (2, 399, 1023),
-    (1, 24577, 17), (3, 131, 1001), (1, 385, 639)])
+    (1, 24577, 17), (3, 131, 1001), (37, 16, 2025), (19, 2047, 16), (11, 32, 1151), (12, 32, 1153),
+    (9, 1599, 32), (8, 1601, 32), (1, 385, 639)])
 def test_tiled_transposes_of_any_length_bit_exact(n, rows, cols, off):
     from tests.conftest import say
     rng = np.random.default_rng(rows + cols)
