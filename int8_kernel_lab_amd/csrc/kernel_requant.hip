@@ -6,7 +6,8 @@
 // thread reads 16 bytes of int32 (four channels of one pixel) and writes
 // their four int8 values as one dword; a scalar form covers N % 4 != 0.
 // The convolution kernels apply the same function in their epilogues instead;
-// this pass serves i8conv_requantize and split-K layers with N % 4 != 0.
+// this pass serves i8conv_requantize, split-K layers with N % 4 != 0, outputs
+// that overlap an input, and layers beyond the 32 x 32 x 32 kernel's sizes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
